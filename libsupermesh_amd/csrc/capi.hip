@@ -709,7 +709,7 @@ int libsupermesh_gpu_count_shape(libsupermesh_gpu_context* ctx, int dim, int* bl
     const CountShape& s = ctx->ctx.shape[dim - 2];
     if (block) *block = s.block;
     if (grid) *grid = s.grid;
-    if (lds_depths) *lds_depths = s.block == 0 ? 0 : (dim == 3 ? 3 - s.reg : 0);
+    if (lds_depths) *lds_depths = s.block == 0 ? 0 : (dim == 3 ? 3 : 0);
     if (ms) *ms = s.ms;
   });
 }

@@ -119,10 +119,9 @@ struct Predictor {
   DevBuf budget, overflow, spill, aoff;  // single-pass clip: budgets, flags, spill offsets, arena offsets
 };
 
-// Launch shape of the count-pass kernel: block size, grid (blocks), and in
-// 3D the walk's tet depths held in registers (the rest of 1..3 in LDS).
+// Launch shape of the count-pass kernel: block size and grid (blocks).
 struct CountShape {
-  int block = 0, grid = 0, reg = 0;
+  int block = 0, grid = 0;
   float ms = 0.f;  // its time on the sample it was measured on
 };
 

@@ -21,6 +21,7 @@
 #include "lsm_geometry.hpp"
 #include "lsm_runtime.hpp"
 #include "predictor.hpp"
+#include "tet_quad.hpp"
 
 namespace lsm {
 
@@ -723,21 +724,11 @@ __global__ void __launch_bounds__(BLOCK) k_clip_tri(ClipArgs g) {
   }
 }
 
-// Tet pairs on the compacted work list, one pair per lane at a time.  Each
-// lane walks its pair's clip tree with walk_next (every step builds one child
-// and classifies or measures it) and, when its pair is done, moves on to its
-// next work item by itself, so lanes never wait for the slowest pair of the
-// wave -- only for the slowest chain of work items, which evens out.
-// The walk of k_clip_tet_walk keeps its depth-1 tet in registers and its
-// depth-2 and depth-3 tets in LDS: a parent there is one LDS read per
-// coordinate and a child one write.  The stack is what limits how many waves
-// share a CU: 192 bytes per lane let three waves per SIMD run (two with all
-// three depths in LDS), at the cost of a register select per coordinate and
-// step.  Lane t's depth-j tet (j = 2, 3), coordinate i, is
-// stk[((j - 2) * 12 + i) * kWalkBlock] with stk = stack + t (consecutive
-// lanes, consecutive words).
+// Tet pairs on the compacted work list, one pair per quad of lanes at a time
+// (QuadClip, tet_quad.hpp).  A quad whose pair is done moves on to its next
+// work item by itself, so quads never wait for the slowest pair of the wave --
+// only for the slowest chain of work items, which evens out.
 constexpr int kWalkBlock = 128;
-constexpr int kWalkReg = 1;
 
 // The CDNA4 dispatcher hands consecutive workgroups to its 8 XCDs (each with
 // its own L2) in turn: with a grid whose size is a multiple of 8, block b
@@ -745,14 +736,14 @@ constexpr int kWalkReg = 1;
 // work list.
 constexpr int kXcds = 8;
 
-// The walk's lanes take work items from queues (counters handing out up to
+// The walk's quads take work items from queues (counters handing out up to
 // kQueueBatch consecutive items at a time): each XCD's share of the work list
 // is cut into kSubQueues contiguous parts, each with its own counter, so the
 // items in flight on an XCD stay a few compact windows of the list whose A
-// and B data its L2 holds (with fixed strides the lanes drift apart over the
+// and B data its L2 holds (with fixed strides the quads drift apart over the
 // whole share), and no counter takes more than a fraction of the atomics.
 // A short list is handed out in smaller batches (about a quarter of the
-// items per lane, at least one): with 16 at a time, a list of a few
+// items per quad, at least one): with 16 at a time, a list of a few
 // thousand items went to a few hundred lanes that walked 16 pairs each in
 // turn while the rest of the resident grid idled.
 constexpr int kQueueBatch = 16;
@@ -763,9 +754,13 @@ struct WalkQueue {
   long begin, end;  // this queue's part of the work list
   long w = 0, wend = 0;
   long batch = kQueueBatch;  // items per counter increment
-  __device__ __forceinline__ bool next() {  // advance to the next item; false when none is left
+  // advance the quad (whole) to its next item; false when none is left
+  __device__ __forceinline__ bool next() {
     if (++w < wend) return true;
-    const long s = begin + (long)atomicAdd(counter, (unsigned long long)batch);
+    unsigned long long got = 0;
+    if ((threadIdx.x & 3) == 0) got = atomicAdd(counter, (unsigned long long)batch);
+    got = (unsigned long long)quad_lane<0>((uint32_t)(got >> 32)) << 32 | quad_lane<0>((uint32_t)got);
+    const long s = begin + (long)got;
     if (s >= end) return false;
     w = s;
     wend = s + batch < end ? s + batch : end;
@@ -788,8 +783,8 @@ __device__ __forceinline__ WalkQueue walk_queue(unsigned long long* queues, long
   q.end = q.begin + sper < e0 ? q.begin + sper : e0;
   q.w = -1;
   q.wend = 0;
-  const long per_lane = n / (4L * gridDim.x * blockDim.x);
-  q.batch = per_lane < 1 ? 1 : (per_lane < kQueueBatch ? per_lane : kQueueBatch);
+  const long share = n / ((long)gridDim.x * blockDim.x);  // a quarter of the items per quad
+  q.batch = share < 1 ? 1 : (share < kQueueBatch ? share : kQueueBatch);
   return q;
 }
 
@@ -804,133 +799,211 @@ static unsigned long long* walk_queues(Context& C) {
   return q;
 }
 
+// The P1 x P1 mass of a pair from its kept tets' moments, one row of the block
+// per lane.  add() takes a kept tet in coordinates local to o, a vertex of the
+// pair's first output (inside both elements, so that the basis functions at o
+// lie in [0, 1] and nothing cancels); its integrals of 1, d_i and d_i d_j are
+// V, V/4 sum_v d_v and V/20 (sum_v d_v d_v' + (sum d)(sum d)'), exact for the
+// quadratic products, where the reference sums its 4-point rule, exact for
+// them too, over the tets (test_parallel_p1_inner_product_3d.F90:226-337).
+struct TetMoments {
+  double m[10];  // 1, x, y, z, xx, xy, xz, yy, yz, zz
+  double o[3];
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int i = 0; i < 10; i++) m[i] = 0.0;
+  }
+  __device__ __forceinline__ void add(const double* t, double vol) {
+    double d[4][3], s[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+#pragma unroll
+      for (int v = 0; v < 4; v++) d[v][k] = t[3 * v + k] - o[k];
+      s[k] = (d[0][k] + d[1][k]) + (d[2][k] + d[3][k]);
+    }
+    const double w4 = 0.25 * vol, w20 = 0.05 * vol;
+    m[0] += vol;
+#pragma unroll
+    for (int k = 0; k < 3; k++) m[1 + k] = __builtin_fma(w4, s[k], m[1 + k]);
+    int n = 4;
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+      for (int j = i; j < 3; j++) {
+        double x = s[i] * s[j];
+#pragma unroll
+        for (int v = 0; v < 4; v++) x = __builtin_fma(d[v][i], d[v][j], x);
+        m[n] = __builtin_fma(w20, x, m[n]);
+        n++;
+      }
+  }
+  // Row q of the block: int phi^A_q phi^B_j, j = 0..3 (whole quad).
+  __device__ __forceinline__ void row(int q, const double* __restrict__ affa, const double* __restrict__ affb,
+                                      double* out) {
+    double M[10];
+#pragma unroll
+    for (int i = 0; i < 10; i++) M[i] = quad_sum(m[i]);
+    double fa[4], fb[4], ga[3], alpha;
+    basis<3>(affa, o, fa);
+    basis<3>(affb, o, fb);
+    alpha = q == 0 ? fa[0] : (q == 1 ? fa[1] : (q == 2 ? fa[2] : fa[3]));
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      const double g1 = affa[3 + k], g2 = affa[6 + k], g3 = affa[9 + k];
+      ga[k] = q == 0 ? -((g1 + g2) + g3) : (q == 1 ? g1 : (q == 2 ? g2 : g3));
+    }
+    // int phi^A_q and int phi^A_q d
+    const double i0 = alpha * M[0] + (ga[0] * M[1] + ga[1] * M[2] + ga[2] * M[3]);
+    const double ix = alpha * M[1] + (ga[0] * M[4] + ga[1] * M[5] + ga[2] * M[6]);
+    const double iy = alpha * M[2] + (ga[0] * M[5] + ga[1] * M[7] + ga[2] * M[8]);
+    const double iz = alpha * M[3] + (ga[0] * M[6] + ga[1] * M[8] + ga[2] * M[9]);
+    double rest = 0.0;
+#pragma unroll
+    for (int j = 1; j < 4; j++) {
+      const double* h = affb + 3 * j;
+      const double g = h[0] * ix + h[1] * iy + h[2] * iz;
+      out[j] = fb[j] * i0 + g;
+      rest += g;
+    }
+    out[0] = fb[0] * i0 - rest;
+  }
+};
+
 // MODES: count (FILL and LEARNED false): counts, measures (and mass blocks);
 // fill (FILL): writes each pair's counts[p] outputs at offsets[p];
 // single pass (LEARNED): the count pass that also writes up to budget[w]
-// outputs of work item w at offsets[p] and the rest to the lane's arena.
-// BLOCK and REG (tet depths held in registers, 0 or 1; the other depths of
-// 1..3 in LDS) are launch shapes the count pass can be tuned over.
-template <bool MASS, bool FILL, bool LEARNED = false, int BLOCK = kWalkBlock, int REG = kWalkReg>
-__global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(MASS || REG == 0 ? 2 : 3)))
+// outputs of work item w at offsets[p] and the rest to the quad's arena.
+// BLOCK is a launch shape the count pass can be tuned over.
+template <bool MASS, bool FILL, bool LEARNED = false, int BLOCK = kWalkBlock>
+__global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(3)))
 k_clip_tet_walk(ClipArgs g) {
-  static_assert(REG == 0 || REG == 1, "depth 1 in registers or not");
-  __shared__ double stack[(3 - REG) * 12 * BLOCK];
-  double* stk = stack + threadIdx.x;
-  double R[REG > 0 ? 12 * REG : 1];
+  __shared__ QuadLds<4> lds[BLOCK / 64];
+  __shared__ uint4 table[256];
+  for (int i = threadIdx.x; i < 256; i += BLOCK) table[i] = reinterpret_cast<const uint4*>(kSplitTable.e)[i];
+  __syncthreads();
+  QuadClip<4> W;
+  W.init(&lds[threadIdx.x >> 6], table);
+  const int q = W.q;
   // blocks go to the XCDs round robin: each XCD takes one contiguous share
   // of the work list, so that its L2 holds one region of A and B
   WalkQueue Q = walk_queue(g.queue, (long)*g.nwork);
   bool more = Q.next();
-  long p = 0, off = 0;
+  bool active = false;
+  long p = 0, off = 0, a = 0, b = 0;
   int cap = 0, k = 0;
-  // single pass: this lane's arena region, its fill level, and whether the
+  // single pass: this quad's arena region, its fill level, and whether the
   // current pair's output outgrew budget and arena
   const long abase =
-      LEARNED ? g.arena_base + ((long)blockIdx.x * blockDim.x + threadIdx.x) * g.arena_per_lane : 0;
+      LEARNED ? g.arena_base + (((long)blockIdx.x * BLOCK + threadIdx.x) >> 2) * g.arena_per_lane : 0;
   long atop = 0;
   bool lost = false;
-  unsigned nsplit = 0, nlost = 0;  // this lane's split runs and pairs to clip again
-  double A[12], tol = 0.0, m = 0.0;
-  double blk[16], affa[12], affb[12];
-  // B's four planes are read from memory at each step (the pair's 128 bytes
-  // stay in cache): held in registers they would cost the third wave per
-  // SIMD, and even planes 2 and 3 alone (16 registers more, no fewer waves)
-  // made the count pass slower (30.2 against 28.1 ms on tet 64^3 vs 60^3)
-  const double* bpl = nullptr;
-  auto plane = [&](int j, double* o) {
-#pragma unroll
-    for (int i = 0; i < 4; i++) o[i] = bpl[4 * j + i];
-  };
-  WalkState<4> W;
-  W.level = 0;
-  bool active = false;
+  unsigned nsplit = 0, nlost = 0;  // this quad's split runs and pairs to clip again
+  double tol = 0.0, m = 0.0;
+  TetMoments mom;
   while (true) {
-    if (!active) {
-      // next work item of this lane (fill pass: skip pairs with no output)
-      while (more) {
-        p = g.work[Q.w];
-        if (!FILL) break;
-        cap = g.counts[p];
-        if (cap > 0 && (!g.ovf || g.ovf[Q.w] == 2)) break;
-        more = Q.next();
-      }
-      if (!more) break;
-      const long w = Q.w;
-      if (FILL) off = g.ovf ? g.aoff[w] : g.offsets[p];
-      if (LEARNED) {
-        cap = (int)((g.budget[w] >> g.bshift) & 0xffu);
-        off = g.offsets[p];
-        lost = false;
-      }
-      const long a = g.rows[p], b = g.cols[p];
+    if (!W.cur) {
+      if (W.pend) {
+        W.pop();
+      } else {
+        if (active) {  // the pair is done
+          if (LEARNED) {
+            const bool any_lost = quad_or(lost ? 1u : 0u) != 0;
+            const bool split = k > cap && !any_lost;
+            if (q == 0) {
+              g.aoff[Q.w] = split ? abase + atop : -1;
+              g.dropped[Q.w] = any_lost ? 2 : (split ? 1 : 0);
+            }
+            if (split) atop += k - cap;
+            nsplit += split ? 1u : 0u;
+            nlost += any_lost ? 1u : 0u;
+          }
+          if (!FILL) {
+            if (q == 0) {
+              __builtin_nontemporal_store(k, g.counts + p);
+              __builtin_nontemporal_store(k == 0 ? 0.0 : m, g.measure + p);
+            }
+            if (MASS) {
+              double row[4] = {0.0, 0.0, 0.0, 0.0};
+              if (k > 0) mom.row(q, g.aaff + a * 12, g.baff + b * 12, row);
 #pragma unroll
-      for (int i = 0; i < 12; i++) A[i] = g.acoords[a * 12 + i];
-      bpl = g.bplanes + b * 16;
-      tol = 10.0 * fmin_f(g.asp[a], g.bsp[b]);
-      m = 0.0;
-      k = 0;
-      if (MASS) {
-#pragma unroll
-        for (int i = 0; i < 16; i++) blk[i] = 0.0;
-#pragma unroll
-        for (int i = 0; i < 12; i++) {
-          affa[i] = g.aaff[a * 12 + i];
-          affb[i] = g.baff[b * 12 + i];
-        }
-      }
-      double p0[4], d0[4];
-      plane(0, p0);
-      walk_distances(A, p0, d0);
-      walk_begin(W, pack_class(d0));
-      active = true;
-    }
-    if (W.level > 0) {
-      walk_next<4, BLOCK, REG>(W, A, R, stk, plane, tol, [&](const double* t, double, bool keep) {
-        // every step hands over its child; only kept leaves count, and the
-        // measure adds 0 for the others (exactly the sum of the kept ones)
-        const double vr = tet_volume_real(t);
-        m = m + (keep ? vr : 0.0);
-        if (keep) {
-          if (MASS) mass_element<3>(t, vr, affa, affb, blk);
-          if ((FILL || LEARNED) && k < cap) {
-            stream_tet(g.elements + (off + k) * 12, t);
-          } else if (LEARNED) {
-            // beyond the budget: the run continues in this lane's arena
-            const long e = atop + (k - cap);
-            if (e < g.arena_per_lane) {
-              stream_tet(g.elements + (abase + e) * 12, t);
-            } else {
-              lost = true;
+              for (int j = 0; j < 4; j++) g.blocks[p * 16 + 4 * q + j] = row[j];
             }
           }
+          more = Q.next();
+          active = false;
         }
-        k += keep ? 1 : 0;
-      });
-      if (W.level > 0) continue;
-    }
-    if (LEARNED) {
-      const bool split = k > cap && !lost;
-      g.aoff[Q.w] = split ? abase + atop : -1;
-      if (split) atop += k - cap;
-      g.dropped[Q.w] = lost ? 2 : (split ? 1 : 0);
-      nsplit += split ? 1u : 0u;
-      nlost += lost ? 1u : 0u;
-    }
-    if (!FILL) {
-      __builtin_nontemporal_store(k, g.counts + p);
-      __builtin_nontemporal_store(k == 0 ? 0.0 : m, g.measure + p);
-      if (MASS) {
+        // next work item of this quad (fill pass: skip pairs with no output)
+        while (more) {
+          p = g.work[Q.w];
+          if (!FILL) break;
+          cap = g.counts[p];
+          if (cap > 0 && (!g.ovf || g.ovf[Q.w] == 2)) break;
+          more = Q.next();
+        }
+        if (!more) break;
+        if (FILL) off = g.ovf ? g.aoff[Q.w] : g.offsets[p];
+        if (LEARNED) {
+          cap = (int)((g.budget[Q.w] >> g.bshift) & 0xffu);
+          off = g.offsets[p];
+          lost = false;
+        }
+        a = g.rows[p];
+        b = g.cols[p];
+        tol = 10.0 * fmin_f(g.asp[a], g.bsp[b]);
+        m = 0.0;
+        k = 0;
+        if (MASS) mom.clear();
+        // lane q brings in B's plane q and A's vertex q
+        double P[4], v[3];
 #pragma unroll
-        for (int i = 0; i < 16; i++) g.blocks[p * 16 + i] = k == 0 ? 0.0 : blk[i];
+        for (int i = 0; i < 4; i++) P[i] = g.bplanes[b * 16 + 4 * q + i];
+#pragma unroll
+        for (int i = 0; i < 3; i++) v[i] = g.acoords[a * 12 + 3 * q + i];
+        W.set_plane(q, P);
+        W.begin(v);
+        active = true;
       }
     }
-    more = Q.next();
-    active = false;
+    W.step([&](const double* t, uint32_t lead) {
+      const bool keep = ((lead >> q) & 1u) && volume_reaches(t, tol);
+      const double vr = keep ? tet_volume_real(t) : 0.0;
+      // the reference's order; 0 for the others adds nothing
+      m = m + quad_lane<0>(vr);
+      m = m + quad_lane<1>(vr);
+      m = m + quad_lane<2>(vr);
+      const uint32_t kept = quad_or((keep ? 1u : 0u) << q);
+      if (MASS) {
+        // the origin: the first output's first vertex
+        const uint32_t first = lead & -lead;
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+          const double x0 = quad_lane<0>(t[i]), x1 = quad_lane<1>(t[i]), x2 = quad_lane<2>(t[i]);
+          const double x = first == 1u ? x0 : (first == 2u ? x1 : x2);
+          mom.o[i] = k == 0 ? x : mom.o[i];
+        }
+        if (keep) mom.add(t, vr);
+      }
+      if (FILL || LEARNED) {
+        const int at = k + __builtin_popcount(kept & ((1u << q) - 1u));
+        if (keep && at < cap) {
+          stream_tet(g.elements + (off + at) * 12, t);
+        } else if (LEARNED && keep) {
+          // beyond the budget: the run continues in this quad's arena
+          const long e = atop + (at - cap);
+          if (e < g.arena_per_lane) {
+            stream_tet(g.elements + (abase + e) * 12, t);
+          } else {
+            lost = true;
+          }
+        }
+      }
+      k += __builtin_popcount(kept);
+    });
   }
   if (LEARNED) {
     // one atomic per wave: one per pair on a single counter serialised the
     // single pass (tet 96^3 at budget level 0.9: 7.4 M of them, ~20 ms)
-    unsigned long long s = nsplit, l = nlost;
+    unsigned long long s = q == 0 ? nsplit : 0u, l = q == 0 ? nlost : 0u;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
       s += __shfl_xor(s, o, 64);
@@ -1097,12 +1170,11 @@ __global__ void __launch_bounds__(kTriBlock) k_clip_mixed(MixedArgs g) {
   }
 }
 
-// 3D: one pair per lane at a time over the six planes of the hexahedron
-// (walk_next<6>, depths 1..2 in registers, 3..5 in LDS); a lane moves on to its next pair
-// as soon as its walk ends.  MODE 0: tet A x hex B; 1: hex A x tet B (the
-// tet is B's); 2: hex A x hex B, A's five tets in turn, outputs and measure
-// accumulated over them in order.  hplanes: planes of the hexahedra,
-// [n][6][4] (hex_planes).
+// 3D: one pair per quad at a time over the six planes of the hexahedron
+// (QuadClip<6>); a quad moves on to its next pair as soon as its walk ends.
+// MODE 0: tet A x hex B; 1: hex A x tet B (the tet is B's); 2: hex A x hex B,
+// A's five tets in turn, outputs and measure accumulated over them in order.
+// hplanes: planes of the hexahedra, [n][6][4] (hex_planes).
 struct HexWalkArgs {
   long npairs;
   const int* rows;
@@ -1117,91 +1189,99 @@ struct HexWalkArgs {
   unsigned long long* queue;  // the walk's work-item counters (zeroed before each launch)
 };
 
-// One wave per block; the walk keeps its depth-1 and depth-2 tets in
-// registers and depths 3..5 in LDS (18 KB per block, eight blocks per CU).
-constexpr int kHexBlock = 64;
-constexpr int kHexReg = 2;
+constexpr int kHexBlock = 128;
 
 template <int MODE, bool FILL>
 __global__ void __launch_bounds__(kHexBlock) __attribute__((amdgpu_waves_per_eu(2)))
 k_clip_hex_walk(HexWalkArgs g) {
-  __shared__ double stack[(5 - kHexReg) * 12 * kHexBlock];
-  double* stk = stack + threadIdx.x;
-  double R[12 * kHexReg];
+  __shared__ QuadLds<6> lds[kHexBlock / 64];
+  __shared__ uint4 table[256];
+  for (int i = threadIdx.x; i < 256; i += kHexBlock) table[i] = reinterpret_cast<const uint4*>(kSplitTable.e)[i];
+  __syncthreads();
+  QuadClip<6> W;
+  W.init(&lds[threadIdx.x >> 6], table);
+  const int q = W.q;
   // pairs from the walk's queues, as k_clip_tet_walk takes its work items
   WalkQueue Q = walk_queue(g.queue, g.npairs);
   bool more = Q.next();
+  bool active = false;
   long p = 0, off = 0, a = 0;
   int cap = 0, k = 0, sub = 0;
-  double T[12], tol = 0.0, m = 0.0;
-  const double* planes = nullptr;
-  auto plane = [&](int j, double* o) {
-#pragma unroll
-    for (int i = 0; i < 4; i++) o[i] = planes[4 * j + i];
-  };
-  WalkState<6> W;
-  W.level = 0;
-  bool active = false;
-  auto start = [&]() {
+  double tol = 0.0, m = 0.0;
+  auto start = [&](const double* T) {
     tol = 10.0 * fspacing(tet_volume_tet(T));
-    double d0[4];
-    walk_distances(T, planes, d0);
-    walk_begin(W, pack_class(d0));
+    double v[3];
+#pragma unroll
+    for (int i = 0; i < 3; i++) v[i] = q == 0 ? T[i] : (q == 1 ? T[3 + i] : (q == 2 ? T[6 + i] : T[9 + i]));
+    W.begin(v);
   };
   while (true) {
-    if (!active) {
-      while (more) {
-        p = Q.w;
-        if (!FILL) break;
-        cap = g.counts[p];
-        if (cap > 0) break;
-        more = Q.next();
-      }
-      if (!more) break;
-      if (FILL) off = g.offsets[p];
-      a = g.rows[p];
-      const long b = g.cols[p];
-      if (MODE == 0) {
-#pragma unroll
-        for (int i = 0; i < 12; i++) T[i] = g.acoords[a * 12 + i];
-        planes = g.hplanes + b * 24;
-      } else if (MODE == 1) {
-#pragma unroll
-        for (int i = 0; i < 12; i++) T[i] = g.bcoords[b * 12 + i];
-        planes = g.hplanes + a * 24;
+    if (!W.cur) {
+      if (W.pend) {
+        W.pop();
       } else {
-        sub = 0;
-        hex_split_tet(g.acoords + a * 24, 0, T);
-        planes = g.hplanes + b * 24;
-      }
-      m = 0.0;
-      k = 0;
-      start();
-      active = true;
-    }
-    if (W.level > 0) {
-      walk_next<6, kHexBlock, kHexReg>(W, T, R, stk, plane, tol, [&](const double* t, double, bool keep) {
-        const double vr = tet_volume_real(t);
-        m = m + (keep ? vr : 0.0);
-        if (FILL && keep && k < cap) {
-          stream_tet(g.elements + (off + k) * 12, t);
+        double T[12];
+        if (MODE == 2 && active && sub < 4) {
+          sub++;
+          hex_split_tet(g.acoords + a * 24, sub, T);
+        } else {
+          if (active) {
+            if (!FILL && q == 0) {
+              __builtin_nontemporal_store(k, g.counts + p);
+              __builtin_nontemporal_store(k == 0 ? 0.0 : m, g.measure + p);
+            }
+            more = Q.next();
+            active = false;
+          }
+          while (more) {
+            p = Q.w;
+            if (!FILL) break;
+            cap = g.counts[p];
+            if (cap > 0) break;
+            more = Q.next();
+          }
+          if (!more) break;
+          if (FILL) off = g.offsets[p];
+          a = g.rows[p];
+          const long b = g.cols[p];
+          const double* planes = g.hplanes + (MODE == 1 ? a : b) * 24;
+          double P[4];
+#pragma unroll
+          for (int i = 0; i < 4; i++) P[i] = planes[4 * q + i];
+          W.set_plane(q, P);
+          if (q < 2) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) P[i] = planes[16 + 4 * q + i];
+            W.set_plane(4 + q, P);
+          }
+          if (MODE == 2) {
+            sub = 0;
+            hex_split_tet(g.acoords + a * 24, 0, T);
+          } else {
+            const double* t = MODE == 0 ? g.acoords + a * 12 : g.bcoords + b * 12;
+#pragma unroll
+            for (int i = 0; i < 12; i++) T[i] = t[i];
+          }
+          m = 0.0;
+          k = 0;
+          active = true;
         }
-        k += keep ? 1 : 0;
-      });
-      if (W.level > 0) continue;
+        start(T);
+      }
     }
-    if (MODE == 2 && sub < 4) {
-      sub++;
-      hex_split_tet(g.acoords + a * 24, sub, T);
-      start();
-      continue;
-    }
-    if (!FILL) {
-      __builtin_nontemporal_store(k, g.counts + p);
-      __builtin_nontemporal_store(k == 0 ? 0.0 : m, g.measure + p);
-    }
-    more = Q.next();
-    active = false;
+    W.step([&](const double* t, uint32_t lead) {
+      const bool keep = ((lead >> q) & 1u) && volume_reaches(t, tol);
+      const double vr = keep ? tet_volume_real(t) : 0.0;
+      m = m + quad_lane<0>(vr);
+      m = m + quad_lane<1>(vr);
+      m = m + quad_lane<2>(vr);
+      const uint32_t kept = quad_or((keep ? 1u : 0u) << q);
+      if (FILL) {
+        const int at = k + __builtin_popcount(kept & ((1u << q) - 1u));
+        if (keep && at < cap) stream_tet(g.elements + (off + at) * 12, t);
+      }
+      k += __builtin_popcount(kept);
+    });
   }
 }
 
@@ -1238,7 +1318,7 @@ static void launch_mixed(Context& C, int la, int lb, MixedArgs g) {
   launch_mixed_as<FILL, true>(C, la, lb, g);
 }
 
-// Persistent lanes for the hexahedron walk: one full wave of resident blocks.
+// Persistent quads for the hexahedron walk: one full wave of resident blocks.
 template <int MODE, bool FILL>
 static void launch_hex_walk_as(Context& C, const HexWalkArgs& g) {
   static int blocks_per_cu = 0;
@@ -1250,9 +1330,9 @@ static void launch_hex_walk_as(Context& C, const HexWalkArgs& g) {
   }
   int cus = 0;
   LSM_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, C.device));
-  const long lanes = (long)blocks_per_cu * (cus > 0 ? cus : 256) * kHexBlock;
-  const long need = (g.npairs + kHexBlock - 1) / kHexBlock;
-  unsigned blocks = (unsigned)std::max(1L, std::min(lanes / kHexBlock, need));
+  const long resident = (long)blocks_per_cu * (cus > 0 ? cus : 256);
+  const long need = (g.npairs + kHexBlock / 4 - 1) / (kHexBlock / 4);
+  unsigned blocks = (unsigned)std::max(1L, std::min(resident, need));
   if (blocks >= kXcds) blocks -= blocks % kXcds;  // whole XCD shares (walk_queue)
   HexWalkArgs h = g;
   h.queue = walk_queues(C);
@@ -1494,7 +1574,8 @@ static unsigned tet_walk_blocks(Context& C, int which) {
   return (unsigned)(blocks_per_cu[which] * (cus > 0 ? cus : 256));
 }
 
-static long tet_walk_lanes(Context& C, int which) { return (long)tet_walk_blocks(C, which) * kWalkBlock; }
+// Quads of the walk's grid: each has an arena share in the single pass.
+static long tet_walk_quads(Context& C, int which) { return (long)tet_walk_blocks(C, which) * (kWalkBlock / 4); }
 
 
 static void launch_tet_walk(Context& C, const ClipArgs& a, int which) {
@@ -1959,7 +2040,7 @@ void clip_pairs(Context& C, const DevMesh& A, const DevMesh& B, long npairs, int
     LSM_HIP(hipMemGetInfo(&free_b, &total_b));
     const double avail = (double)free_b + (double)C.elements.bytes - 4e9;
     const double expect = (double)hs[4] / 1024.0;
-    const long lanes = tet_walk_lanes(C, mass ? 4 : 3);  // the grid of the single-pass launch
+    const long lanes = tet_walk_quads(C, mass ? 4 : 3);  // the grid of the single-pass launch
     arena_per_lane = ((long)(P.arena_fraction * expect) + P.arena_min) / lanes;
     nspill = (long)(P.spill_fraction * expect) + P.spill_min;
     gap = dense ? (long)(expect / 256.0) + 4096 : 0;
@@ -2136,12 +2217,12 @@ __global__ void k_min_u64(const unsigned long long* __restrict__ n, unsigned lon
   if (threadIdx.x == 0 && blockIdx.x == 0) *out = *n < cap ? *n : cap;
 }
 
-template <int BLOCK, int REG>
+template <int BLOCK>
 static int walk_blocks_per_cu() {
   static int nb = 0;
   if (nb == 0) {
     LSM_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &nb, reinterpret_cast<const void*>(k_clip_tet_walk<false, false, false, BLOCK, REG>), BLOCK, 0));
+        &nb, reinterpret_cast<const void*>(k_clip_tet_walk<false, false, false, BLOCK>), BLOCK, 0));
     nb = nb > 0 ? nb : 1;
   }
   return nb;
@@ -2153,22 +2234,17 @@ static int device_cus(Context& C) {
   return cus > 0 ? cus : 256;
 }
 
-template <int BLOCK, int REG>
+template <int BLOCK>
 static void walk_count_as(Context& C, const ClipArgs& g, int grid) {
-  hipLaunchKernelGGL((k_clip_tet_walk<false, false, false, BLOCK, REG>), dim3(grid), dim3(BLOCK), 0, C.stream, g);
+  hipLaunchKernelGGL((k_clip_tet_walk<false, false, false, BLOCK>), dim3(grid), dim3(BLOCK), 0, C.stream, g);
 }
 
 static void launch_count_walk(Context& C, const ClipArgs& a, const CountShape& s) {
   ClipArgs g = a;
   g.queue = walk_queues(C);
-  switch (s.block * 2 + s.reg) {
-    case 128: walk_count_as<64, 0>(C, g, s.grid); break;
-    case 129: walk_count_as<64, 1>(C, g, s.grid); break;
-    case 256: walk_count_as<128, 0>(C, g, s.grid); break;
-    case 257: walk_count_as<128, 1>(C, g, s.grid); break;
-    case 512: walk_count_as<256, 0>(C, g, s.grid); break;
-    default: walk_count_as<256, 1>(C, g, s.grid); break;
-  }
+  if (s.block == 64) walk_count_as<64>(C, g, s.grid);
+  else if (s.block == 128) walk_count_as<128>(C, g, s.grid);
+  else walk_count_as<256>(C, g, s.grid);
   LSM_HIP(hipGetLastError());
 }
 
@@ -2191,9 +2267,8 @@ static void launch_count_tri(Context& C, const ClipArgs& g, const CountShape& s,
 
 // Times every candidate shape on a prefix of the pairs (3D: of the work list
 // the triage left in g) and keeps the fastest in C.shape.  Candidates:
-// blocks of 64, 128 or 256 lanes; 3D: the depth-1 tet in registers or in
-// LDS, and every resident block (the walk's lanes are persistent) or half
-// of them; 2D: grids of 1024 to 8192 blocks (pairs per lane of the
+// blocks of 64, 128 or 256 lanes; 3D: every resident block (the walk's
+// quads are persistent) or half of them; 2D: grids of 1024 to 8192 blocks (pairs per lane of the
 // grid-stride loop) or one block per `block` pairs.  Each candidate runs once
 // to warm up, then once timed.
 static void tune_count_pass(Context& C, ClipArgs g, int dim) {
@@ -2201,18 +2276,15 @@ static void tune_count_pass(Context& C, ClipArgs g, int dim) {
   std::vector<CountShape> cand;
   const int cus = device_cus(C);
   if (dim == 3) {
-    const int bpc[6] = {walk_blocks_per_cu<64, 0>(), walk_blocks_per_cu<64, 1>(), walk_blocks_per_cu<128, 0>(),
-                        walk_blocks_per_cu<128, 1>(), walk_blocks_per_cu<256, 0>(), walk_blocks_per_cu<256, 1>()};
+    const int bpc[3] = {walk_blocks_per_cu<64>(), walk_blocks_per_cu<128>(), walk_blocks_per_cu<256>()};
     const int blocks[3] = {64, 128, 256};
     for (int b = 0; b < 3; b++)
-      for (int reg = 0; reg < 2; reg++)
-        for (int half = 0; half < 2; half++) {
-          CountShape c;
-          c.block = blocks[b];
-          c.reg = reg;
-          c.grid = std::max(kXcds, (bpc[2 * b + reg] * cus) >> half);
-          cand.push_back(c);
-        }
+      for (int half = 0; half < 2; half++) {
+        CountShape c;
+        c.block = blocks[b];
+        c.grid = std::max(kXcds, (bpc[b] * cus) >> half);
+        cand.push_back(c);
+      }
     unsigned long long* ns = C.scalars.as<unsigned long long>(16) + 3;
     hipLaunchKernelGGL(k_min_u64, dim3(1), dim3(64), 0, C.stream, g.nwork, kSample, ns);
     g.nwork = ns;
@@ -2366,7 +2438,7 @@ void count_pass_graph(Context& C, const DevMesh& A, const DevMesh& B, long npair
   const CountShape s = C.shape[dim - 2];
   const std::vector<const void*> key = {
       reinterpret_cast<const void*>((long)dim), reinterpret_cast<const void*>(cap),
-      reinterpret_cast<const void*>(ngroups), reinterpret_cast<const void*>((long)(s.block * 4 + s.reg)),
+      reinterpret_cast<const void*>(ngroups), reinterpret_cast<const void*>((long)s.block),
       reinterpret_cast<const void*>((long)s.grid), g.npairs_dev, g.rows, g.cols, g.acoords, g.bcoords, g.asp,
       g.bsp, g.ascale, g.bscale, g.bplanes, g.counts, g.measure, parts, C.mflag.ptr, C.work.ptr, C.nwork.ptr,
       C.queue.ptr, scal, a_off, out->indptr, C.gpairs.ptr, C.gsum.ptr};
@@ -2518,52 +2590,68 @@ __global__ void __launch_bounds__(kClipBlock) k_clip_direct_tri_stream(DirectArg
 }
 
 // 3D: B's planes per pair (get_planes_tet, as staged for the bulk path) and
-// the depth-first walk of k_clip_tet_walk.
+// the clip of k_clip_tet_walk, one pair per quad and a fixed stride.
 __global__ void __launch_bounds__(kWalkBlock) k_clip_direct_tet(DirectArgs g) {
-  __shared__ double stack[(3 - kWalkReg) * 12 * kWalkBlock];
-  double* stk = stack + threadIdx.x;
-  double R[12 * kWalkReg];
-  const long stride = (long)gridDim.x * blockDim.x;
-  for (long p = (long)blockIdx.x * blockDim.x + threadIdx.x; p < g.npairs; p += stride) {
-    double A[12], Bv[12];
-    if (!gather_pair<3>(g, p, A, Bv)) {
-      g.counts[p] = -1;
-      g.measure[p] = 0.0;
-      continue;
-    }
-    Planes P;
-    tet_planes(Bv, P);
-    auto plane = [&](int j, double* o) {
+  __shared__ QuadLds<4> lds[kWalkBlock / 64];
+  __shared__ uint4 table[256];
+  for (int i = threadIdx.x; i < 256; i += kWalkBlock) table[i] = reinterpret_cast<const uint4*>(kSplitTable.e)[i];
+  __syncthreads();
+  QuadClip<4> W;
+  W.init(&lds[threadIdx.x >> 6], table);
+  const int q = W.q;
+  const long stride = (long)gridDim.x * (kWalkBlock / 4);
+  long next = ((long)blockIdx.x * kWalkBlock + threadIdx.x) >> 2, p = 0;
+  bool active = false;
+  int k = 0;
+  double tol = 0.0, m = 0.0;
+  while (true) {
+    if (!W.cur) {
+      if (W.pend) {
+        W.pop();
+      } else {
+        if (active && q == 0) {
+          g.counts[p] = k;
+          g.measure[p] = k == 0 ? 0.0 : m;
+        }
+        active = false;
+        double A[12], Bv[12];
+        while (next < g.npairs) {
+          p = next;
+          next += stride;
+          if (gather_pair<3>(g, p, A, Bv)) {
+            active = true;
+            break;
+          }
+          if (q == 0) {
+            g.counts[p] = -1;
+            g.measure[p] = 0.0;
+          }
+        }
+        if (!active) break;
+        tol = tet_tol(tet_volume_tet(A), tet_volume_tet(Bv));
+        m = 0.0;
+        k = 0;
+        Planes P;
+        tet_planes(Bv, P);
+        double pl[4], v[3];
 #pragma unroll
-      for (int i = 0; i < 3; i++) {
-        double v = in_reg(P.n[3][i]);
-        v = j == 2 ? in_reg(P.n[2][i]) : v;
-        v = j == 1 ? in_reg(P.n[1][i]) : v;
-        v = j == 0 ? in_reg(P.n[0][i]) : v;
-        o[i] = v;
+        for (int i = 0; i < 3; i++) {
+          pl[i] = q == 0 ? P.n[0][i] : (q == 1 ? P.n[1][i] : (q == 2 ? P.n[2][i] : P.n[3][i]));
+          v[i] = q == 0 ? A[i] : (q == 1 ? A[3 + i] : (q == 2 ? A[6 + i] : A[9 + i]));
+        }
+        pl[3] = q == 0 ? P.c[0] : (q == 1 ? P.c[1] : (q == 2 ? P.c[2] : P.c[3]));
+        W.set_plane(q, pl);
+        W.begin(v);
       }
-      double c = in_reg(P.c[3]);
-      c = j == 2 ? in_reg(P.c[2]) : c;
-      c = j == 1 ? in_reg(P.c[1]) : c;
-      c = j == 0 ? in_reg(P.c[0]) : c;
-      o[3] = c;
-    };
-    const double tol = tet_tol(tet_volume_tet(A), tet_volume_tet(Bv));
-    double p0[4], d0[4];
-    plane(0, p0);
-    walk_distances(A, p0, d0);
-    WalkState<4> W;
-    walk_begin(W, pack_class(d0));
-    double m = 0.0;
-    int nk = 0;
-    while (W.level > 0)
-      walk_next<4, kWalkBlock, kWalkReg>(W, A, R, stk, plane, tol, [&](const double* t, double, bool keep) {
-        const double vr = tet_volume_real(t);
-        m = m + (keep ? vr : 0.0);
-        nk += keep ? 1 : 0;
-      });
-    g.counts[p] = nk;
-    g.measure[p] = nk == 0 ? 0.0 : m;
+    }
+    W.step([&](const double* t, uint32_t lead) {
+      const bool keep = ((lead >> q) & 1u) && volume_reaches(t, tol);
+      const double vr = keep ? tet_volume_real(t) : 0.0;
+      m = m + quad_lane<0>(vr);
+      m = m + quad_lane<1>(vr);
+      m = m + quad_lane<2>(vr);
+      k += __builtin_popcount(quad_or((keep ? 1u : 0u) << q));
+    });
   }
 }
 
@@ -2626,7 +2714,7 @@ void clip_pairs_noalloc(int device, hipStream_t stream, const libsupermesh_gpu_m
       hipLaunchKernelGGL(k_clip_direct_tri_stream, dim3(64), dim3(kClipBlock), 0, stream, g);
     }
   } else if (npairs > 0) {
-    hipLaunchKernelGGL(k_clip_direct_tet, dim3(grid_for(npairs, kWalkBlock)), dim3(kWalkBlock), 0, stream, g);
+    hipLaunchKernelGGL(k_clip_direct_tet, dim3(grid_for(npairs, kWalkBlock / 4)), dim3(kWalkBlock), 0, stream, g);
   }
   hipLaunchKernelGGL(k_reduce_pairs, dim3(kClipGrid), dim3(kClipBlock), 0, stream, npairs, nullptr, counts, measure, parts);
   hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(kClipBlock), 0, stream, kClipGrid, parts);
