@@ -270,10 +270,9 @@ __device__ __forceinline__ void load_planes(const double* __restrict__ bp, long 
   }
 }
 
-// Output elements are written once and not read again by the pass that
+// Output triangles are written once and not read again by the pass that
 // writes them: streaming (nontemporal) stores keep them from evicting the
-// meshes' coordinates and planes that the clippers read from L2 (materialised
-// tet 96^3 vs 90^3: the fill walk and the single pass each 6 ms faster).
+// meshes' coordinates that the clippers read from L2.
 __device__ __forceinline__ void stream_tri(double* o, double x0, double y0, double x1, double y1, double x2,
                                            double y2) {
   __builtin_nontemporal_store(x0, o);
@@ -284,9 +283,14 @@ __device__ __forceinline__ void stream_tri(double* o, double x0, double y0, doub
   __builtin_nontemporal_store(y2, o + 5);
 }
 
-__device__ __forceinline__ void stream_tet(double* o, const double* t) {
+// Output tets, by one lane each in 16-byte words: plain stores, which L2
+// gathers into lines.  Streaming ones went out piecewise (5.6 GB written for
+// 2.5 GB of tets; fill of tet 32^3 vs 29^3 3.9 ms instead of 1.4, single pass
+// at 48^3 14.0 instead of 6.6), and writing the words of a quad's tets in
+// consecutive lanes gave nothing more.
+__device__ __forceinline__ void write_tet(double* o, const double* t) {
 #pragma unroll
-  for (int i = 0; i < 12; i++) __builtin_nontemporal_store(t[i], o + i);
+  for (int i = 0; i < 12; i++) o[i] = t[i];
 }
 
 // One 16-byte word of a run copy, stored the same way.
@@ -454,7 +458,7 @@ __global__ void __launch_bounds__(kClipBlock) k_clip(ClipArgs g) {
         m = m + vr;
         if (MASS) mass_element<3>(T.v, vr, affa, affb, blk);
         if (FILL && k < cap) {
-          stream_tet(g.elements + (off + k) * 12, T.v);
+          write_tet(g.elements + (off + k) * 12, T.v);
         }
         k++;
       });
@@ -736,57 +740,107 @@ constexpr int kWalkBlock = 128;
 // work list.
 constexpr int kXcds = 8;
 
-// The walk's quads take work items from queues (counters handing out up to
-// kQueueBatch consecutive items at a time): each XCD's share of the work list
-// is cut into kSubQueues contiguous parts, each with its own counter, so the
-// items in flight on an XCD stay a few compact windows of the list whose A
-// and B data its L2 holds (with fixed strides the quads drift apart over the
-// whole share), and no counter takes more than a fraction of the atomics.
-// A short list is handed out in smaller batches (about a quarter of the
-// items per quad, at least one): with 16 at a time, a list of a few
-// thousand items went to a few hundred lanes that walked 16 pairs each in
-// turn while the rest of the resident grid idled.
-constexpr int kQueueBatch = 16;
+// The walks' waves take work items from queues (counters handing out chunks
+// of consecutive items): each XCD's share of the work list is cut into
+// kSubQueues contiguous parts, each with its own counter, so the items in
+// flight on an XCD stay a few compact windows of the list whose A and B data
+// its L2 holds, and no counter takes more than a fraction of the atomics.  A
+// wave loads the pairs of a whole chunk at once, one item per lane, and deals
+// them to its quads as they finish: the chain of dependent loads (counter,
+// work list, pair) is paid once per chunk instead of once per item, and the
+// quads of a wave work on neighbouring pairs.  A short list is handed out in
+// chunks of a quarter of the items per wave, so that no wave holds work that
+// another could do.
 constexpr int kSubQueues = 4;
 constexpr int kQueues = kXcds * kSubQueues;
-struct WalkQueue {
+
+struct QuadItems {
   unsigned long long* counter;
-  long begin, end;  // this queue's part of the work list
-  long w = 0, wend = 0;
-  long batch = kQueueBatch;  // items per counter increment
-  // advance the quad (whole) to its next item; false when none is left
-  __device__ __forceinline__ bool next() {
-    if (++w < wend) return true;
-    unsigned long long got = 0;
-    if ((threadIdx.x & 3) == 0) got = atomicAdd(counter, (unsigned long long)batch);
-    got = (unsigned long long)quad_lane<0>((uint32_t)(got >> 32)) << 32 | quad_lane<0>((uint32_t)got);
-    const long s = begin + (long)got;
-    if (s >= end) return false;
-    w = s;
-    wend = s + batch < end ? s + batch : end;
-    return true;
+  long begin, end;         // this wave's part of the list
+  int chunk;               // items per counter increment, at most 64
+  int cnt = 0, used = 0;   // items of the current chunk, and how many are dealt
+  bool dry = false;        // the part has no further chunk
+  int p = 0, a = 0, b = 0, w = 0;  // this lane's item of the chunk: its pair, elements and list index
+
+  __device__ __forceinline__ void init(unsigned long long* queues, long n) {
+    const int nx = gridDim.x % kXcds == 0 ? kXcds : 1;
+    // every part needs blocks to drain it: a grid with fewer blocks per share
+    // than parts keeps one part per share
+    const int nsub = (int)(gridDim.x / nx) >= kSubQueues ? kSubQueues : 1;
+    const long xcd = blockIdx.x % nx, sub = (blockIdx.x / nx) % nsub;
+    const long per = (n + nx - 1) / nx;
+    const long b0 = xcd * per, e0 = b0 + per < n ? b0 + per : n;
+    const long sper = (e0 - b0 + nsub - 1) / nsub;
+    counter = queues + xcd * kSubQueues + sub;
+    begin = b0 + sub * sper < e0 ? b0 + sub * sper : e0;
+    end = begin + sper < e0 ? begin + sper : e0;
+    const long share = n / (4 * (long)gridDim.x * (blockDim.x / 64));
+    chunk = share < 1 ? 1 : (share < 64 ? (int)share : 64);
+  }
+
+  // The next chunk with an item to do: load(i, p, a, b) gives item i's pair
+  // and elements, or false to pass over it.
+  template <class Load>
+  __device__ __forceinline__ void refill(Load&& load) {
+    const int lane = threadIdx.x & 63;
+    cnt = used = 0;
+    while (cnt == 0 && !dry) {
+      unsigned long long got = 0;
+      if (lane == 0) got = atomicAdd(counter, (unsigned long long)chunk);
+      const long base = begin + (long)((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(got >> 32)) << 32 |
+                                       (unsigned)__builtin_amdgcn_readfirstlane((int)got));
+      if (base >= end) {
+        dry = true;
+        break;
+      }
+      const int n = end - base < chunk ? (int)(end - base) : chunk;
+      bool valid = false;
+      if (lane < n) {
+        w = (int)(base + lane);
+        valid = load(base + lane, p, a, b);
+      }
+      const unsigned long long m = __ballot(valid);
+      cnt = __popcll(m);
+      if (cnt < n) {  // close the gaps: the k-th valid item to lane k, the others behind
+        const int before = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
+        const int to = (valid ? before : cnt + lane - before) * 4;
+        p = __builtin_amdgcn_ds_permute(to, p);
+        a = __builtin_amdgcn_ds_permute(to, a);
+        b = __builtin_amdgcn_ds_permute(to, b);
+        w = __builtin_amdgcn_ds_permute(to, w);
+      }
+    }
+  }
+
+  // Deals an item to each quad that wants one (whole wave; want is the same
+  // in a quad's lanes), as far as the chunk and the next one go; true in the
+  // quads that got one.
+  template <class Load>
+  __device__ __forceinline__ bool take(bool want, int& ip, int& ia, int& ib, int& iw, Load&& load) {
+    const unsigned long long m = __ballot(want);
+    const int n = __popcll(m) >> 2;
+    const int rank = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0)) >> 2;
+    bool got = false;
+    int before = 0;  // quads served from the chunk that ran out
+    for (int pass = 0; pass < 2 && before < n; pass++) {
+      if (used == cnt && !dry) refill(load);
+      const int left = cnt - used, r = rank - before;
+      const bool now = want && r >= 0 && r < left;
+      const int src = now ? used + r : 0;
+      const int xp = __shfl(p, src, 64), xa = __shfl(a, src, 64), xb = __shfl(b, src, 64), xw = __shfl(w, src, 64);
+      ip = now ? xp : ip;
+      ia = now ? xa : ia;
+      ib = now ? xb : ib;
+      iw = now ? xw : iw;
+      got = got || now;
+      const int served = n - before < left ? n - before : left;
+      used += served;
+      before += served;
+      if (dry) break;
+    }
+    return got;
   }
 };
-
-__device__ __forceinline__ WalkQueue walk_queue(unsigned long long* queues, long n) {
-  const int nx = gridDim.x % kXcds == 0 ? kXcds : 1;
-  // every part needs blocks to drain it: a grid with fewer blocks per share
-  // than parts keeps one part per share
-  const int nsub = (int)(gridDim.x / nx) >= kSubQueues ? kSubQueues : 1;
-  const long xcd = blockIdx.x % nx, sub = (blockIdx.x / nx) % nsub;
-  const long per = (n + nx - 1) / nx;
-  const long b0 = xcd * per, e0 = b0 + per < n ? b0 + per : n;
-  const long sper = (e0 - b0 + nsub - 1) / nsub;
-  WalkQueue q;
-  q.counter = queues + xcd * kSubQueues + sub;
-  q.begin = b0 + sub * sper < e0 ? b0 + sub * sper : e0;
-  q.end = q.begin + sper < e0 ? q.begin + sper : e0;
-  q.w = -1;
-  q.wend = 0;
-  const long share = n / ((long)gridDim.x * blockDim.x);  // a quarter of the items per quad
-  q.batch = share < 1 ? 1 : (share < kQueueBatch ? share : kQueueBatch);
-  return q;
-}
 
 __global__ void k_zero_queues(unsigned long long* __restrict__ q) {
   if (threadIdx.x < kQueues && blockIdx.x == 0) q[threadIdx.x] = 0;
@@ -886,10 +940,32 @@ k_clip_tet_walk(ClipArgs g) {
   const int q = W.q;
   // blocks go to the XCDs round robin: each XCD takes one contiguous share
   // of the work list, so that its L2 holds one region of A and B
-  WalkQueue Q = walk_queue(g.queue, (long)*g.nwork);
-  bool more = Q.next();
+  const long nwork = (long)*g.nwork;
+  QuadItems Q;
+  Q.init(g.queue, nwork);
+  auto load = [&](long i, int& p, int& a, int& b) {
+    p = g.work[i];
+    a = g.rows[p];
+    b = g.cols[p];
+    // fill pass: pairs with output, or only those to be clipped again
+    return !FILL || (g.counts[p] > 0 && (!g.ovf || g.ovf[i] == 2));
+  };
+  // The quad's next item, its vertex and plane already on their way: loaded
+  // when the one before is begun, so that no quad waits for memory between
+  // items.  Not in the passes that write tets, where loads and stores
+  // complete in order and a load begun earlier would wait for the stores in
+  // between (single pass at tet 48^3: 6.95 ms instead of 6.64), nor with the
+  // mass, whose registers it would spill.  A list with few items per quad is
+  // not dealt ahead.
+  constexpr bool AHEAD = !FILL && !LEARNED && !MASS;
+  const bool ahead = AHEAD && nwork >= 8L * gridDim.x * (BLOCK / 4);
+  bool has_next = false;
+  int np = 0, na = 0, nb = 0, nw = 0, ncap = 0;
+  long noff = 0;
+  double nv[3] = {0.0, 0.0, 0.0}, nP[4] = {0.0, 0.0, 0.0, 0.0}, nsa = 0.0, nsb = 0.0;
   bool active = false;
-  long p = 0, off = 0, a = 0, b = 0;
+  long off = 0;
+  int p = 0, a = 0, b = 0, w = 0;
   int cap = 0, k = 0;
   // single pass: this quad's arena region, its fill level, and whether the
   // current pair's output outgrew budget and arena
@@ -900,70 +976,86 @@ k_clip_tet_walk(ClipArgs g) {
   unsigned nsplit = 0, nlost = 0;  // this quad's split runs and pairs to clip again
   double tol = 0.0, m = 0.0;
   TetMoments mom;
+  auto start = [&]() {
+    p = np;
+    a = na;
+    b = nb;
+    w = nw;
+    cap = ncap;
+    off = noff;
+    tol = 10.0 * fmin_f(nsa, nsb);
+    m = 0.0;
+    k = 0;
+    lost = false;
+    if (MASS) mom.clear();
+    W.set_plane(q, nP);
+    W.begin(nv);
+    active = true;
+    has_next = false;
+  };
   while (true) {
-    if (!W.cur) {
-      if (W.pend) {
-        W.pop();
-      } else {
-        if (active) {  // the pair is done
-          if (LEARNED) {
-            const bool any_lost = quad_or(lost ? 1u : 0u) != 0;
-            const bool split = k > cap && !any_lost;
-            if (q == 0) {
-              g.aoff[Q.w] = split ? abase + atop : -1;
-              g.dropped[Q.w] = any_lost ? 2 : (split ? 1 : 0);
-            }
-            if (split) atop += k - cap;
-            nsplit += split ? 1u : 0u;
-            nlost += any_lost ? 1u : 0u;
-          }
-          if (!FILL) {
-            if (q == 0) {
-              __builtin_nontemporal_store(k, g.counts + p);
-              __builtin_nontemporal_store(k == 0 ? 0.0 : m, g.measure + p);
-            }
-            if (MASS) {
-              double row[4] = {0.0, 0.0, 0.0, 0.0};
-              if (k > 0) mom.row(q, g.aaff + a * 12, g.baff + b * 12, row);
+    const bool idle = W.done();
+    if (idle && active) {  // the pair is done
+      if (LEARNED) {
+        const bool any_lost = quad_or(lost ? 1u : 0u) != 0;
+        const bool split = k > cap && !any_lost;
+        if (q == 0) {
+          g.aoff[w] = split ? abase + atop : -1;
+          g.dropped[w] = any_lost ? 2 : (split ? 1 : 0);
+        }
+        if (split) atop += k - cap;
+        nsplit += split ? 1u : 0u;
+        nlost += any_lost ? 1u : 0u;
+      }
+      if (!FILL) {
+        if (q == 0) {
+          g.counts[p] = k;
+          g.measure[p] = k == 0 ? 0.0 : m;
+        }
+        if (MASS) {
+          double row[4] = {0.0, 0.0, 0.0, 0.0};
+          if (k > 0) mom.row(q, g.aaff + (long)a * 12, g.baff + (long)b * 12, row);
 #pragma unroll
-              for (int j = 0; j < 4; j++) g.blocks[p * 16 + 4 * q + j] = row[j];
-            }
-          }
-          more = Q.next();
-          active = false;
+          for (int j = 0; j < 4; j++) g.blocks[(long)p * 16 + 4 * q + j] = row[j];
         }
-        // next work item of this quad (fill pass: skip pairs with no output)
-        while (more) {
-          p = g.work[Q.w];
-          if (!FILL) break;
-          cap = g.counts[p];
-          if (cap > 0 && (!g.ovf || g.ovf[Q.w] == 2)) break;
-          more = Q.next();
-        }
-        if (!more) break;
-        if (FILL) off = g.ovf ? g.aoff[Q.w] : g.offsets[p];
-        if (LEARNED) {
-          cap = (int)((g.budget[Q.w] >> g.bshift) & 0xffu);
-          off = g.offsets[p];
-          lost = false;
-        }
-        a = g.rows[p];
-        b = g.cols[p];
-        tol = 10.0 * fmin_f(g.asp[a], g.bsp[b]);
-        m = 0.0;
-        k = 0;
-        if (MASS) mom.clear();
+      }
+      active = false;
+    }
+    // Beginning an item costs the wave as much as a third of a step whether
+    // one quad does or all: four quads are waited for, unless few are left
+    // (tet 64^3 vs 60^3 count: 9.8 -> 9.2 ms; the sweep was flat from 3 to 5).
+    const int going = __popcll(__ballot(!idle));
+    if (AHEAD) {
+      const int ready = __popcll(__ballot(idle && has_next));
+      if ((ready >= 16 || going <= 16) && idle && has_next) start();
+    }
+    const bool want = !has_next && (ahead || !active);
+    const int wanting = __popcll(__ballot(want));
+    if ((AHEAD ? wanting > 0 : wanting >= 16 || (wanting > 0 && going <= 16)) && !(Q.dry && Q.used == Q.cnt)) {
+      const bool got = Q.take(want, np, na, nb, nw, load);
+      if (got) {
         // lane q brings in B's plane q and A's vertex q
-        double P[4], v[3];
 #pragma unroll
-        for (int i = 0; i < 4; i++) P[i] = g.bplanes[b * 16 + 4 * q + i];
+        for (int i = 0; i < 4; i++) nP[i] = g.bplanes[(long)nb * 16 + 4 * q + i];
 #pragma unroll
-        for (int i = 0; i < 3; i++) v[i] = g.acoords[a * 12 + 3 * q + i];
-        W.set_plane(q, P);
-        W.begin(v);
-        active = true;
+        for (int i = 0; i < 3; i++) nv[i] = g.acoords[(long)na * 12 + 3 * q + i];
+        nsa = g.asp[na];
+        nsb = g.bsp[nb];
+        if (FILL) {
+          ncap = g.counts[np];
+          noff = g.ovf ? g.aoff[nw] : g.offsets[np];
+        }
+        if (LEARNED) {
+          ncap = (int)((g.budget[nw] >> g.bshift) & 0xffu);
+          noff = g.offsets[np];
+        }
+        has_next = true;
+        if (!AHEAD) start();
       }
     }
+    if (!__any(active || has_next)) break;  // the list is dry
+    if (!active || W.done()) continue;
+    if (!W.cur) W.pop();
     W.step([&](const double* t, uint32_t lead) {
       const bool keep = ((lead >> q) & 1u) && volume_reaches(t, tol);
       const double vr = keep ? tet_volume_real(t) : 0.0;
@@ -986,12 +1078,12 @@ k_clip_tet_walk(ClipArgs g) {
       if (FILL || LEARNED) {
         const int at = k + __builtin_popcount(kept & ((1u << q) - 1u));
         if (keep && at < cap) {
-          stream_tet(g.elements + (off + at) * 12, t);
+          write_tet(g.elements + (off + at) * 12, t);
         } else if (LEARNED && keep) {
           // beyond the budget: the run continues in this quad's arena
           const long e = atop + (at - cap);
           if (e < g.arena_per_lane) {
-            stream_tet(g.elements + (abase + e) * 12, t);
+            write_tet(g.elements + (abase + e) * 12, t);
           } else {
             lost = true;
           }
@@ -1202,10 +1294,17 @@ k_clip_hex_walk(HexWalkArgs g) {
   W.init(&lds[threadIdx.x >> 6], table);
   const int q = W.q;
   // pairs from the walk's queues, as k_clip_tet_walk takes its work items
-  WalkQueue Q = walk_queue(g.queue, g.npairs);
-  bool more = Q.next();
+  QuadItems Q;
+  Q.init(g.queue, g.npairs);
+  auto load = [&](long i, int& p, int& a, int& b) {
+    p = (int)i;
+    a = g.rows[i];
+    b = g.cols[i];
+    return !FILL || g.counts[i] > 0;
+  };
   bool active = false;
-  long p = 0, off = 0, a = 0;
+  int p = 0, a = 0, b = 0, w = 0;
+  long off = 0;
   int cap = 0, k = 0, sub = 0;
   double tol = 0.0, m = 0.0;
   auto start = [&](const double* T) {
@@ -1216,59 +1315,53 @@ k_clip_hex_walk(HexWalkArgs g) {
     W.begin(v);
   };
   while (true) {
-    if (!W.cur) {
-      if (W.pend) {
-        W.pop();
-      } else {
-        double T[12];
-        if (MODE == 2 && active && sub < 4) {
-          sub++;
-          hex_split_tet(g.acoords + a * 24, sub, T);
-        } else {
-          if (active) {
-            if (!FILL && q == 0) {
-              __builtin_nontemporal_store(k, g.counts + p);
-              __builtin_nontemporal_store(k == 0 ? 0.0 : m, g.measure + p);
-            }
-            more = Q.next();
-            active = false;
-          }
-          while (more) {
-            p = Q.w;
-            if (!FILL) break;
-            cap = g.counts[p];
-            if (cap > 0) break;
-            more = Q.next();
-          }
-          if (!more) break;
-          if (FILL) off = g.offsets[p];
-          a = g.rows[p];
-          const long b = g.cols[p];
-          const double* planes = g.hplanes + (MODE == 1 ? a : b) * 24;
-          double P[4];
-#pragma unroll
-          for (int i = 0; i < 4; i++) P[i] = planes[4 * q + i];
-          W.set_plane(q, P);
-          if (q < 2) {
-#pragma unroll
-            for (int i = 0; i < 4; i++) P[i] = planes[16 + 4 * q + i];
-            W.set_plane(4 + q, P);
-          }
-          if (MODE == 2) {
-            sub = 0;
-            hex_split_tet(g.acoords + a * 24, 0, T);
-          } else {
-            const double* t = MODE == 0 ? g.acoords + a * 12 : g.bcoords + b * 12;
-#pragma unroll
-            for (int i = 0; i < 12; i++) T[i] = t[i];
-          }
-          m = 0.0;
-          k = 0;
-          active = true;
+    if (MODE == 2 && active && W.done() && sub < 4) {
+      sub++;
+      double T[12];
+      hex_split_tet(g.acoords + (long)a * 24, sub, T);
+      start(T);
+    }
+    if (active && W.done()) {
+      if (!FILL && q == 0) {
+        __builtin_nontemporal_store(k, g.counts + p);
+        __builtin_nontemporal_store(k == 0 ? 0.0 : m, g.measure + p);
+      }
+      active = false;
+    }
+    if (__any(!active) && !(Q.dry && Q.used == Q.cnt)) {
+      const bool got = Q.take(!active, p, a, b, w, load);
+      if (got) {
+        if (FILL) {
+          cap = g.counts[p];
+          off = g.offsets[p];
         }
+        const double* planes = g.hplanes + (long)(MODE == 1 ? a : b) * 24;
+        double P[4], T[12];
+#pragma unroll
+        for (int i = 0; i < 4; i++) P[i] = planes[4 * q + i];
+        W.set_plane(q, P);
+        if (q < 2) {
+#pragma unroll
+          for (int i = 0; i < 4; i++) P[i] = planes[16 + 4 * q + i];
+          W.set_plane(4 + q, P);
+        }
+        if (MODE == 2) {
+          sub = 0;
+          hex_split_tet(g.acoords + (long)a * 24, 0, T);
+        } else {
+          const double* t = MODE == 0 ? g.acoords + (long)a * 12 : g.bcoords + (long)b * 12;
+#pragma unroll
+          for (int i = 0; i < 12; i++) T[i] = t[i];
+        }
+        m = 0.0;
+        k = 0;
         start(T);
+        active = true;
       }
     }
+    if (!__any(active)) break;  // no pair is left
+    if (!active || W.done()) continue;
+    if (!W.cur) W.pop();
     W.step([&](const double* t, uint32_t lead) {
       const bool keep = ((lead >> q) & 1u) && volume_reaches(t, tol);
       const double vr = keep ? tet_volume_real(t) : 0.0;
@@ -1278,7 +1371,7 @@ k_clip_hex_walk(HexWalkArgs g) {
       const uint32_t kept = quad_or((keep ? 1u : 0u) << q);
       if (FILL) {
         const int at = k + __builtin_popcount(kept & ((1u << q) - 1u));
-        if (keep && at < cap) stream_tet(g.elements + (off + at) * 12, t);
+        if (keep && at < cap) write_tet(g.elements + (off + at) * 12, t);
       }
       k += __builtin_popcount(kept);
     });
@@ -1333,7 +1426,7 @@ static void launch_hex_walk_as(Context& C, const HexWalkArgs& g) {
   const long resident = (long)blocks_per_cu * (cus > 0 ? cus : 256);
   const long need = (g.npairs + kHexBlock / 4 - 1) / (kHexBlock / 4);
   unsigned blocks = (unsigned)std::max(1L, std::min(resident, need));
-  if (blocks >= kXcds) blocks -= blocks % kXcds;  // whole XCD shares (walk_queue)
+  if (blocks >= kXcds) blocks -= blocks % kXcds;  // whole XCD shares (QuadItems)
   HexWalkArgs h = g;
   h.queue = walk_queues(C);
   hipLaunchKernelGGL((k_clip_hex_walk<MODE, FILL>), dim3(blocks), dim3(kHexBlock), 0, C.stream, h);

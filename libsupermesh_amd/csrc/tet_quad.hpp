@@ -30,8 +30,7 @@ namespace lsm {
 // 2 outside (d > 0), 3 none of these (NaN), as the split's case counts them
 // (Tetrahedron_Intersection.F90:264-276).
 LSM_HD unsigned side_code(double d) {
-  unsigned c = d < 0.0 ? 1u : (d > 0.0 ? 2u : 3u);
-  return __builtin_fabs(d) < kEpsilon ? 0u : c;
+  return (d > -kEpsilon ? 0u : 1u) | (d < kEpsilon ? 0u : 2u);
 }
 
 // How a tet whose vertices have these sides against the splitting plane is
@@ -135,9 +134,13 @@ LSM_HD unsigned planes_cut(uint32_t s, unsigned* inside) {
 // Index of the split table for plane j (0..3) of code word s.
 LSM_HD unsigned case_index(uint32_t s, int j) {
   const uint32_t x = (s >> (2 * j)) & 0x03030303u;
+#ifdef __HIP_DEVICE_COMPILE__
+  return __builtin_amdgcn_udot4(x, 0x40100401u, 0u, false);
+#else
   // gathers the four bytes' low pairs into the top byte; no two partial
   // products share a bit, so nothing carries
   return (x * 0x01041040u) >> 24;
+#endif
 }
 
 // s with every vertex inside planes 0..j.
@@ -249,9 +252,12 @@ struct QuadClip {
   int q;            // lane of the quad
   uint32_t T;       // the current tet's vertex ids
   uint32_t S[SW];   // and their sides
-  uint32_t pend;    // pending stack entries: 3 a row, a later child lower
+  uint32_t pend;    // pending stack entries: four bits a row, child 0 highest, the lowest unused
   int r;            // row of the next split's points
   bool cur;         // T is to be done
+  // planes 1..NP-1, which every new vertex is classified against (in LDS they
+  // took a fifth of its traffic, which bounds the step beside the VALU)
+  double P[NP - 1][4];
 
   __device__ __forceinline__ void init(QuadLds<NP>* lds, const uint4* tab) {
     const int lane = threadIdx.x & 63, g = lane >> 2;
@@ -281,22 +287,16 @@ struct QuadClip {
     for (int k = 0; k < 3; k++) v[k] = pool[k * kRows + id];
   }
 
-  // Sides of a vertex against planes FROM..NP-1, as code bytes (the planes
-  // below read "inside").
-  template <int FROM>
-  __device__ __forceinline__ void sides(const double* v, uint32_t* c) const {
+  // Sides of a vertex against planes 1..NP-1, as code bytes; plane 0 reads
+  // side0.
+  __device__ __forceinline__ void sides(const double* v, unsigned side0, uint32_t* c) const {
 #pragma unroll
     for (int w = 0; w < SW; w++) {
-      c[w] = 0;
+      c[w] = w == 0 ? side0 : 0u;
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
+      for (int j = w == 0 ? 1 : 0; j < 4; j++) {
         const int p = 4 * w + j;
-        unsigned s = 1u;
-        if (p >= FROM && p < NP) {
-          double P[4];
-          get_plane(p, P);
-          s = side_code(plane_distance(P, v));
-        }
+        const unsigned s = p < NP ? side_code(plane_distance(P[p < NP ? p - 1 : 0], v)) : 1u;
         c[w] |= s << (2 * j);
       }
     }
@@ -312,8 +312,12 @@ struct QuadClip {
 #pragma unroll
     for (int k = 0; k < 3; k++) pool[k * kRows + q] = v[k];
     quad_fence();
+#pragma unroll
+    for (int j = 1; j < NP; j++) get_plane(j, P[j - 1]);
+    double P0[4];
+    get_plane(0, P0);
     uint32_t c[SW];
-    sides<0>(v, c);
+    sides(v, side_code(plane_distance(P0, v)), c);
     gather_codes(c, S);
     T = 0x03020100u;
     pend = 0;
@@ -324,10 +328,11 @@ struct QuadClip {
   __device__ __forceinline__ void pop() {
     const int e = 31 - __builtin_clz(pend);
     pend ^= 1u << e;
-    r = e / 3 + 2;
-    T = stk[e * kWords * 16];
+    r = (e >> 2) + 2;
+    const int at = (e - 1 - (e >> 2)) * kWords * 16;
+    T = stk[at];
 #pragma unroll
-    for (int w = 0; w < SW; w++) S[w] = stk[(e * kWords + 1 + w) * 16];
+    for (int w = 0; w < SW; w++) S[w] = stk[at + (1 + w) * 16];
   }
 
   // Cuts the current tet by the first plane that cuts it.  Calls leaf(t,
@@ -355,21 +360,22 @@ struct QuadClip {
       sc = table[case_index(sj, j & 3)];
       // this lane's split point
       const uint32_t b = sc.w >> (8 * q);
-      double P[4], vp[3], vn[3], x[3];
-      get_plane(j, P);
+      double pj[4], vp[3], vn[3], x[3];
+      get_plane(j, pj);
       vertex((T >> (b & 24u)) & 255u, vp);
       vertex((T >> ((b << 3) & 24u)) & 255u, vn);
-      split_edge(plane_distance(P, vp), plane_distance(P, vn), vp, vn, x);
+      split_edge(plane_distance(pj, vp), plane_distance(pj, vn), vp, vn, x);
 #pragma unroll
       for (int k = 0; k < 3; k++) pool[k * kRows + 16 * r + q] = x[k];
       uint32_t c[SW];
-      sides<1>(x, c);
+      sides(x, 1u, c);  // any split is by plane 0 or later
       gather_codes(c, rowS);
     }
     quad_fence();
     // the children, one per lane
     const uint32_t sel = q == 0 ? sc.x : (q == 1 ? sc.y : sc.z);
-    const uint32_t ct = byte_permute((uint32_t)r * 0x10101010u + 0x03020100u, T, sel);
+    const uint32_t row = byte_permute(0u, (uint32_t)r << 4, 0u) + 0x03020100u;  // the new points' ids
+    const uint32_t ct = byte_permute(row, T, sel);
     uint32_t cs[SW];
     unsigned ccut = 0, cin = 0;
 #pragma unroll
@@ -392,14 +398,14 @@ struct QuadClip {
     if ((kinds & 15u & ~lead | more) != 0) {
       const bool keep = mine && !((lead >> q) & 1u) && (whole || cuts);
       if (keep) {
-        const int e = 3 * r - 1 - q;
-        stk[e * kWords * 16] = ct;
+        const int at = (3 * r - 1 - q) * kWords * 16;  // row r's entries 3 r - 3 .. 3 r - 1, child 0 last
+        stk[at] = ct;
 #pragma unroll
-        for (int w = 0; w < SW; w++) stk[(e * kWords + 1 + w) * 16] = cs[w];
+        for (int w = 0; w < SW; w++) stk[at + (1 + w) * 16] = cs[w];
       }
-      // children 0, 1, 2 at bits 3 r - 1, 3 r - 2, 3 r - 3
+      // children 0, 1, 2 at bits 3, 2, 1 of the row's four
       const uint32_t left = (kinds & 15u & ~lead) | more;
-      pend |= (((left & 1u) << 2) | (left & 2u) | ((left >> 2) & 1u)) << (3 * r - 3);
+      pend |= (__builtin_bitreverse32(left) >> 28) << (4 * r - 4);
     }
     cur = false;
     if (lead) {
