@@ -81,7 +81,7 @@ static void free_context(Context& C) {
                     &C.predictor.features, &C.predictor.labels, &C.predictor.act,
                     &C.predictor.loss, &C.predictor.index, &C.predictor.budget,
                     &C.predictor.overflow, &C.predictor.spill, &C.predictor.aoff, &C.offsets_dense, &C.queue,
-                    &C.elements_dense, &C.dense_ctl, &C.fscratch};
+                    &C.elements_dense, &C.dense_ctl, &C.ftasks, &C.fspan, &C.fcount};
   release_graph(C);
   for (DevBuf* b : bufs) b->release();
   if (C.hstat) hipHostFree(C.hstat);

@@ -12,16 +12,14 @@
 // centres and grouped into an implicit F-ary hierarchy (node i of level l
 // covers children [F*i, F*i+F) of level l-1; level 0 = elements).  Internal
 // boxes are exact unions, so pruning with the same predicate never loses a
-// pair.  A elements are visited in Morton order, one per lane, with a
-// stackless depth-first walk (level, index) that needs no per-lane stack.
-// A count pass sizes the CSR rows, a fill pass writes them, and each row is
-// then sorted by B id so the output is canonical.
+// pair.  A elements are taken in Morton order, 32 to a wave, which walks the
+// union of their depth-first paths; a row is in leaf order.  A count pass
+// sizes the CSR rows, a fill pass writes them.
 #include <cstring>
 #include <utility>
 #include <vector>
 
 #include <rocprim/device/device_radix_sort.hpp>
-#include <rocprim/device/device_reduce.hpp>
 #include <rocprim/device/device_segmented_radix_sort.hpp>
 #include <rocprim/device/device_scan.hpp>
 
@@ -454,12 +452,13 @@ void build_bvh(Context& C, const DevMesh& B) {
   H.levels = L;
   H.total = total;
   int w = 2 * B.dim;
-  double* boxes = H.boxes.as<double>((size_t)total * w);
+  // a walk reads whole groups of children, past the last node too
+  double* boxes = H.boxes.as<double>((size_t)(total + kFanout) * w);
   const double* bbox = static_cast<const double*>(B.bbox.ptr);
   const int* perm = static_cast<const int*>(H.perm.ptr);
   H.grouped = B.ngroups > 0;
   const int* group = H.grouped ? static_cast<const int*>(B.group.ptr) : nullptr;
-  int* gr = H.grouped ? H.granges.as<int>((size_t)total * 2) : nullptr;
+  int* gr = H.grouped ? H.granges.as<int>((size_t)(total + kFanout) * 2) : nullptr;
   if (B.dim == 2)
     hipLaunchKernelGGL(k_leaf_boxes<2>, dim3(grid_for(H.n, kBlock)), dim3(kBlock), 0, C.stream, H.n,
                        bbox, perm, boxes, group, gr);
@@ -485,291 +484,402 @@ void build_bvh(Context& C, const DevMesh& B) {
 // Traversal
 // ---------------------------------------------------------------------------
 
+// Raises *max to the largest x of the wave; the value read first spares
+// nearly all waves the atomic.
+__device__ __forceinline__ void raise_max(long* max, int x) {
+  for (int o = 32; o > 0; o >>= 1) {
+    const int y = __shfl_xor(x, o, 64);
+    x = y > x ? y : x;
+  }
+  if ((threadIdx.x & 63) == 0 && x > *reinterpret_cast<volatile long*>(max)) atomicMax(reinterpret_cast<unsigned long long*>(max), (unsigned long long)x);
+}
+
+__global__ void k_clear_words(int n, long* __restrict__ w) {
+  if ((int)threadIdx.x < n && blockIdx.x == 0) w[threadIdx.x] = 0;
+}
+
+struct SearchArgs {
+  long na;
+  const int* qperm;     // A's elements in Morton order, kQueries to a wave
+  const double* abox;   // [2 DIM][na]
+  const int* agroup;    // batches: A's and the nodes' meshes
+  const int* granges;
+  const double* boxes;
+  const int* perm;
+  LevelInfo info;
+  // tasks: (query wave, node at `level`) pairs; without them, every wave
+  // starts at the root
+  const int2* tasks;
+  const unsigned* ntasks;
+  unsigned cap;         // tasks that the arrays hold
+  int level;
+  int* tcount;          // [cap][kQueries]: results of the wave's queries below the task's node, then their prefix sums
+  long* row_count;      // [na]
+  long* maxrow;
+  const long* indptr;
+  int* indices;
+  int* rows;
+};
+
+// A wave tests its queries eight at a time against a node's eight children:
+// lane 8 q + c holds child c's box and the queries q of each of the kGroups
+// groups of eight.  A node's boxes are then three loads for the wave, one
+// compare tests 64 (query, child) pairs, and a query's results lie in
+// neighbouring lanes, so that they are written together.
+constexpr int kGroups = 4;
+constexpr int kQueries = 8 * kGroups;
+
+template <int DIM, bool GROUPED>
+struct Queries {
+  int a[kGroups], g[kGroups];
+  double lo[kGroups][DIM], hi[kGroups][DIM];
+  __device__ __forceinline__ Queries(const SearchArgs& s, long wave) {
+#pragma unroll
+    for (int i = 0; i < kGroups; i++) {
+      const long t = wave * kQueries + 8 * i + ((threadIdx.x & 63) >> 3);
+      const bool live = t < s.na;
+      a[i] = live ? s.qperm[t] : -1;
+#pragma unroll
+      for (int d = 0; d < DIM; d++) {  // no box overlaps NaN bounds
+        lo[i][d] = live ? s.abox[(long)d * s.na + a[i]] : __builtin_nan("");
+        hi[i][d] = live ? s.abox[(long)(DIM + d) * s.na + a[i]] : __builtin_nan("");
+      }
+      g[i] = GROUPED && live ? s.agroup[a[i]] : -1;
+    }
+  }
+};
+
+// Lanes of `start` whose box [lo, hi] (and mesh range) overlaps the query:
+// each compare narrows the execution mask that the next one runs under, so
+// the conjunction costs no mask arithmetic on the scalar unit, which one walk
+// with a scalar `and` per compare was bound by.  `full` is the mask to go on
+// with.  Strict: hi > qlo and lo < qhi (Quadtree_...F90:411-420); closed: not
+// strict.
 template <int DIM, bool CLOSED>
-__device__ __forceinline__ bool overlaps(const double* __restrict__ box, const double* qlo,
-                                         const double* qhi) {
-  bool hit = true;
-#pragma unroll
-  for (int d = 0; d < DIM; d++) {
-    double lo = box[d], hi = box[DIM + d];
-    // strict: b.max > a.min and b.min < a.max (Quadtree_...F90:411-420)
-    hit = hit && (CLOSED ? (hi >= qlo[d] && lo <= qhi[d]) : (hi > qlo[d] && lo < qhi[d]));
-  }
-  return hit;
-}
-
-template <int DIM, bool CLOSED, bool FILL, bool GROUPED>
-__global__ void __launch_bounds__(kBlock)
-k_query(long na, const int* __restrict__ qperm, const double* __restrict__ abox, LevelInfo info,
-        const double* __restrict__ boxes, const int* __restrict__ perm, long* __restrict__ row_count,
-        const long* __restrict__ indptr, int* __restrict__ indices, int* __restrict__ rows,
-        const int* __restrict__ agroup, const int* __restrict__ granges, long skip_upto) {
-  long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= na) return;
-  const int a = qperm[t];
-  // fill pass after the single pass: only the rows that outgrew its scratch
-  if (FILL && row_count[a] <= skip_upto) return;
-  // in a batch, only nodes whose mesh range holds A's mesh are visited
-  const int g = GROUPED ? agroup[a] : 0;
-  double qlo[DIM], qhi[DIM];
-#pragma unroll
-  for (int d = 0; d < DIM; d++) {
-    qlo[d] = abox[(long)d * na + a];
-    qhi[d] = abox[(long)(DIM + d) * na + a];
-  }
-  const int top = info.levels - 1;
-  long base = FILL ? indptr[a] : 0;
-  long cnt = 0;
-  int l = top;
-  long i = 0;
-  while (true) {
-    bool hit = false;
-    if (i < info.count[l]) {
-      hit = overlaps<DIM, CLOSED>(boxes + (info.offset[l] + i) * 2 * DIM, qlo, qhi);
-      if (GROUPED) {
-        const int* r = granges + 2 * (info.offset[l] + i);
-        hit = hit && r[0] <= g && g <= r[1];
-      }
-    }
-    if (hit) {
-      if (l == 0) {
-        if (FILL) {
-          indices[base + cnt] = perm[i];
-          rows[base + cnt] = a;
-        }
-        cnt++;
-      } else {
-        l--;
-        i *= kFanout;
-        continue;
-      }
-    }
-    // advance to the next sibling, climbing while at the end of a group
-    bool done = false;
-    while (true) {
-      if (l == top) {
-        done = true;
-        break;
-      }
-      if ((i % kFanout) != kFanout - 1 && i + 1 < info.count[l]) {
-        i++;
-        break;
-      }
-      i /= kFanout;
-      l++;
-    }
-    if (done) break;
-  }
-  if (!FILL) row_count[a] = cnt;
-}
-
-// Boxes of the up to F children first .. first+F-1 of level K that overlap
-// the query, as a bit mask.
-template <int DIM, bool CLOSED, bool GROUPED>
-__device__ __forceinline__ unsigned child_mask(const LevelInfo& info, const double* __restrict__ boxes,
-                                               const int* __restrict__ granges, int K, long first,
-                                               const double* qlo, const double* qhi, int g) {
-  const long n = info.count[K];
-  const long base = info.offset[K] + first;
-  unsigned m = 0;
-#pragma unroll
-  for (int c = 0; c < kFanout; c++) {
-    if (first + c < n) {
-      bool hit = overlaps<DIM, CLOSED>(boxes + (base + c) * 2 * DIM, qlo, qhi);
-      if (GROUPED) {
-        const int* r = granges + 2 * (base + c);
-        hit = hit && r[0] <= g && g <= r[1];
-      }
-      m |= (unsigned)hit << c;
-    }
+__device__ __forceinline__ unsigned long long overlap_lanes(unsigned long long start, unsigned long long full,
+                                                            const double* lo, const double* hi, const double* qlo,
+                                                            const double* qhi) {
+  unsigned long long m;
+  if constexpr (DIM == 2) {
+    if constexpr (CLOSED)
+      asm volatile("s_mov_b64 exec, %1\n\tv_cmpx_ge_f64 vcc, %3, %4\n\tv_cmpx_le_f64 vcc, %5, %6\n\t"
+                   "v_cmpx_ge_f64 vcc, %7, %8\n\tv_cmpx_le_f64 vcc, %9, %10\n\ts_mov_b64 %0, exec\n\ts_mov_b64 exec, %2"
+                   : "=&s"(m)
+                   : "s"(start), "s"(full), "v"(hi[0]), "v"(qlo[0]), "v"(lo[0]), "v"(qhi[0]), "v"(hi[1]), "v"(qlo[1]),
+                     "v"(lo[1]), "v"(qhi[1])
+                   : "vcc");
+    else
+      asm volatile("s_mov_b64 exec, %1\n\tv_cmpx_gt_f64 vcc, %3, %4\n\tv_cmpx_lt_f64 vcc, %5, %6\n\t"
+                   "v_cmpx_gt_f64 vcc, %7, %8\n\tv_cmpx_lt_f64 vcc, %9, %10\n\ts_mov_b64 %0, exec\n\ts_mov_b64 exec, %2"
+                   : "=&s"(m)
+                   : "s"(start), "s"(full), "v"(hi[0]), "v"(qlo[0]), "v"(lo[0]), "v"(qhi[0]), "v"(hi[1]), "v"(qlo[1]),
+                     "v"(lo[1]), "v"(qhi[1])
+                   : "vcc");
+  } else {
+    if constexpr (CLOSED)
+      asm volatile("s_mov_b64 exec, %1\n\tv_cmpx_ge_f64 vcc, %3, %4\n\tv_cmpx_le_f64 vcc, %5, %6\n\t"
+                   "v_cmpx_ge_f64 vcc, %7, %8\n\tv_cmpx_le_f64 vcc, %9, %10\n\tv_cmpx_ge_f64 vcc, %11, %12\n\t"
+                   "v_cmpx_le_f64 vcc, %13, %14\n\ts_mov_b64 %0, exec\n\ts_mov_b64 exec, %2"
+                   : "=&s"(m)
+                   : "s"(start), "s"(full), "v"(hi[0]), "v"(qlo[0]), "v"(lo[0]), "v"(qhi[0]), "v"(hi[1]), "v"(qlo[1]),
+                     "v"(lo[1]), "v"(qhi[1]), "v"(hi[2]), "v"(qlo[2]), "v"(lo[2]), "v"(qhi[2])
+                   : "vcc");
+    else
+      asm volatile("s_mov_b64 exec, %1\n\tv_cmpx_gt_f64 vcc, %3, %4\n\tv_cmpx_lt_f64 vcc, %5, %6\n\t"
+                   "v_cmpx_gt_f64 vcc, %7, %8\n\tv_cmpx_lt_f64 vcc, %9, %10\n\tv_cmpx_gt_f64 vcc, %11, %12\n\t"
+                   "v_cmpx_lt_f64 vcc, %13, %14\n\ts_mov_b64 %0, exec\n\ts_mov_b64 exec, %2"
+                   : "=&s"(m)
+                   : "s"(start), "s"(full), "v"(hi[0]), "v"(qlo[0]), "v"(lo[0]), "v"(qhi[0]), "v"(hi[1]), "v"(qlo[1]),
+                     "v"(lo[1]), "v"(qhi[1]), "v"(hi[2]), "v"(qlo[2]), "v"(lo[2]), "v"(qhi[2])
+                   : "vcc");
   }
   return m;
 }
 
-// OR of an 8-bit mask over the wave's active lanes (uniform result).
-__device__ __forceinline__ unsigned wave_or8(unsigned x) {
-  unsigned r = 0;
+// Bit c of the result: some query's byte has bit c.
+__device__ __forceinline__ unsigned any_query(const unsigned long long* m) {
+  unsigned long long u = 0;
 #pragma unroll
-  for (int b = 0; b < 8; b++) r |= (__ballot((x >> b) & 1u) != 0ULL ? 1u : 0u) << b;
-  return r;
+  for (int i = 0; i < kGroups; i++) u |= m[i];
+  unsigned v = (unsigned)u | (unsigned)(u >> 32);
+  v |= v >> 16;
+  return (v | v >> 8) & 0xffu;
 }
 
-// Single-pass search: the same depth-first order as k_query, but a node's
-// children are tested together (their boxes are contiguous) and the walk
-// keeps, per level, a byte of the hit children not yet visited; the node
-// index is implicit (parent = child / F).  The first `cap` results of a query
-// go to scratch (slot-major: scratch[k * na + t]); all are counted.  The wave
-// walks one path: the union of its 64 queries' paths (consecutive queries are
-// close in Morton order, so their paths mostly coincide).  Every lane tests the children of the wave's current node
-// (the same boxes: one broadcast load per box, no divergent gathers) and
-// keeps its own per-level hit masks, so its hits, and their order, are those
-// of its own depth-first walk alone: each level's union mask is
-// consumed lowest child first, which is each lane's own order.
+// Visits the nodes below `start` (a node of level `from`, above `to`) whose
+// children at level `to` some query overlaps, in index order: hit(first, m)
+// with the first child's index and, per group, bit 8 q + c where query q
+// overlaps child c.  The wave walks the union of its queries' depth-first
+// paths (consecutive queries are close in Morton order, so their paths mostly
+// coincide) and keeps, per level, a byte of the children still to visit.  A
+// query may be tested against a node whose parent it misses: the boxes are
+// exact unions, so it misses that node too.  from == to: start itself, as
+// the only child.
+template <int DIM, bool CLOSED, bool GROUPED, class Hit>
+__device__ __forceinline__ void walk_union(const SearchArgs& s, const Queries<DIM, GROUPED>& Q, int from, long start,
+                                           int to, Hit&& hit) {
+  const int c = threadIdx.x & 7;
+  const unsigned long long full = __ballot(true);
+  // level l's first node and node count, in lane l
+  const int lane = threadIdx.x & 63;
+  const long my_offset = lane < 32 ? s.info.offset[lane & 31] : 0, my_count = lane < 32 ? s.info.count[lane & 31] : 0;
+  auto at_level = [](long x, int l) {
+    return (long)((unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(x >> 32), l) << 32 |
+                  (unsigned)__builtin_amdgcn_readlane((int)x, l));
+  };
+  // the boxes (and mesh ranges) of a node's children, child c in this lane
+  struct Boxes {
+    double lo[DIM], hi[DIM];
+    int2 r;
+  };
+  auto load = [&](long at, Boxes& x) {
+    const long b = (at + c) * 2 * DIM;
+#pragma unroll
+    for (int d = 0; d < DIM; d++) {
+      x.lo[d] = s.boxes[b + d];
+      x.hi[d] = s.boxes[b + DIM + d];
+    }
+    if (GROUPED) x.r = *reinterpret_cast<const int2*>(s.granges + 2 * (at + c));
+  };
+  unsigned long long m[kGroups];
+  auto test = [&](const Boxes& x, long n) {  // the first n children
+    const unsigned long long in = __ballot(c < n);
+#pragma unroll
+    for (int i = 0; i < kGroups; i++) {
+      // in a batch, only nodes whose mesh range holds A's mesh are visited
+      const unsigned long long meshes = GROUPED ? in & __ballot(x.r.x <= Q.g[i] && Q.g[i] <= x.r.y) : in;
+      m[i] = overlap_lanes<DIM, CLOSED>(meshes, full, x.lo, x.hi, Q.lo[i], Q.hi[i]);
+    }
+  };
+  Boxes x, y;
+  load(at_level(my_offset, from) + start, x);
+  test(x, 1);
+  if (any_query(m) == 0) return;
+  if (from == to) {
+    hit(start, m);
+    return;
+  }
+  const long to_offset = at_level(my_offset, to), to_count = at_level(my_count, to);
+  if (from == to + 1) {
+    load(to_offset + start * kFanout, x);
+    test(x, to_count - start * kFanout);
+    hit(start * kFanout, m);
+    return;
+  }
+  // levels to + 2 .. from, a byte each (1..8 and 9..16): the children to visit
+  unsigned long long ulo = 0, uhi = 0;
+  int L = from;
+  long node = start;
+  while (true) {
+    const long first = node * kFanout;
+    load(at_level(my_offset, L - 1) + first, x);
+    test(x, at_level(my_count, L - 1) - first);
+    unsigned u = any_query(m);
+    if (L - 1 == to + 1) {
+      // the children's children are what is asked for: two nodes' boxes on
+      // their way at a time
+      while (u) {
+        const int k = __builtin_ctz(u);
+        u &= u - 1;
+        const int k2 = u ? __builtin_ctz(u) : k;
+        u &= u - 1u;
+        const long f = (first + k) * kFanout, f2 = (first + k2) * kFanout;
+        load(to_offset + f, x);
+        load(to_offset + f2, y);
+        test(x, to_count - f);
+        hit(f, m);
+        if (k2 == k) break;
+        test(y, to_count - f2);
+        hit(f2, m);
+      }
+    } else if (L <= 8) {
+      ulo |= (unsigned long long)u << (8 * (L - 1));
+    } else {
+      uhi |= (unsigned long long)u << (8 * (L - 9));
+    }
+    // the next node: a child of this one, or of the nearest with one left
+    while (true) {
+      u = L - 1 == to + 1 ? 0u
+                          : (L <= 8 ? (unsigned)(ulo >> (8 * (L - 1))) : (unsigned)(uhi >> (8 * (L - 9)))) & 0xffu;
+      if (u || L == from) break;
+      node /= kFanout;
+      L++;
+    }
+    if (u == 0) break;
+    const int k = __builtin_ctz(u);
+    if (L <= 8) ulo &= ~(1ULL << (8 * (L - 1) + k));
+    else uhi &= ~(1ULL << (8 * (L - 9) + k));
+    node = node * kFanout + k;
+    L--;
+  }
+}
+
+// The wave's index in the grid, as a scalar.
+__device__ __forceinline__ long grid_wave() {
+  return (long)blockIdx.x * (kBlock / 64) + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+}
+
+// Splits long walks: for every query wave, the nodes at `level` that its
+// queries overlap, one task each.  A wave's tasks are consecutive and in node
+// order; first[w] and count[w] say which.
 template <int DIM, bool CLOSED, bool GROUPED>
 __global__ void __launch_bounds__(kBlock)
-k_query_wave(long na, const int* __restrict__ qperm, const double* __restrict__ abox, LevelInfo info,
-             const double* __restrict__ boxes, const int* __restrict__ perm, int cap,
-             int* __restrict__ scratch, long* __restrict__ row_count, const int* __restrict__ agroup,
-             const int* __restrict__ granges) {
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= na) return;  // the rest of the wave walks on without these lanes
-  const int a = qperm[t];
-  const int g = GROUPED ? agroup[a] : 0;
-  double qlo[DIM], qhi[DIM];
+k_search_tasks(SearchArgs s, int2* __restrict__ tasks, unsigned* __restrict__ ntasks, uint2* __restrict__ span) {
+  const long w = grid_wave();
+  if (w * kQueries >= s.na) return;
+  const Queries<DIM, GROUPED> Q(s, w);
+  const int top = s.info.levels - 1, lane = threadIdx.x & 63;
+  unsigned n = 0;
+  walk_union<DIM, CLOSED, GROUPED>(s, Q, top, 0, s.level, [&](long, const unsigned long long* m) {
+    n += __builtin_popcount(any_query(m));
+  });
+  unsigned at = 0;
+  if (lane == 0) {
+    if (n) at = atomicAdd(ntasks, n);
+    span[w] = make_uint2(at, n);
+  }
+  at = (unsigned)__builtin_amdgcn_readfirstlane((int)at);
+  if (at + n > s.cap) return;  // the host sees the total and calls again with room
+  walk_union<DIM, CLOSED, GROUPED>(s, Q, top, 0, s.level, [&](long first, const unsigned long long* m) {
+    const unsigned u = any_query(m);
+    if (lane < kFanout && ((u >> lane) & 1u))
+      tasks[at + __builtin_popcount(u & ((1u << lane) - 1u))] = make_int2((int)w, (int)first + lane);
+    at += __builtin_popcount(u);
+  });
+}
+
+// The search below every task's node (or the root): counts the results per
+// query, or writes them at their places in the CSR arrays.  Two walks instead
+// of one into a scratch of fixed row length: a walk is cheaper than writing
+// and reading the results once more, and rows of any length take the same
+// path.
+template <int DIM, bool CLOSED, bool GROUPED, bool FILL>
+__global__ void __launch_bounds__(kBlock) k_search(SearchArgs s) {
+  const int lane = threadIdx.x & 63, q8 = lane & 56, c = lane & 7;
+  const long total = s.tasks ? (long)*s.ntasks : (s.na + kQueries - 1) / kQueries;
+  if (s.tasks && total > (long)s.cap) return;
+  for (long t = grid_wave(); t < total; t += (long)gridDim.x * (kBlock / 64)) {
+    long w = t, node = 0;
+    int from = s.info.levels - 1;
+    if (s.tasks) {
+      const int2 task = s.tasks[t];
+      w = __builtin_amdgcn_readfirstlane(task.x);
+      node = __builtin_amdgcn_readfirstlane(task.y);
+      from = s.level;
+    }
+    const Queries<DIM, GROUPED> Q(s, w);
+    if (FILL) {
+      long at[kGroups];
 #pragma unroll
-  for (int d = 0; d < DIM; d++) {
-    qlo[d] = abox[(long)d * na + a];
-    qhi[d] = abox[(long)(DIM + d) * na + a];
-  }
-  long cnt = 0;
-  auto emit = [&](long leaf) {
-    if (cnt < cap) {
-      // 2D: streaming stores keep the hierarchy's boxes in L2 (0.96 -> 0.93 ms
-      // on tri 1024^2 vs 1000^2); in 3D they made the search slower
-      if constexpr (DIM == 2) __builtin_nontemporal_store(perm[leaf], scratch + cnt * na + t);
-      else scratch[cnt * na + t] = perm[leaf];
-    }
-    cnt++;
-  };
-  const int top = info.levels - 1;
-  if (top == 0) {
-    if (child_mask<DIM, CLOSED, GROUPED>(info, boxes, granges, 0, 0, qlo, qhi, g) & 1u) emit(0);
-  } else {
-    const bool root = child_mask<DIM, CLOSED, GROUPED>(info, boxes, granges, top, 0, qlo, qhi, g) & 1u;
-    // per lane: masks of levels 1..16, a byte each; per wave: their union
-    unsigned long long mlo = 0, mhi = 0, ulo = 0, uhi = 0;
-    auto get = [](unsigned long long lo, unsigned long long hi, int L) -> unsigned {
-      return L <= 8 ? (unsigned)(lo >> (8 * (L - 1))) & 0xffu : (unsigned)(hi >> (8 * (L - 9))) & 0xffu;
-    };
-    auto put = [](unsigned long long& lo, unsigned long long& hi, int L, unsigned m) {
-      if (L <= 8) {
-        const int sh = 8 * (L - 1);
-        lo = (lo & ~(0xffULL << sh)) | ((unsigned long long)m << sh);
-      } else {
-        const int sh = 8 * (L - 9);
-        hi = (hi & ~(0xffULL << sh)) | ((unsigned long long)m << sh);
+      for (int i = 0; i < kGroups; i++) {
+        at[i] = Q.a[i] >= 0 ? s.indptr[Q.a[i]] : 0;
+        if (s.tasks) at[i] += s.tcount[t * kQueries + 8 * i + (lane >> 3)];
       }
-    };
-    int L = top;
-    long node = 0;
-    {
-      unsigned m = child_mask<DIM, CLOSED, GROUPED>(info, boxes, granges, top - 1, 0, qlo, qhi, g);
-      if (!root) m = 0;
-      put(mlo, mhi, L, m);
-      put(ulo, uhi, L, wave_or8(m));
-    }
-    while (true) {
-      const unsigned um = get(ulo, uhi, L);
-      if (um == 0) {
-        if (L == top) break;
-        node /= kFanout;
-        L++;
-        continue;
-      }
-      if (L == 1) {  // children are elements: each lane its own hits
-        unsigned m = get(mlo, mhi, 1);
-        while (m) {
-          const int c = __builtin_ctz(m);
-          m &= m - 1;
-          emit(node * kFanout + c);
+      walk_union<DIM, CLOSED, GROUPED>(s, Q, from, node, 0, [&](long first, const unsigned long long* m) {
+        const int b = first + c < s.info.count[0] ? s.perm[first + c] : 0;
+#pragma unroll
+        for (int i = 0; i < kGroups; i++) {
+          if (m[i] == 0) continue;
+          const unsigned mine = (unsigned)(m[i] >> q8) & 0xffu;  // this lane's query's results among the children
+          if ((mine >> c) & 1u) {
+            const long o = at[i] + __builtin_popcount(mine & ((1u << c) - 1u));
+            s.indices[o] = b;
+            s.rows[o] = Q.a[i];
+          }
+          at[i] += __builtin_popcount(mine);
         }
-        put(mlo, mhi, 1, 0);
-        put(ulo, uhi, 1, 0);
-        continue;
-      }
-      const int c = __builtin_ctz(um);
-      put(ulo, uhi, L, um & (um - 1));
-      const unsigned mine = get(mlo, mhi, L);
-      put(mlo, mhi, L, mine & ~(1u << c));
-      const long child = node * kFanout + c;
-      unsigned mm = child_mask<DIM, CLOSED, GROUPED>(info, boxes, granges, L - 2, child * kFanout, qlo, qhi, g);
-      if (!((mine >> c) & 1u)) mm = 0;
-      const unsigned umm = wave_or8(mm);
-      if (umm) {
-        node = child;
-        L--;
-        put(mlo, mhi, L, mm);
-        put(ulo, uhi, L, umm);
-      }
-    }
-  }
-  row_count[a] = cnt;
-}
-
-// Rows that fit the scratch: copy them into the CSR arrays.  A wave takes 64
-// consecutive queries and transposes their slot-major scratch through LDS in
-// J-slot tiles, so that both the scratch reads and the row writes are
-// contiguous across the wave.  The tile is 16 slots tall when that holds the
-// longest row, else 32 (longer rows take several tiles): a small tile lets
-// more waves share a CU (8 and 4 per SIMD; 2 with 64 slots, which measured
-// slower on 3D rows).
-template <int J>
-__global__ void __launch_bounds__(kBlock)
-k_rows_from_scratch(long na, const int* __restrict__ qperm, int cap, const int* __restrict__ scratch,
-                    const long* __restrict__ row_count, const long* __restrict__ indptr,
-                    int* __restrict__ indices, int* __restrict__ rows) {
-  static_assert(J == 16 || J == 32, "tile height");
-  __shared__ int tile[kBlock / 64][J][65];
-  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const long base = ((long)blockIdx.x * (kBlock / 64) + wv) * 64;
-  if (base >= na) return;  // whole waves only; no block barriers below
-  const long t = base + lane;
-  int a = 0;
-  long n = 0, o = 0;
-  if (t < na) {
-    a = qperm[t];
-    n = row_count[a];
-    o = indptr[a];
-    if (n > cap) n = 0;  // left to the fill pass
-  }
-  long nmax = n;
-  for (int off = 32; off > 0; off >>= 1) {
-    const long v = __shfl_xor(nmax, off, 64);
-    nmax = v > nmax ? v : nmax;
-  }
-  int (*T)[65] = tile[wv];
-  for (long s0 = 0; s0 < nmax; s0 += J) {
-    // tile[j][q] = slot s0 + j of query base + q
-    const int nj = nmax - s0 < J ? (int)(nmax - s0) : J;
-    for (int j = 0; j < nj; j++) {
-      const long s = s0 + j;
-      T[j][lane] = (s < cap && t < na) ? scratch[s * na + t] : 0;
-    }
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-    // 64 / J queries at a time: lane l writes slot l % J of query q + l / J
-    for (int q0 = 0; q0 < 64; q0 += 64 / J) {
-      const int q = q0 + lane / J, sl = lane % J;
-      const long nq = __shfl(n, q, 64), oq = __shfl(o, q, 64);
-      const int aq = __shfl(a, q, 64);
-      const long s = s0 + sl;
-      if (s < nq) {
-        indices[oq + s] = T[sl][q];
-        rows[oq + s] = aq;
+      });
+    } else {
+      int n[kGroups];
+#pragma unroll
+      for (int i = 0; i < kGroups; i++) n[i] = 0;
+      walk_union<DIM, CLOSED, GROUPED>(s, Q, from, node, 0, [&](long, const unsigned long long* m) {
+#pragma unroll
+        for (int i = 0; i < kGroups; i++) n[i] += __builtin_amdgcn_inverse_ballot_w64(m[i]) ? 1 : 0;
+      });
+#pragma unroll
+      for (int i = 0; i < kGroups; i++) {
+#pragma unroll
+        for (int o = 1; o < 8; o <<= 1) n[i] += __shfl_xor(n[i], o, 64);
+        if (c == 0) {
+          if (s.tasks) s.tcount[t * kQueries + 8 * i + (lane >> 3)] = n[i];
+          else if (Q.a[i] >= 0) s.row_count[Q.a[i]] = n[i];
+        }
+        if (!s.tasks) raise_max(s.maxrow, n[i]);
       }
     }
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
   }
 }
 
-// Insertion sort of each row by B id (rows are short: tens of entries).
-__global__ void __launch_bounds__(kBlock)
-k_sort_rows(long na, const int* __restrict__ qperm, const long* __restrict__ indptr,
-            int* __restrict__ indices) {
-  long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= na) return;
-  int a = qperm[t];
-  long b0 = indptr[a], b1 = indptr[a + 1];
-  for (long i = b0 + 1; i < b1; i++) {
-    int v = indices[i];
-    long j = i - 1;
-    while (j >= b0 && indices[j] > v) {
-      indices[j + 1] = indices[j];
-      j--;
+// Row lengths from the tasks' counts, which become each task's offset in its
+// queries' rows.  A lane per query.
+__global__ void __launch_bounds__(kBlock) k_task_rows(SearchArgs s, const uint2* __restrict__ span) {
+  const long t = (long)blockIdx.x * kBlock + threadIdx.x;
+  if (*s.ntasks > s.cap) return;
+  long run = 0;
+  if (t < s.na) {
+    const uint2 sp = span[t / kQueries];
+    for (unsigned k = 0; k < sp.y; k++) {
+      int* c = s.tcount + ((long)sp.x + k) * kQueries + t % kQueries;
+      const int n = *c;
+      *c = (int)run;
+      run += n;
     }
-    indices[j + 1] = v;
+    s.row_count[s.qperm[t]] = run;
   }
+  raise_max(s.maxrow, (int)run);
+}
+
+// Sorts each row of at most 256 entries by B id, a wave per row: an entry's
+// place is the number of smaller ones (ids are distinct), counted against
+// every entry in turn.
+__global__ void __launch_bounds__(kBlock)
+k_sort_rows(long na, const long* __restrict__ indptr, int* __restrict__ indices) {
+  const int lane = threadIdx.x & 63;
+  for (long a = grid_wave(); a < na; a += (long)gridDim.x * (kBlock / 64)) {
+    const long o = indptr[a];
+    const int n = (int)(indptr[a + 1] - o);
+    if (n < 2) continue;
+    int v[4], place[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int k = 0; k < 4; k++) v[k] = 64 * k + lane < n ? indices[o + 64 * k + lane] : 0x7fffffff;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      if (64 * k >= n) break;
+      const int m = n - 64 * k < 64 ? n - 64 * k : 64;
+      for (int j = 0; j < m; j++) {
+        const int x = __builtin_amdgcn_readlane(v[k], j);
+#pragma unroll
+        for (int i = 0; i < 4; i++) place[i] += x < v[i] ? 1 : 0;
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+      if (64 * k + lane < n) indices[o + place[k]] = v[k];
+  }
+}
+
+// The words that the host waits for, in its own memory: [0] the pairs, [1]
+// the longest row, [2] the tasks.
+__global__ void k_publish(const long* __restrict__ npairs, const long* __restrict__ maxrow,
+                          const unsigned* __restrict__ ntasks, long* __restrict__ host) {
+  if (threadIdx.x == 0 && blockIdx.x == 0) {
+    host[0] = *npairs;
+    host[1] = *maxrow;
+    host[2] = ntasks ? (long)*ntasks : 0L;
+  }
+}
+
+// Level of the hierarchy at which walks are cut into tasks, levels - 1 for
+// none.  A wave walks its part of the tree by itself, a few microseconds per
+// node on an idle card, so a search with few query waves is cut until the
+// card is full of tasks: nodes of 8^level elements.  In a batch, where a mesh
+// of a few elements may face one of tens of thousands, always to 512 elements.
+static int task_level(const LevelInfo& info, long waves, bool grouped) {
+  const int top = info.levels - 1;
+  int level = waves >= 8192 ? top : (waves >= 2048 ? 3 : (waves >= 256 ? 2 : 1));
+  if (grouped && level > 3) level = 3;
+  return level < top ? level : top;
 }
 
 long find_pairs(Context& C, const DevMesh& A, const DevMesh& B, int finder, int sort_rows) {
@@ -783,101 +893,102 @@ long find_pairs(Context& C, const DevMesh& A, const DevMesh& B, int finder, int 
   }
   LSM_REQUIRE(A.dim == B.dim, LIBSUPERMESH_GPU_ERROR_INVALID, "Invalid dimension: meshes differ");
   const DevBVH& H = C.bvh;
-  LevelInfo info;
-  info.levels = H.levels;
-  for (int l = 0; l < 32; l++) {
-    info.count[l] = l < H.levels ? H.count[l] : 0;
-    info.offset[l] = l < H.levels ? H.offset[l] : 0;
-  }
   morton_order(C, A, C.qperm);
-  const int* qperm = static_cast<const int*>(C.qperm.ptr);
-  const double* abox = static_cast<const double*>(A.bbox.ptr);
-  const double* boxes = static_cast<const double*>(H.boxes.ptr);
-  const int* perm = static_cast<const int*>(H.perm.ptr);
-  dim3 grid(grid_for(na, kBlock)), block(kBlock);
   LSM_REQUIRE((A.ngroups > 0) == H.grouped && (!H.grouped || A.ngroups == B.ngroups),
               LIBSUPERMESH_GPU_ERROR_INVALID, "batches of A and B hold different mesh counts");
-  const int* agroup = H.grouped ? static_cast<const int*>(A.group.ptr) : nullptr;
-  const int* granges = H.grouped ? static_cast<const int*>(H.granges.ptr) : nullptr;
-#define LSM_QUERY(DIM, CL, FILL, SKIP)                                                              \
-  do {                                                                                            \
-    if (H.grouped)                                                                                \
-      hipLaunchKernelGGL((k_query<DIM, CL, FILL, true>), grid, block, 0, C.stream, na, qperm, abox, \
-                         info, boxes, perm, row_count, indptr, indices, rows, agroup, granges,    \
-                         (long)(SKIP));                                                           \
-    else                                                                                          \
-      hipLaunchKernelGGL((k_query<DIM, CL, FILL, false>), grid, block, 0, C.stream, na, qperm,      \
-                         abox, info, boxes, perm, row_count, indptr, indices, rows, agroup,        \
-                         granges, (long)(SKIP));                                                  \
-  } while (0)
-#define LSM_MASK(DIM, CL)                                                                           \
-  do {                                                                                            \
-    if (H.grouped)                                                                                \
-      hipLaunchKernelGGL((k_query_wave<DIM, CL, true>), grid, block, 0, C.stream, na, qperm, abox,  \
-                         info, boxes, perm, cap, scratch, row_count, agroup, granges);            \
-    else                                                                                          \
-      hipLaunchKernelGGL((k_query_wave<DIM, CL, false>), grid, block, 0, C.stream, na, qperm, abox, \
-                         info, boxes, perm, cap, scratch, row_count, agroup, granges);            \
-  } while (0)
-  int* indices = nullptr;
-  int* rows = nullptr;
-  bool closed = finder == LIBSUPERMESH_GPU_FINDER_RTREE;
-  // single pass into a scratch of `cap` results per query; longer rows are
-  // searched again by the fill pass
-  const int cap = A.dim == 2 ? 32 : 160;
   LSM_REQUIRE(H.levels <= 17, LIBSUPERMESH_GPU_ERROR_OVERFLOW, "hierarchy too deep");
-  int* scratch = C.fscratch.as<int>((size_t)cap * na);
-  if (A.dim == 2) {
-    if (closed) LSM_MASK(2, true);
-    else LSM_MASK(2, false);
-  } else {
-    if (closed) LSM_MASK(3, true);
-    else LSM_MASK(3, false);
+  const bool closed = finder == LIBSUPERMESH_GPU_FINDER_RTREE;
+  const long waves = (na + kQueries - 1) / kQueries;
+  SearchArgs s = {};
+  s.na = na;
+  s.qperm = static_cast<const int*>(C.qperm.ptr);
+  s.abox = static_cast<const double*>(A.bbox.ptr);
+  s.agroup = H.grouped ? static_cast<const int*>(A.group.ptr) : nullptr;
+  s.granges = H.grouped ? static_cast<const int*>(H.granges.ptr) : nullptr;
+  s.boxes = static_cast<const double*>(H.boxes.ptr);
+  s.perm = static_cast<const int*>(H.perm.ptr);
+  s.info.levels = H.levels;
+  for (int l = 0; l < 32; l++) {
+    s.info.count[l] = l < H.levels ? H.count[l] : 0;
+    s.info.offset[l] = l < H.levels ? H.offset[l] : 0;
   }
-  LSM_HIP(hipGetLastError());
-  size_t tmp_bytes = 0;
-  LSM_HIP(rocprim::inclusive_scan(nullptr, tmp_bytes, row_count, indptr + 1, (size_t)na,
-                                  rocprim::plus<long>(), C.stream));
-  void* tmp = C.scan_tmp.get(tmp_bytes);
-  LSM_HIP(rocprim::inclusive_scan(tmp, tmp_bytes, row_count, indptr + 1, (size_t)na,
-                                  rocprim::plus<long>(), C.stream));
-  // longest row: decides whether the fill pass is needed
-  long* dmax = C.scalars.as<long>(64) + 16;
-  {
-    size_t bytes = 0;
-    LSM_HIP(rocprim::reduce(nullptr, bytes, row_count, dmax, 0L, (size_t)na, rocprim::maximum<long>(), C.stream));
-    void* t2 = C.sort_tmp.get(bytes);
-    LSM_HIP(rocprim::reduce(t2, bytes, row_count, dmax, 0L, (size_t)na, rocprim::maximum<long>(), C.stream));
-  }
-  long hdr[2] = {0, 0};
-  LSM_HIP(hipMemcpyAsync(&hdr[0], indptr + na, sizeof(long), hipMemcpyDeviceToHost, C.stream));
-  LSM_HIP(hipMemcpyAsync(&hdr[1], dmax, sizeof(long), hipMemcpyDeviceToHost, C.stream));
-  LSM_HIP(hipStreamSynchronize(C.stream));
-  const long npairs = hdr[0], maxrow = hdr[1];
-  LSM_REQUIRE(npairs < (1L << 40), LIBSUPERMESH_GPU_ERROR_OVERFLOW, "too many candidate pairs");
-  indices = C.indices.as<int>(npairs);
-  rows = C.rows.as<int>(npairs);
-  if (npairs > 0) {
-    const long tall = maxrow < cap ? maxrow : cap;  // the most slots a copied row holds
-    if (tall <= 16)
-      hipLaunchKernelGGL(k_rows_from_scratch<16>, grid, block, 0, C.stream, na, qperm, cap, scratch, row_count,
-                         indptr, indices, rows);
-    else
-      hipLaunchKernelGGL(k_rows_from_scratch<32>, grid, block, 0, C.stream, na, qperm, cap, scratch, row_count,
-                         indptr, indices, rows);
-    if (maxrow > cap) {
-      if (A.dim == 2) {
-        if (closed) LSM_QUERY(2, true, true, cap);
-        else LSM_QUERY(2, false, true, cap);
-      } else {
-        if (closed) LSM_QUERY(3, true, true, cap);
-        else LSM_QUERY(3, false, true, cap);
-      }
+  s.row_count = row_count;
+  s.indptr = indptr;
+  s.level = task_level(s.info, waves, H.grouped);
+  const bool split = s.level < H.levels - 1;
+  const dim3 block(kBlock), wave_grid(grid_for(waves, kBlock / 64));
+#define LSM_SEARCH(K, ...)                                                                    \
+  do {                                                                                        \
+    if (A.dim == 2) {                                                                         \
+      if (closed) {                                                                           \
+        if (H.grouped) hipLaunchKernelGGL((K(2, true, true)), grid, block, 0, C.stream, __VA_ARGS__);   \
+        else hipLaunchKernelGGL((K(2, true, false)), grid, block, 0, C.stream, __VA_ARGS__);  \
+      } else {                                                                                \
+        if (H.grouped) hipLaunchKernelGGL((K(2, false, true)), grid, block, 0, C.stream, __VA_ARGS__);  \
+        else hipLaunchKernelGGL((K(2, false, false)), grid, block, 0, C.stream, __VA_ARGS__); \
+      }                                                                                       \
+    } else {                                                                                  \
+      if (closed) {                                                                           \
+        if (H.grouped) hipLaunchKernelGGL((K(3, true, true)), grid, block, 0, C.stream, __VA_ARGS__);   \
+        else hipLaunchKernelGGL((K(3, true, false)), grid, block, 0, C.stream, __VA_ARGS__);  \
+      } else {                                                                                \
+        if (H.grouped) hipLaunchKernelGGL((K(3, false, true)), grid, block, 0, C.stream, __VA_ARGS__);  \
+        else hipLaunchKernelGGL((K(3, false, false)), grid, block, 0, C.stream, __VA_ARGS__); \
+      }                                                                                       \
+    }                                                                                         \
+    LSM_HIP(hipGetLastError());                                                               \
+  } while (0)
+#define LSM_TASKS(D, CL, G) k_search_tasks<D, CL, G>
+#define LSM_COUNT(D, CL, G) k_search<D, CL, G, false>
+#define LSM_FILL(D, CL, G) k_search<D, CL, G, true>
+  long* words = C.scalars.as<long>(64) + 16;  // [0] longest row, [1] tasks
+  s.maxrow = words;
+  volatile long* host = C.hstat + 8;
+  dim3 grid = wave_grid;
+  long room = 16 * waves + 16384;
+  while (true) {
+    hipLaunchKernelGGL(k_clear_words, dim3(1), dim3(64), 0, C.stream, 2, words);
+    if (split) {
+      s.cap = (unsigned)room;
+      int2* tasks = C.ftasks.as<int2>(room);
+      uint2* span = C.fspan.as<uint2>(waves);
+      s.tcount = C.fcount.as<int>((size_t)room * kQueries);
+      unsigned* ntasks = reinterpret_cast<unsigned*>(words + 1);
+      s.tasks = nullptr;
+      grid = wave_grid;
+      LSM_SEARCH(LSM_TASKS, s, tasks, ntasks, span);
+      s.tasks = tasks;
+      s.ntasks = ntasks;
+      grid = dim3(std::min<unsigned>(grid_for(room, kBlock / 64), 8192));
+      LSM_SEARCH(LSM_COUNT, s);
+      hipLaunchKernelGGL(k_task_rows, dim3(grid_for(na, kBlock)), block, 0, C.stream, s, span);
+    } else {
+      LSM_SEARCH(LSM_COUNT, s);
     }
+    size_t tmp_bytes = 0;
+    LSM_HIP(rocprim::inclusive_scan(nullptr, tmp_bytes, row_count, indptr + 1, (size_t)na,
+                                    rocprim::plus<long>(), C.stream));
+    void* tmp = C.scan_tmp.get(tmp_bytes);
+    LSM_HIP(rocprim::inclusive_scan(tmp, tmp_bytes, row_count, indptr + 1, (size_t)na,
+                                    rocprim::plus<long>(), C.stream));
+    hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, C.stream, indptr + na, s.maxrow, split ? s.ntasks : nullptr,
+                       C.hstat + 8);
     LSM_HIP(hipGetLastError());
+    LSM_HIP(hipStreamSynchronize(C.stream));
+    if (!split || host[2] <= room) break;
+    LSM_REQUIRE(host[2] < (1L << 31), LIBSUPERMESH_GPU_ERROR_OVERFLOW, "too many search tasks");
+    room = host[2] + host[2] / 8;
+  }
+  const long npairs = host[0], maxrow = host[1];
+  LSM_REQUIRE(npairs < (1L << 40), LIBSUPERMESH_GPU_ERROR_OVERFLOW, "too many candidate pairs");
+  s.indices = C.indices.as<int>(npairs);
+  s.rows = C.rows.as<int>(npairs);
+  if (npairs > 0) {
+    LSM_SEARCH(LSM_FILL, s);
     if (sort_rows) {
-      if (maxrow <= 64) {
-        hipLaunchKernelGGL(k_sort_rows, grid, block, 0, C.stream, na, qperm, indptr, indices);
+      if (maxrow <= 256) {
+        hipLaunchKernelGGL(k_sort_rows, dim3(std::min<unsigned>(grid_for(na, kBlock / 64), 65536)), block, 0, C.stream,
+                           na, indptr, s.indices);
       } else {
         // long rows (a coarse A element over a fine B mesh): segmented radix
         // sort of the rows, then the sorted copy becomes the indices buffer
@@ -887,18 +998,20 @@ long find_pairs(Context& C, const DevMesh& A, const DevMesh& B, int finder, int 
         unsigned end_bit = 1;
         while (end_bit < 31 && (1L << end_bit) < B.nelements) end_bit++;
         size_t bytes = 0;
-        LSM_HIP(rocprim::segmented_radix_sort_keys(nullptr, bytes, indices, sorted, (unsigned)npairs, (unsigned)na,
+        LSM_HIP(rocprim::segmented_radix_sort_keys(nullptr, bytes, s.indices, sorted, (unsigned)npairs, (unsigned)na,
                                                    indptr, indptr + 1, 0u, end_bit, C.stream));
         void* t3 = C.sort_tmp.get(bytes);
-        LSM_HIP(rocprim::segmented_radix_sort_keys(t3, bytes, indices, sorted, (unsigned)npairs, (unsigned)na,
+        LSM_HIP(rocprim::segmented_radix_sort_keys(t3, bytes, s.indices, sorted, (unsigned)npairs, (unsigned)na,
                                                    indptr, indptr + 1, 0u, end_bit, C.stream));
         std::swap(C.indices, C.vals_alt);
       }
       LSM_HIP(hipGetLastError());
     }
   }
-#undef LSM_MASK
-#undef LSM_QUERY
+#undef LSM_SEARCH
+#undef LSM_TASKS
+#undef LSM_COUNT
+#undef LSM_FILL
   return npairs;
 }
 

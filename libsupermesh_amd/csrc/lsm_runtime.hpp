@@ -135,7 +135,7 @@ struct Context {
   DevBuf keys, keys_alt, vals, vals_alt, sort_tmp, scan_tmp;
   DevBuf qperm;                  // A elements in Morton order
   DevBuf row_count, indptr, indices, rows;
-  DevBuf fscratch;               // single-pass search results (slot-major)
+  DevBuf ftasks, fspan, fcount;  // search tasks, each query wave's, and their per-query counts
   // clipping
   DevBuf counts, measure, partials, scalars, offsets, elements, blocks;
   DevBuf offsets_dense, elements_dense;  // LIBSUPERMESH_GPU_DENSE: the single pass's runs compacted
@@ -150,7 +150,8 @@ struct Context {
   // batches: per-mesh pair offsets and measure sums
   DevBuf gpairs, gsum;
   // pinned status words the pipeline copies back asynchronously and reads
-  // after its next synchronisation: [0] staging flag, [1] longest mass row
+  // after its next synchronisation: [0] staging flag, [1] longest mass row,
+  // [8..10] the search's pairs, longest row and tasks
   long* hstat = nullptr;
   Predictor predictor;
   // 2D mixed mass: rows laid out before the clip and filled by it
