@@ -76,7 +76,7 @@ static void free_context(Context& C) {
                     &C.mkeys, &C.mvals, &C.mkeys_alt, &C.mvals_alt, &C.ukeys, &C.uvals, &C.nuniq,
                     &C.mindptr, &C.mindices, &C.mrbase, &C.mesh_a.scale,
                     &C.mesh_b.scale, &C.mesh_a.group, &C.mesh_b.group, &C.bvh.granges, &C.gpairs,
-                    &C.gsum, &C.predictor.weights, &C.predictor.bias, &C.predictor.master,
+                    &C.gsum, &C.gparts, &C.predictor.weights, &C.predictor.bias, &C.predictor.master,
                     &C.predictor.adam_m, &C.predictor.adam_v, &C.predictor.grad,
                     &C.predictor.features, &C.predictor.labels, &C.predictor.act,
                     &C.predictor.loss, &C.predictor.index, &C.predictor.budget,

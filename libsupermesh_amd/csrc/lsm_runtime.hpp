@@ -148,7 +148,7 @@ struct Context {
   // 2D row slots: each (element, vertex) row's first slot
   DevBuf mrbase;
   // batches: per-mesh pair offsets and measure sums
-  DevBuf gpairs, gsum;
+  DevBuf gpairs, gsum, gparts;
   // pinned status words the pipeline copies back asynchronously and reads
   // after its next synchronisation: [0] staging flag, [1] longest mass row,
   // [8..10] the search's pairs, longest row and tasks

@@ -1532,13 +1532,17 @@ k_batch_pairs(long ngroups, const long* __restrict__ a_off, const long* __restri
   if (g <= ngroups) gpairs[g] = indptr[a_off[g]];
 }
 
-// ... and its measure sum: one block per mesh, double-double in a fixed order.
+// ... and its measure sum, double-double in a fixed order: kSumParts blocks a
+// mesh, then one wave adds their parts.  (One block a mesh was a chain of
+// thousands of dependent loads and adds on the largest mesh: 2.0 ms of a batch
+// of ~100 mesh pairs of up to 50 000 tets.)
+constexpr int kSumParts = 64;
 __global__ void __launch_bounds__(kClipBlock)
-k_batch_sum(const long* __restrict__ gpairs, const double* __restrict__ measure,
-            double* __restrict__ gsum) {
-  const long g = blockIdx.x;
+k_batch_sum(const long* __restrict__ gpairs, const double* __restrict__ measure, double2* __restrict__ parts) {
+  const long g = blockIdx.y, first = gpairs[g], n = gpairs[g + 1] - first;
   double hi = 0.0, lo = 0.0;
-  for (long p = gpairs[g] + threadIdx.x; p < gpairs[g + 1]; p += kClipBlock) dd_add(hi, lo, measure[p]);
+  for (long p = (long)blockIdx.x * kClipBlock + threadIdx.x; p < n; p += kSumParts * kClipBlock)
+    dd_add(hi, lo, measure[first + p]);
   __shared__ double rh[kClipBlock], rl[kClipBlock];
   rh[threadIdx.x] = hi;
   rl[threadIdx.x] = lo;
@@ -1552,7 +1556,20 @@ k_batch_sum(const long* __restrict__ gpairs, const double* __restrict__ measure,
     }
     __syncthreads();
   }
-  if (threadIdx.x == 0) gsum[g] = rh[0] + rl[0];
+  if (threadIdx.x == 0) parts[g * kSumParts + blockIdx.x] = make_double2(rh[0], rl[0]);
+}
+
+__global__ void __launch_bounds__(64)
+k_batch_total(const double2* __restrict__ parts, double* __restrict__ gsum) {
+  static_assert(kSumParts == 64, "a lane per part");
+  const double2 x = parts[(long)blockIdx.x * kSumParts + threadIdx.x];
+  double hi = x.x, lo = x.y;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const double h2 = __shfl_down(hi, o, 64), l2 = __shfl_down(lo, o, 64);
+    dd_merge(hi, lo, h2, l2);
+  }
+  if (threadIdx.x == 0) gsum[blockIdx.x] = hi + lo;
 }
 
 // Order-sensitive 64-bit checksum of a device buffer: sum over its 32-bit
@@ -1603,9 +1620,12 @@ void batch_sums(Context& C, long ngroups, const long* a_offsets, const long* ind
   double* gs = C.gsum.as<double>((size_t)ngroups);
   hipLaunchKernelGGL(k_batch_pairs, dim3(grid_for(ngroups + 1, kClipBlock)), dim3(kClipBlock), 0,
                      C.stream, ngroups, a_offsets, indptr, gp);
-  if (ngroups > 0)
-    hipLaunchKernelGGL(k_batch_sum, dim3((unsigned)ngroups), dim3(kClipBlock), 0, C.stream, gp,
-                       measure, gs);
+  // the grid's second dimension holds 65535 meshes
+  double2* parts = C.gparts.as<double2>((size_t)ngroups * kSumParts);
+  for (long g0 = 0; g0 < ngroups; g0 += 65535)
+    hipLaunchKernelGGL(k_batch_sum, dim3(kSumParts, (unsigned)std::min<long>(65535, ngroups - g0)), dim3(kClipBlock), 0,
+                       C.stream, gp + g0, measure, parts + g0 * kSumParts);
+  if (ngroups > 0) hipLaunchKernelGGL(k_batch_total, dim3((unsigned)ngroups), dim3(64), 0, C.stream, parts, gs);
   LSM_HIP(hipGetLastError());
 }
 
@@ -2519,6 +2539,7 @@ void count_pass_graph(Context& C, const DevMesh& A, const DevMesh& B, long npair
   if (ngroups > 0) {
     C.gpairs.as<long>((size_t)ngroups + 1);
     C.gsum.as<double>((size_t)ngroups);
+    C.gparts.as<double2>((size_t)ngroups * kSumParts);
   }
   if (dim == 2) {
     g.olist = static_cast<int*>(C.work.ptr);
@@ -2534,7 +2555,7 @@ void count_pass_graph(Context& C, const DevMesh& A, const DevMesh& B, long npair
       reinterpret_cast<const void*>(ngroups), reinterpret_cast<const void*>((long)s.block),
       reinterpret_cast<const void*>((long)s.grid), g.npairs_dev, g.rows, g.cols, g.acoords, g.bcoords, g.asp,
       g.bsp, g.ascale, g.bscale, g.bplanes, g.counts, g.measure, parts, C.mflag.ptr, C.work.ptr, C.nwork.ptr,
-      C.queue.ptr, scal, a_off, out->indptr, C.gpairs.ptr, C.gsum.ptr};
+      C.queue.ptr, scal, a_off, out->indptr, C.gpairs.ptr, C.gsum.ptr, C.gparts.ptr};
   const int d = dim - 2;
   if (C.graph_exec[d] && key != C.graph_key[d]) release_graph(C, d);
   if (!C.graph_exec[d] && !C.graph_refused &&

@@ -395,7 +395,7 @@ struct QuadClip {
     const uint32_t kinds = quad_or((mine && whole ? 1u : 0u) << q | (mine && cuts ? 16u : 0u) << q);
     const uint32_t more = kinds >> 4;
     const uint32_t lead = kinds & 15u & ((more & -more) - 1u);  // the outputs before any other child
-    if ((kinds & 15u & ~lead | more) != 0) {
+    if (((kinds & 15u & ~lead) | more) != 0) {
       const bool keep = mine && !((lead >> q) & 1u) && (whole || cuts);
       if (keep) {
         const int at = (3 * r - 1 - q) * kWords * 16;  // row r's entries 3 r - 3 .. 3 r - 1, child 0 last
