@@ -2898,11 +2898,10 @@ k_segment_sum(long n, const uint64_t* __restrict__ keys, const double* __restric
 // Row-wise mixed mass assembly.  Row i of M (A node i) collects, from every A
 // element e containing i (local vertex li) and every non-empty pair p of e,
 // the entries (B node of local vertex j, blocks[p][li][j]).  One wave owns a
-// row: it gathers the row's entries into LDS in a fixed order (elements of i
-// in ascending (e, li), pairs of e in CSR order, j ascending), finds the
-// distinct B nodes with an LDS hash table, sorts them, and each lane sums
-// its columns' entries in gather order -- no global sort, and the same result
-// on every run.  Rows too long for LDS take the global sort path.
+// row: it takes the row's entries in a fixed order (elements of i in ascending
+// (e, li), pairs of e in CSR order, j ascending), finds the distinct B nodes
+// with an LDS hash table and sorts them -- no global sort, and the same result
+// on every run.  Rows with too many columns take the global sort path.
 // ---------------------------------------------------------------------------
 
 
@@ -2953,18 +2952,10 @@ k_row_bounds(long nn, const long* __restrict__ nptr, const long* __restrict__ sl
   if (i < nn) raw[i] = slot[nptr[i + 1]] - slot[nptr[i]];
 }
 
-__global__ void __launch_bounds__(256)
-k_elem_nonempty(long ne, const long* __restrict__ indptr, const int* __restrict__ counts,
-                int* __restrict__ out) {
-  long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= ne) return;
-  int c = 0;
-  for (long p = indptr[e]; p < indptr[e + 1]; p++) c += counts[p] > 0;
-  out[e] = c;
-}
-
-// Moves each row's reduced (column, value) list from its slot range to the
-// CSR: 16 lanes per row (rows hold a few dozen columns).
+// Moves each row's reduced (column, value) list from its slot range (at
+// raw_off[i], or kMaxDistinct apart) to the CSR: 16 lanes per row (rows hold a
+// few dozen columns).
+constexpr int kMaxDistinct = 256;  // columns a row may hold on the row kernels
 constexpr int kCopyLanes = 16;
 __global__ void __launch_bounds__(256)
 k_mass_copy(long nn, const long* __restrict__ raw_off, const long* __restrict__ mptr,
@@ -2972,7 +2963,7 @@ k_mass_copy(long nn, const long* __restrict__ raw_off, const long* __restrict__ 
             double* __restrict__ mval) {
   const long i = ((long)blockIdx.x * blockDim.x + threadIdx.x) / kCopyLanes;
   if (i >= nn) return;
-  const long o = mptr[i], n = mptr[i + 1] - o, r = raw_off[i];
+  const long o = mptr[i], n = mptr[i + 1] - o, r = raw_off ? raw_off[i] : i * kMaxDistinct;
   for (long t = threadIdx.x % kCopyLanes; t < n; t += kCopyLanes) {
     mind[o + t] = tkey[r + t];
     mval[o + t] = tval[r + t];
@@ -3043,6 +3034,11 @@ static void assemble_mass_sorted(Context& C, const DevMesh& A, const DevMesh& B,
   out->mass_values = mval;
 }
 
+// Adds to a sum in LDS (ds_add_f64).
+__device__ __forceinline__ void lds_add(double* p, double v) {
+  (void)__builtin_amdgcn_ds_atomic_fadd_f64((__attribute__((address_space(3))) double*)p, v);
+}
+
 // Bitonic sort of up to 64*EPL int keys in registers (element t = lane + 64*r),
 // keys only.
 template <int EPL>
@@ -3080,16 +3076,7 @@ __device__ __forceinline__ void wave_bitonic_keys(int* key, int lane) {
 }
 
 constexpr int kHashSlots = 512;   // per-row table of distinct B nodes
-constexpr int kMaxDistinct = 256;  // columns a row may hold on this path
 
-// One wave per row of the mixed mass: gathers the row's contributions (its
-// incident A elements in node-list order, their non-empty pairs in CSR order,
-// B's local nodes in order) into LDS, finds the distinct columns with an LDS
-// hash table, sorts them, and sums each column's contributions in gather
-// order -- a fixed order, so the result is reproducible.  Writes the row's
-// (column, value) list at raw_off[i] and its length to ucount[i]; rows whose
-// distinct columns exceed kMaxDistinct raise *overflow (the caller then uses
-// the global sort path).
 // Deduplicates and sums one row held in LDS (rk/rv, n entries): distinct
 // columns through an LDS hash table, sorted, each summed in entry order.
 // Writes them at tkey/tval + o; returns the count, or -1 if the row has more
@@ -3196,13 +3183,12 @@ __device__ __forceinline__ int row_reduce(const int* rk, const double* rv, int n
   return nd;
 }
 
-template <int LOC, int CAP, int WAVES, bool SLOTS = false>
+// Long rows laid out by the clip pass (2D, up to CAP slots; empty pairs as
+// node -1), read as they are.
+template <int CAP, int WAVES>
 __global__ void __launch_bounds__(64 * WAVES)
-k_mass_rows_gather(long nn, const long* __restrict__ nptr, const int* __restrict__ nlist,
-                   const long* __restrict__ indptr, const int* __restrict__ cols,
-                   const int* __restrict__ counts, const double* __restrict__ blocks,
-                   const int* __restrict__ enlb, const long* __restrict__ raw_off, int* __restrict__ tkey,
-                   double* __restrict__ tval, long* __restrict__ ucount, int* __restrict__ overflow) {
+k_mass_rows_long(long nn, const long* __restrict__ raw_off, int* __restrict__ tkey, double* __restrict__ tval,
+                 long* __restrict__ ucount, int* __restrict__ overflow) {
   __shared__ __align__(16) int s_rk[WAVES][CAP + 8];
   __shared__ __align__(16) double s_rv[WAVES][CAP + 8];
   __shared__ int s_ht[WAVES][kHashSlots];
@@ -3215,12 +3201,8 @@ k_mass_rows_gather(long nn, const long* __restrict__ nptr, const int* __restrict
   for (long base = (long)blockIdx.x * WAVES; base < nn; base += nwaves) {
     const long i = base + wv;
     const bool valid = i < nn;
-    // 1. gather: up to 64 incident elements at a time, one per lane; their
-    // pair ranges are laid end to end and the lanes walk that flat list.  With
-    // SLOTS the clip pass already wrote the row in that order (empty pairs as
-    // node -1): it is read as is.
     int n = 0;
-    if (SLOTS && valid) {
+    if (valid) {
       const long r0 = raw_off[i], r1 = raw_off[i + 1];
       for (long rb = r0; rb < r1; rb += 64) {
         const long r = rb + lane;
@@ -3235,55 +3217,9 @@ k_mass_rows_gather(long nn, const long* __restrict__ nptr, const int* __restrict
         n += __popcll(m);
       }
     }
-    if (!SLOTS && valid) {
-      const long x0 = nptr[i], x1 = nptr[i + 1];
-      for (long xb = x0; xb < x1; xb += 64) {
-        const long x = xb + lane;
-        long p0 = 0;
-        int np = 0, li = 0;
-        if (x < x1) {
-          const int el = nlist[x];
-          const int e = el / LOC;
-          li = el - e * LOC;
-          p0 = indptr[e];
-          np = (int)(indptr[e + 1] - p0);
-        }
-        int incl = np;
-        for (int o = 1; o < 64; o <<= 1) {
-          const int v = __shfl_up(incl, o, 64);
-          if (lane >= o) incl += v;
-        }
-        const int excl = incl - np;
-        const int total = __shfl(incl, 63, 64);
-        for (int f0 = 0; f0 < total; f0 += 64) {
-          const int f = f0 + lane;
-          // owner: the last lane whose range starts at or before f
-          int own = 0;
-          for (int step = 32; step > 0; step >>= 1) {
-            const int cand = own + step;
-            const int ev = __shfl(excl, cand < 64 ? cand : 63, 64);
-            if (cand < 64 && ev <= f) own = cand;
-          }
-          const long p = __shfl(p0, own, 64) + (f - __shfl(excl, own, 64));
-          const int lio = __shfl(li, own, 64);
-          const bool ne = f < total && counts[p] > 0;
-          const unsigned long long m = __ballot(ne);
-          if (ne) {
-            const int pos = n + LOC * __popcll(m & ((1ULL << lane) - 1));
-            const long b = cols[p];
-#pragma unroll
-            for (int j = 0; j < LOC; j++) {
-              rk[pos + j] = enlb[b * LOC + j];
-              rv[pos + j] = blocks[p * LOC * LOC + lio * LOC + j];
-            }
-          }
-          n += LOC * __popcll(m);
-        }
-      }
-    }
     if (lane < 8) rk[n + lane] = -2;  // tail of the last 8-entry group
     __syncthreads();
-    // 2-4. distinct columns, sorted, summed in gather order (every wave of the
+    // distinct columns, sorted, summed in entry order (every wave of the
     // block calls this, valid row or not, so that the barriers match)
     const int nd = row_reduce(rk, rv, valid ? n : 0, ht, lane, tkey, tval, valid ? raw_off[i] : 0);
     if (valid && lane == 0) {
@@ -3292,6 +3228,162 @@ k_mass_rows_gather(long nn, const long* __restrict__ nptr, const int* __restrict
     }
     __syncthreads();  // the LDS rows are refilled next
   }
+}
+
+// 3D rows, one wave each, from the per-pair blocks: the wave takes the node's
+// elements in ascending order, an element's candidate pairs 64 at a time, and
+// its non-empty pairs sixteen at a time, four lanes a pair (a B node each).
+// Every entry goes straight into an LDS hash table, where it is added to its
+// column's sum, so a row may hold any number of entries; at the end the
+// columns are sorted and written.  One wave adds to a table, its instructions
+// in order and the lanes of each in theirs, so the sums are the same on every
+// run.  (Rows of up to 2048 entries used to be gathered into LDS and longer
+// ones, which any two like tet meshes have, sorted globally: 6.9 ms of sort
+// and segment sums at 32^3 vs 30^3 against 0.3 ms here.)
+__global__ void __launch_bounds__(256)
+k_mass_rows_tet(long nn, const long* __restrict__ nptr, int* __restrict__ nlist, const long* __restrict__ indptr,
+                const int* __restrict__ cols, const int* __restrict__ counts, const double* __restrict__ blocks,
+                const int* __restrict__ enlb, int* __restrict__ tkey, double* __restrict__ tval,
+                long* __restrict__ ucount, int* __restrict__ overflow) {
+  __shared__ int s_key[4][kHashSlots];
+  __shared__ double s_sum[4][kHashSlots];
+  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 3;
+  int* hk = s_key[wv];
+  double* hv = s_sum[wv];
+  const long i = (long)blockIdx.x * 4 + wv;
+  if (i >= nn) return;  // whole waves; no block barriers below
+  for (int t = lane; t < kHashSlots; t += 64) {
+    hk[t] = -1;
+    hv[t] = 0.0;
+  }
+  const long x0 = nptr[i], x1 = nptr[i + 1];
+  if (x1 - x0 > 64 && lane == 0) {  // the atomics that filled the list left it in any order
+    for (long x = x0 + 1; x < x1; x++) {
+      const int v = nlist[x];
+      long y = x - 1;
+      while (y >= x0 && nlist[y] > v) {
+        nlist[y + 1] = nlist[y];
+        y--;
+      }
+      nlist[y + 1] = v;
+    }
+    __threadfence();
+  }
+  quad_fence();
+  bool full = false;
+  for (long xb = x0; xb < x1 && !full; xb += 64) {
+    const int nel = x1 - xb < 64 ? (int)(x1 - xb) : 64;
+    int el = lane < nel ? nlist[xb + lane] : 0x7fffffff;
+    if (x1 - x0 <= 64) {  // in ascending order: to the lane of its rank
+      int rank = 0;
+      for (int k = 0; k < nel; k++) rank += __builtin_amdgcn_readlane(el, k) < el ? 1 : 0;
+      el = __builtin_amdgcn_ds_permute((lane < nel ? rank : lane) * 4, el);
+    }
+    long p0 = 0;
+    int np = 0;
+    if (lane < nel) {
+      p0 = indptr[el >> 2];
+      np = (int)(indptr[(el >> 2) + 1] - p0);
+    }
+    // the next 64 candidates' counts and columns on their way
+    auto load = [&](long p, int n, int& c, int& b) {
+      c = lane < n ? counts[p + lane] : 0;
+      b = lane < n ? cols[p + lane] : 0;
+    };
+    int k = 0, f = 0, c = 0, b = 0;
+    long pk = 0;
+    auto seek = [&]() {  // the element at k, skipping those without candidates
+      while (k < nel && f >= __builtin_amdgcn_readlane(np, k)) {
+        k++;
+        f = 0;
+      }
+      if (k < nel) {
+        pk = (long)((unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(p0 >> 32), k) << 32 |
+                    (unsigned)__builtin_amdgcn_readlane((int)p0, k));
+        load(pk + f, __builtin_amdgcn_readlane(np, k) - f, c, b);
+      }
+    };
+    seek();
+    while (k < nel) {
+      const int cc = c, cb = b, li = __builtin_amdgcn_readlane(el, k) & 3;
+      const long cp = pk + f;
+      f += 64;
+      seek();
+      const unsigned long long m = __ballot(cc > 0);
+      const int nz = __popcll(m);
+      const int before = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
+      const int to = (cc > 0 ? before : nz + lane - before) * 4;
+      const int at = __builtin_amdgcn_ds_permute(to, lane), bb = __builtin_amdgcn_ds_permute(to, cb);
+      for (int g = 0; g < nz; g += 16) {
+        const int r = g + (lane >> 2);
+        const long p = cp + __shfl(at, r & 63, 64);
+        const long e = __shfl(bb, r & 63, 64);
+        if (r < nz) {
+          const int key = enlb[e * 4 + j];
+          const double v = blocks[p * 16 + li * 4 + j];
+          unsigned h = ((unsigned)key * 2654435761u) >> (32 - 9);
+          int tries = 0;
+          while (true) {
+            const int prev = atomicCAS(&hk[h], -1, key);
+            if (prev == -1 || prev == key) break;
+            h = (h + 1) & (kHashSlots - 1);
+            if (++tries >= kHashSlots) {
+              full = true;
+              break;
+            }
+          }
+          if (!full) lds_add(&hv[h], v);
+        }
+      }
+      full = __any(full);
+      if (full) break;
+    }
+  }
+  quad_fence();
+  // the distinct columns, four a lane, sorted
+  int nd = 0, key[4] = {0x7fffffff, 0x7fffffff, 0x7fffffff, 0x7fffffff};
+  for (int s0 = 0; s0 < kHashSlots; s0 += 64) nd += __popcll(__ballot(hk[s0 + lane] != -1));
+  if (full || nd > kMaxDistinct) {
+    if (lane == 0) {
+      atomicOr(overflow, 1);
+      ucount[i] = 0;
+    }
+    return;
+  }
+  // each lane's columns, packed across the wave through the output row
+  int* out_key = tkey + i * kMaxDistinct;
+  double* out_val = tval + i * kMaxDistinct;
+  int done = 0;
+#pragma unroll
+  for (int s0 = 0; s0 < kHashSlots; s0 += 64) {
+    const int x = hk[s0 + lane];
+    const unsigned long long m = __ballot(x != -1);
+    const int n = __popcll(m);
+    const int before = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
+    // lane l of the packed group goes to place done + l
+    const int y = __builtin_amdgcn_ds_permute((x != -1 ? before : n + lane - before) * 4, x);
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int from = 64 * r + lane - done;
+      const int z = __shfl(y, from & 63, 64);
+      if (from >= 0 && from < n) key[r] = z;
+    }
+    done += n;
+  }
+  if (nd <= 64) wave_bitonic_keys<1>(key, lane);
+  else if (nd <= 128) wave_bitonic_keys<2>(key, lane);
+  else wave_bitonic_keys<4>(key, lane);
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    const int t = lane + 64 * r;
+    if (t < nd) {
+      unsigned h = ((unsigned)key[r] * 2654435761u) >> (32 - 9);
+      while (hk[h] != key[r]) h = (h + 1) & (kHashSlots - 1);
+      out_key[t] = key[r];
+      out_val[t] = hv[h];
+    }
+  }
+  if (lane == 0) ucount[i] = nd;
 }
 
 // Rows laid out by the clip pass (2D): one wave per block, rows i, i + grid,
@@ -3453,8 +3545,7 @@ static void assemble_mass_slots(Context& C, const DevMesh& A, const DevMesh& B, 
     hipLaunchKernelGGL((k_mass_rows_slots<512, 4, 9>), dim3(grid.x * 4), dim3(64), 0, C.stream, nn, raw_off, tkey,
                        tval, ucount, ovf);
   else
-    hipLaunchKernelGGL((k_mass_rows_gather<3, 2048, 2, true>), grid, dim3(128), 0, C.stream, nn, nptr, nullptr,
-                       nullptr, nullptr, nullptr, nullptr, nullptr, raw_off, tkey, tval, ucount, ovf);
+    hipLaunchKernelGGL((k_mass_rows_long<2048, 2>), grid, dim3(128), 0, C.stream, nn, raw_off, tkey, tval, ucount, ovf);
   LSM_HIP(hipGetLastError());
   // row lengths scanned before the overflow flag is known: one read-back for
   // both (an overflowing row leaves the scan meaningless, and it is unused)
@@ -3578,87 +3669,36 @@ void assemble_mass(Context& C, const DevMesh& A, const DevMesh& B, long npairs,
   const long nent = na * loc;
   hipLaunchKernelGGL(k_node_count, dim3(grid_for(nent, 256)), dim3(256), 0, C.stream, na, loc,
                      A.enlist_dev, ncount);
-  long* nptr = C.nuniq.as<long>(3 * (nn + 1));
-  long* raw = nptr + (nn + 1);
-  long* raw_off = raw + (nn + 1);
+  long* nptr = C.nuniq.as<long>(nn + 1);
   LSM_HIP(hipMemsetAsync(nptr, 0, sizeof(long), C.stream));
-  LSM_HIP(hipMemsetAsync(raw_off, 0, sizeof(long), C.stream));
   inclusive_scan_long(C, ncount, nptr + 1, nn);
   int* nlist = C.ukeys.as<int>(nent + 1);
   hipLaunchKernelGGL(k_node_fill, dim3(grid_for(nent, 256)), dim3(256), 0, C.stream, na, loc,
                      A.enlist_dev, nptr, cursor, nlist);
-  int* elem_ne = C.mkeys_alt.as<int>(na + 1);
-  hipLaunchKernelGGL(k_elem_nonempty, dim3(grid_for(na, 256)), dim3(256), 0, C.stream, na, out->indptr,
-                     out->counts, elem_ne);
-  long* contrib = C.mslot.as<long>(2 * nent + 2);
-  long* slot = contrib + nent + 1;
-  hipLaunchKernelGGL(k_node_rows, dim3(grid_for(nn, 256)), dim3(256), 0, C.stream, nn, loc, nptr, nlist,
-                     elem_ne, contrib);
-  LSM_HIP(hipGetLastError());
-  LSM_HIP(hipMemsetAsync(slot, 0, sizeof(long), C.stream));
-  inclusive_scan_long(C, contrib, slot + 1, nent);
-  hipLaunchKernelGGL(k_row_bounds, dim3(grid_for(nn + 1, 256)), dim3(256), 0, C.stream, nn, nptr, slot,
-                     raw_off, raw);
-  LSM_HIP(hipGetLastError());
-  long maxraw = 0;
-  {
-    // the longest row decides the LDS capacity of the row kernel
-    size_t bytes = 0;
-    long* dmax = reinterpret_cast<long*>(C.scalars.as<long>(64)) + 8;
-    LSM_HIP(rocprim::reduce(nullptr, bytes, raw, dmax, 0L, (size_t)nn, rocprim::maximum<long>(), C.stream));
-    void* tmp = C.sort_tmp.get(bytes);
-    LSM_HIP(rocprim::reduce(tmp, bytes, raw, dmax, 0L, (size_t)nn, rocprim::maximum<long>(), C.stream));
-    LSM_HIP(hipMemcpyAsync(&maxraw, dmax, sizeof(long), hipMemcpyDeviceToHost, C.stream));
-  }
-  long total_raw = 0;
-  LSM_HIP(hipMemcpyAsync(&total_raw, raw_off + nn, sizeof(long), hipMemcpyDeviceToHost, C.stream));
-  LSM_HIP(hipStreamSynchronize(C.stream));
-  if (maxraw > 2048) {  // rows too long for a register-resident sort: global sort path
-    assemble_mass_sorted(C, A, B, npairs, out);
-    return;
-  }
-  int* tkey = C.mkeys.as<int>(total_raw + 1);
-  double* tval = C.mvals.as<double>(total_raw + 1);
+  int* tkey = C.mkeys.as<int>((size_t)nn * kMaxDistinct);
+  double* tval = C.mvals.as<double>((size_t)nn * kMaxDistinct);
   long* ucount = C.mvals_alt.as<long>(nn + 1);
   int* ovf = C.scalars.as<int>(64) + 4;
   LSM_HIP(hipMemsetAsync(ovf, 0, sizeof(int), C.stream));
-  {
-    // rows gathered, deduplicated and summed in one pass (LDS capacity by the
-    // longest row)
-    int cus = 0;
-    LSM_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, C.device));
-    const dim3 grid((unsigned)std::max<long>(1, std::min<long>((long)(cus > 0 ? cus : 256) * 16, nn)));
-#define LSM_ROWS(L, CAPV, W)                                                                           \
-  hipLaunchKernelGGL((k_mass_rows_gather<L, CAPV, W>), grid, dim3(64 * W), 0, C.stream, nn, nptr, nlist,  \
-                     out->indptr, out->indices, out->counts, out->blocks, B.enlist_dev, raw_off, tkey,     \
-                     tval, ucount, ovf)
-    if (loc == 3) {
-      if (maxraw <= 512) LSM_ROWS(3, 512, 4);
-      else LSM_ROWS(3, 2048, 2);
-    } else {
-      if (maxraw <= 512) LSM_ROWS(4, 512, 4);
-      else LSM_ROWS(4, 2048, 2);
-    }
-#undef LSM_ROWS
-  }
+  hipLaunchKernelGGL(k_mass_rows_tet, dim3(grid_for(nn, 4)), dim3(256), 0, C.stream, nn, nptr, nlist, out->indptr,
+                     out->indices, out->counts, out->blocks, B.enlist_dev, tkey, tval, ucount, ovf);
   LSM_HIP(hipGetLastError());
-  int hovf = 0;
-  LSM_HIP(hipMemcpyAsync(&hovf, ovf, sizeof(int), hipMemcpyDeviceToHost, C.stream));
+  // scanned before the overflow flag is known: one read-back for both
+  inclusive_scan_long(C, ucount, mindptr + 1, nn);
+  C.hstat[2] = 0;
+  LSM_HIP(hipMemcpyAsync(C.hstat + 2, ovf, sizeof(int), hipMemcpyDeviceToHost, C.stream));
+  LSM_HIP(hipMemcpyAsync(C.hstat + 3, mindptr + nn, sizeof(long), hipMemcpyDeviceToHost, C.stream));
   LSM_HIP(hipStreamSynchronize(C.stream));
-  if (hovf) {  // a row with more distinct columns than the row kernel holds
+  if (*reinterpret_cast<const int*>(C.hstat + 2)) {  // a row with more distinct columns than the row kernel holds
     assemble_mass_sorted(C, A, B, npairs, out);
     return;
   }
-  inclusive_scan_long(C, ucount, mindptr + 1, nn);
-  long nnz = 0;
-  LSM_HIP(hipMemcpyAsync(&nnz, mindptr + nn, sizeof(long), hipMemcpyDeviceToHost, C.stream));
-  LSM_HIP(hipStreamSynchronize(C.stream));
+  const long nnz = C.hstat[3];
   int* mind = C.mindices.as<int>(nnz);
   double* mval = C.uvals.as<double>(nnz);
-  hipLaunchKernelGGL(k_mass_copy, dim3(grid_for(nn, 256 / kCopyLanes)), dim3(256), 0, C.stream, nn, raw_off, mindptr, tkey,
-                     tval, mind, mval);
+  hipLaunchKernelGGL(k_mass_copy, dim3(grid_for(nn, 256 / kCopyLanes)), dim3(256), 0, C.stream, nn, nullptr, mindptr,
+                     tkey, tval, mind, mval);
   LSM_HIP(hipGetLastError());
-  LSM_HIP(hipStreamSynchronize(C.stream));
   out->mass_nnz = nnz;
   out->mass_indices = mind;
   out->mass_values = mval;
