@@ -212,78 +212,93 @@ void stage_groups(Context& C, DevMesh& M, long ngroups, const long* offsets) {
 // Morton codes and bounds
 // ---------------------------------------------------------------------------
 
+// Bounds of the block's values b (minima, then maxima), in every lane.
 template <int DIM>
-__global__ void __launch_bounds__(kBlock)
-k_center_bounds(long ne, const double* __restrict__ bbox, double* __restrict__ partial) {
-  __shared__ double red[2 * DIM][kBlock];
-  double lo[DIM], hi[DIM];
-#pragma unroll
-  for (int d = 0; d < DIM; d++) {
-    lo[d] = __builtin_inf();
-    hi[d] = -__builtin_inf();
-  }
-  for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < ne; e += (long)gridDim.x * blockDim.x) {
+__device__ __forceinline__ void block_bounds(double* b) {
+  __shared__ double red[kBlock / 64][2 * DIM];
+  for (int o = 32; o > 0; o >>= 1) {
 #pragma unroll
     for (int d = 0; d < DIM; d++) {
-      double c = 0.5 * (bbox[(long)d * ne + e] + bbox[(long)(DIM + d) * ne + e]);
-      lo[d] = fmin_f(lo[d], c);
-      hi[d] = fmax_f(hi[d], c);
+      b[d] = fmin_f(b[d], __shfl_xor(b[d], o, 64));
+      b[DIM + d] = fmax_f(b[DIM + d], __shfl_xor(b[DIM + d], o, 64));
     }
   }
+  if ((threadIdx.x & 63) == 0) {
 #pragma unroll
-  for (int d = 0; d < DIM; d++) {
-    red[d][threadIdx.x] = lo[d];
-    red[DIM + d][threadIdx.x] = hi[d];
+    for (int k = 0; k < 2 * DIM; k++) red[threadIdx.x >> 6][k] = b[k];
   }
   __syncthreads();
-  for (int s = kBlock / 2; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) {
 #pragma unroll
-      for (int d = 0; d < DIM; d++) {
-        red[d][threadIdx.x] = fmin_f(red[d][threadIdx.x], red[d][threadIdx.x + s]);
-        red[DIM + d][threadIdx.x] = fmax_f(red[DIM + d][threadIdx.x], red[DIM + d][threadIdx.x + s]);
-      }
+  for (int w = 0; w < kBlock / 64; w++) {
+#pragma unroll
+    for (int d = 0; d < DIM; d++) {
+      b[d] = fmin_f(b[d], red[w][d]);
+      b[DIM + d] = fmax_f(b[DIM + d], red[w][DIM + d]);
     }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-#pragma unroll
-    for (int k = 0; k < 2 * DIM; k++) partial[blockIdx.x * 2 * DIM + k] = red[k][0];
   }
 }
 
+// A sort of one mesh's elements by Morton code, or of two meshes' (the
+// hierarchy's and the queries') in the same launches.
+//
+// A least-significant-digit radix sort, four passes of 8 bits: a pass counts
+// the digits of every tile of kTile keys, then every tile adds up the counts
+// before its own and moves its keys.  The counts of 2^shift tiles are also
+// summed, so that a tile reads about 2 sqrt(tiles) rows of 256 counts.  Nine
+// launches for both meshes and no block waits for another; the passes of a
+// chained scan, where each block waits for the one before, took 30 us each
+// for 2 M keys and three launches, and the merge sort below 1 M keys 11 to 21
+// launches.
+constexpr int kSortItems = 8;
+constexpr int kTile = kSortItems * kBlock;
+constexpr int kDigits = 256;
+constexpr int kSortPasses = 4;
+constexpr int kBoundParts = 256;
+
+struct OrderJob {
+  long ne;
+  const double* bbox;
+  const int* group;   // batches: the elements' meshes, above the code's leading bits
+  int gbits;
+  int nparts;
+  double* bounds;     // [nparts][2 DIM]: parts of the centres' bounds
+  uint32_t* keys[2];
+  int* vals[2];
+  int* perm;          // the order
+  unsigned* counts;   // [tiles][kDigits]
+  unsigned* sums;     // [kSortPasses][groups][kDigits]: counts of 2^shift tiles
+  int tiles, groups, shift;
+};
+
+struct OrderArgs {
+  OrderJob job[2];
+};
+
 template <int DIM>
-__global__ void __launch_bounds__(kBlock) k_bounds_final(int nparts, double* __restrict__ partial) {
-  __shared__ double red[2 * DIM][kBlock];
+__global__ void __launch_bounds__(kBlock) k_center_bounds(OrderArgs args) {
+  const OrderJob& J = args.job[blockIdx.y];
+  for (long k = (long)blockIdx.x * kBlock + threadIdx.x; k < (long)kSortPasses * J.groups * kDigits;
+       k += (long)gridDim.x * kBlock)
+    J.sums[k] = 0;
+  if ((int)blockIdx.x >= J.nparts) return;
   double b[2 * DIM];
 #pragma unroll
   for (int d = 0; d < DIM; d++) {
     b[d] = __builtin_inf();
     b[DIM + d] = -__builtin_inf();
   }
-  for (int p = threadIdx.x; p < nparts; p += kBlock) {
+  for (long e = (long)blockIdx.x * kBlock + threadIdx.x; e < J.ne; e += (long)J.nparts * kBlock) {
 #pragma unroll
     for (int d = 0; d < DIM; d++) {
-      b[d] = fmin_f(b[d], partial[p * 2 * DIM + d]);
-      b[DIM + d] = fmax_f(b[DIM + d], partial[p * 2 * DIM + DIM + d]);
+      double c = 0.5 * (J.bbox[(long)d * J.ne + e] + J.bbox[(long)(DIM + d) * J.ne + e]);
+      b[d] = fmin_f(b[d], c);
+      b[DIM + d] = fmax_f(b[DIM + d], c);
     }
   }
-#pragma unroll
-  for (int k = 0; k < 2 * DIM; k++) red[k][threadIdx.x] = b[k];
-  __syncthreads();
-  for (int s = kBlock / 2; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) {
-#pragma unroll
-      for (int d = 0; d < DIM; d++) {
-        red[d][threadIdx.x] = fmin_f(red[d][threadIdx.x], red[d][threadIdx.x + s]);
-        red[DIM + d][threadIdx.x] = fmax_f(red[DIM + d][threadIdx.x], red[DIM + d][threadIdx.x + s]);
-      }
-    }
-    __syncthreads();
-  }
+  block_bounds<DIM>(b);
   if (threadIdx.x == 0) {
 #pragma unroll
-    for (int k = 0; k < 2 * DIM; k++) partial[k] = red[k][0];
+    for (int k = 0; k < 2 * DIM; k++) J.bounds[blockIdx.x * 2 * DIM + k] = b[k];
   }
 }
 
@@ -309,70 +324,280 @@ __device__ __forceinline__ uint64_t spread3(uint64_t x) {  // 21 bits -> every t
 
 // Sort key of element e: its Morton code, or in a batch the mesh id in the
 // top gbits bits above the code's leading bits, so that each mesh is one
-// contiguous run of the order.
+// contiguous run of the order.  The leading 32 bits (16 per axis in 2D, 10-11
+// in 3D, below a batch's mesh id) order the elements finely enough for the
+// hierarchy; ties keep element order (the sort is stable), and the candidate
+// sets do not depend on the order at all.
 template <int DIM>
-__global__ void __launch_bounds__(kBlock)
-k_morton(long ne, const double* __restrict__ bbox, const double* __restrict__ bounds,
-         const int* __restrict__ group, int gbits, uint32_t* __restrict__ keys,
-         int* __restrict__ vals) {
-  long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= ne) return;
+__device__ __forceinline__ uint32_t morton_key(const OrderJob& J, const double* bounds, long e) {
   constexpr int BITS = DIM == 2 ? 32 : 21;
   const double maxq = (double)((1ULL << BITS) - 1);
   uint64_t code = 0;
 #pragma unroll
   for (int d = 0; d < DIM; d++) {
     double lo = bounds[d], hi = bounds[DIM + d];
-    double c = 0.5 * (bbox[(long)d * ne + e] + bbox[(long)(DIM + d) * ne + e]);
+    double c = 0.5 * (J.bbox[(long)d * J.ne + e] + J.bbox[(long)(DIM + d) * J.ne + e]);
     double t = hi > lo ? (c - lo) / (hi - lo) : 0.0;
     t = fmin_f(fmax_f(t, 0.0), 1.0);
     uint64_t q = (uint64_t)(t * maxq);
     code |= (DIM == 2 ? spread2(q) : spread3(q)) << d;
   }
   constexpr int KEYBITS = DIM == 2 ? 64 : 63;
-  if (group && gbits > 0) code = ((uint64_t)group[e] << (KEYBITS - gbits)) | (code >> gbits);
-  // the leading 32 bits (16 per axis in 2D, 10-11 in 3D, below a batch's
-  // mesh id) order the elements finely enough for the hierarchy; ties keep
-  // element order (the sort is stable), and the candidate sets do not depend
-  // on the order at all
-  keys[e] = (uint32_t)(code >> (KEYBITS - 32));
-  vals[e] = (int)e;
+  if (J.group && J.gbits > 0) code = ((uint64_t)J.group[e] << (KEYBITS - J.gbits)) | (code >> J.gbits);
+  return (uint32_t)(code >> (KEYBITS - 32));
 }
 
+// The block's job and its tile in that job.
+__device__ __forceinline__ const OrderJob& tile_job(const OrderArgs& args, int& tile) {
+  tile = blockIdx.x;
+  if (tile < args.job[0].tiles) return args.job[0];
+  tile -= args.job[0].tiles;
+  return args.job[1];
+}
 
-// Sorts the elements of M by Morton code; returns the permutation in `perm`.
-static void morton_order(Context& C, const DevMesh& M, DevBuf& perm) {
-  long ne = M.nelements;
-  int dim = M.dim;
-  int nparts = (int)std::min<long>(1024, std::max<long>(1, (ne + kBlock - 1) / kBlock));
-  double* part = C.partials.as<double>((size_t)nparts * 6 + 6);
-  uint32_t* keys = C.keys.as<uint32_t>(ne);
-  uint32_t* keys2 = C.keys_alt.as<uint32_t>(ne);
-  int* vals = C.vals.as<int>(ne);
-  int* out = perm.as<int>(ne);
-  const double* bbox = static_cast<const double*>(M.bbox.ptr);
-  const int* group = M.ngroups > 0 ? static_cast<const int*>(M.group.ptr) : nullptr;
-  int gbits = 0;
-  while (group && (1L << gbits) < M.ngroups) gbits++;
-  if (dim == 2) {
-    hipLaunchKernelGGL(k_center_bounds<2>, dim3(nparts), dim3(kBlock), 0, C.stream, ne, bbox, part);
-    hipLaunchKernelGGL(k_bounds_final<2>, dim3(1), dim3(kBlock), 0, C.stream, nparts, part);
-    hipLaunchKernelGGL(k_morton<2>, dim3(grid_for(ne, kBlock)), dim3(kBlock), 0, C.stream, ne, bbox,
-                       part, group, gbits, keys, vals);
-  } else {
-    hipLaunchKernelGGL(k_center_bounds<3>, dim3(nparts), dim3(kBlock), 0, C.stream, ne, bbox, part);
-    hipLaunchKernelGGL(k_bounds_final<3>, dim3(1), dim3(kBlock), 0, C.stream, nparts, part);
-    hipLaunchKernelGGL(k_morton<3>, dim3(grid_for(ne, kBlock)), dim3(kBlock), 0, C.stream, ne, bbox,
-                       part, group, gbits, keys, vals);
+// A tile's digit counts to its row and to its group's sums.
+__device__ __forceinline__ void write_counts(const OrderJob& J, int tile, int pass, unsigned n) {
+  J.counts[(long)tile * kDigits + threadIdx.x] = n;
+  if (n) atomicAdd(J.sums + ((long)pass * J.groups + (tile >> J.shift)) * kDigits + threadIdx.x, n);
+}
+
+// Keys of a tile's elements, and the counts of their lowest digit.  With
+// `vals`, element ids beside the keys, for the library's sort.
+template <int DIM, bool VALS>
+__global__ void __launch_bounds__(kBlock) k_morton(OrderArgs args) {
+  __shared__ unsigned hist[kDigits];
+  int tile;
+  const OrderJob& J = tile_job(args, tile);
+  double b[2 * DIM];
+#pragma unroll
+  for (int d = 0; d < DIM; d++) {
+    b[d] = __builtin_inf();
+    b[DIM + d] = -__builtin_inf();
   }
+  if ((int)threadIdx.x < J.nparts) {
+#pragma unroll
+    for (int k = 0; k < 2 * DIM; k++) b[k] = J.bounds[threadIdx.x * 2 * DIM + k];
+  }
+  hist[threadIdx.x] = 0;
+  block_bounds<DIM>(b);  // a barrier
+#pragma unroll
+  for (int i = 0; i < kSortItems; i++) {
+    const long e = (long)tile * kTile + i * kBlock + threadIdx.x;
+    if (e >= J.ne) break;
+    const uint32_t key = morton_key<DIM>(J, b, e);
+    J.keys[0][e] = key;
+    if (VALS) J.vals[0][e] = (int)e;
+    else atomicAdd(&hist[key & (kDigits - 1)], 1u);
+  }
+  if (VALS) return;
+  __syncthreads();
+  write_counts(J, tile, 0, hist[threadIdx.x]);
+}
+
+__global__ void __launch_bounds__(kBlock) k_sort_counts(OrderArgs args, int pass) {
+  __shared__ unsigned hist[kDigits];
+  int tile;
+  const OrderJob& J = tile_job(args, tile);
+  const uint32_t* __restrict__ keys = J.keys[pass & 1];
+  hist[threadIdx.x] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kSortItems; i++) {
+    const long e = (long)tile * kTile + i * kBlock + threadIdx.x;
+    if (e < J.ne) atomicAdd(&hist[(keys[e] >> (8 * pass)) & (kDigits - 1)], 1u);
+  }
+  __syncthreads();
+  write_counts(J, tile, pass, hist[threadIdx.x]);
+}
+
+// Moves a tile's keys and element ids to their places for one digit.  A wave
+// ranks 64 keys at a time among its own (the lanes of equal digit by eight
+// ballots), the tile is put in digit order in LDS, and neighbouring lanes
+// then write neighbouring places.  The first pass's ids are the indices, the
+// last one writes the order alone.
+template <int PASS>
+__global__ void __launch_bounds__(kBlock) k_sort_move(OrderArgs args) {
+  constexpr int kWaves = kBlock / 64;
+  constexpr bool kLast = PASS == kSortPasses - 1;
+  __shared__ unsigned hist[kWaves][kDigits], place[kDigits], wsum[2][kWaves];
+  __shared__ uint32_t skey[kTile];
+  __shared__ int sval[kTile];
+  int tile;
+  const OrderJob& J = tile_job(args, tile);
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const uint32_t* __restrict__ keys = J.keys[PASS & 1];
+  const int* __restrict__ vals = J.vals[PASS & 1];
+  const long first = (long)tile * kTile;
+  const int n = J.ne - first < kTile ? (int)(J.ne - first) : kTile;
+#pragma unroll
+  for (int w = 0; w < kWaves; w++) hist[w][t] = 0;
+  uint32_t key[kSortItems];
+  int val[kSortItems], rank[kSortItems];
+#pragma unroll
+  for (int i = 0; i < kSortItems; i++) {
+    const int k = (wave * kSortItems + i) * 64 + lane;
+    key[i] = k < n ? keys[first + k] : 0;
+    val[i] = PASS == 0 ? (int)(first + k) : (k < n ? vals[first + k] : 0);
+  }
+  // digit t: its keys in all tiles, and in the tiles before this one
+  unsigned all = 0, before = 0;
+  {
+    const int mine = tile >> J.shift;
+    const unsigned* __restrict__ s = J.sums + (long)PASS * J.groups * kDigits + t;
+#pragma unroll 8
+    for (int g = 0; g < J.groups; g++) {
+      const unsigned v = s[(long)g * kDigits];
+      all += v;
+      before += g < mine ? v : 0u;
+    }
+    const unsigned* __restrict__ c = J.counts + t;
+#pragma unroll 8
+    for (int k = mine << J.shift; k < tile; k++) before += c[(long)k * kDigits];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kSortItems; i++) {
+    const bool live = (wave * kSortItems + i) * 64 + lane < n;
+    const unsigned d = (key[i] >> (8 * PASS)) & (kDigits - 1);
+    unsigned long long m = __ballot(live);
+#pragma unroll
+    for (int b = 0; b < 8; b++) {
+      const unsigned long long v = __ballot((d >> b) & 1u);
+      m &= (d >> b) & 1u ? v : ~v;
+    }
+    const int lower = __builtin_popcountll(m & ((1ULL << lane) - 1));
+    unsigned old = 0;
+    if (live && lower == 0) old = atomicAdd(&hist[wave][d], (unsigned)__builtin_popcountll(m));
+    rank[i] = (int)__shfl(old, live ? __builtin_ctzll(m) : lane, 64) + lower;
+  }
+  __syncthreads();
+  unsigned mine = 0;  // digit t's keys in this tile; each wave's first place among them
+#pragma unroll
+  for (int w = 0; w < kWaves; w++) {
+    const unsigned c = hist[w][t];
+    hist[w][t] = mine;
+    mine += c;
+  }
+  unsigned local = mine, global = all;  // inclusive scans over the digits
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const unsigned x = __shfl_up(local, o, 64), y = __shfl_up(global, o, 64);
+    if (lane >= o) {
+      local += x;
+      global += y;
+    }
+  }
+  if (lane == 63) {
+    wsum[0][wave] = local;
+    wsum[1][wave] = global;
+  }
+  __syncthreads();
+  for (int w = 0; w < wave; w++) {
+    local += wsum[0][w];
+    global += wsum[1][w];
+  }
+  local -= mine;  // digit t's first place in the tile
+#pragma unroll
+  for (int w = 0; w < kWaves; w++) hist[w][t] += local;
+  place[t] = global - all + before - local;  // place in the output = this + place in the tile
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kSortItems; i++) {
+    if ((wave * kSortItems + i) * 64 + lane < n) {
+      const unsigned o = hist[wave][(key[i] >> (8 * PASS)) & (kDigits - 1)] + (unsigned)rank[i];
+      skey[o] = key[i];
+      sval[o] = val[i];
+    }
+  }
+  __syncthreads();
+  int* __restrict__ out = kLast ? J.perm : J.vals[(PASS + 1) & 1];
+#pragma unroll
+  for (int i = 0; i < kSortItems; i++) {
+    const int k = i * kBlock + t;
+    if (k >= n) break;
+    const unsigned o = place[(skey[k] >> (8 * PASS)) & (kDigits - 1)] + (unsigned)k;
+    if (!kLast) J.keys[(PASS + 1) & 1][o] = skey[k];
+    out[o] = sval[k];
+  }
+}
+
+// Elements of a mesh above which the library's sort takes over: a tile then
+// reads more counts than keys.
+constexpr long kOrderMax = 1L << 23;
+
+// Sorts the elements of M[0], and of M[1] if it is given, by Morton code:
+// perm[j] gets the permutation.
+static void morton_order(Context& C, int n, const DevMesh* const* M, DevBuf* const* perm) {
+  OrderArgs args = {};
+  size_t total = 0, words = 0;
+  bool large = false;
+  for (int j = 0; j < n; j++) {
+    OrderJob& J = args.job[j];
+    J.ne = M[j]->nelements;
+    J.bbox = static_cast<const double*>(M[j]->bbox.ptr);
+    J.group = M[j]->ngroups > 0 ? static_cast<const int*>(M[j]->group.ptr) : nullptr;
+    while (J.group && (1L << J.gbits) < M[j]->ngroups) J.gbits++;
+    J.nparts = (int)std::min<long>(kBoundParts, (J.ne + kBlock - 1) / kBlock);
+    J.tiles = (int)((J.ne + kTile - 1) / kTile);
+    while ((1 << (2 * J.shift)) < J.tiles) J.shift++;
+    J.groups = (J.tiles + (1 << J.shift) - 1) >> J.shift;
+    J.perm = perm[j]->as<int>(J.ne);
+    total += (size_t)J.ne;
+    words += (size_t)(J.tiles + kSortPasses * J.groups) * kDigits;
+    large = large || J.ne > kOrderMax;
+  }
+  double* part = C.partials.as<double>((size_t)n * kBoundParts * 6);
+  uint32_t* keys[2] = {C.keys.as<uint32_t>(total), C.keys_alt.as<uint32_t>(total)};
+  int* vals[2] = {C.vals.as<int>(total), C.vals_alt.as<int>(total)};
+  unsigned* table = large ? nullptr : C.sort_tmp.as<unsigned>(words);
+  size_t at = 0;
+  for (int j = 0; j < n; j++) {
+    OrderJob& J = args.job[j];
+    J.bounds = part + (size_t)j * kBoundParts * 6;
+    for (int k = 0; k < 2; k++) {
+      J.keys[k] = keys[k] + at;
+      J.vals[k] = vals[k] + at;
+    }
+    at += (size_t)J.ne;
+    if (large) {
+      J.groups = 0;
+      continue;
+    }
+    J.counts = table;
+    J.sums = table + (size_t)J.tiles * kDigits;
+    table += (size_t)(J.tiles + kSortPasses * J.groups) * kDigits;
+  }
+  const dim3 block(kBlock), parts((unsigned)std::max(1, std::max(args.job[0].nparts, args.job[1].nparts)), (unsigned)n);
+  const dim3 tiles((unsigned)std::max(1, args.job[0].tiles + args.job[1].tiles));
+  const bool flat = M[0]->dim == 2;
+  if (flat) hipLaunchKernelGGL(k_center_bounds<2>, parts, block, 0, C.stream, args);
+  else hipLaunchKernelGGL(k_center_bounds<3>, parts, block, 0, C.stream, args);
+  if (large) {
+    if (flat) hipLaunchKernelGGL((k_morton<2, true>), tiles, block, 0, C.stream, args);
+    else hipLaunchKernelGGL((k_morton<3, true>), tiles, block, 0, C.stream, args);
+    LSM_HIP(hipGetLastError());
+    for (int j = 0; j < n; j++) {
+      const OrderJob& J = args.job[j];
+      if (J.ne == 0) continue;
+      size_t bytes = 0;
+      LSM_HIP(rocprim::radix_sort_pairs(nullptr, bytes, J.keys[0], J.keys[1], J.vals[0], J.perm, (size_t)J.ne, 0u, 32u,
+                                        C.stream));
+      void* tmp = C.sort_tmp.get(bytes);
+      LSM_HIP(rocprim::radix_sort_pairs(tmp, bytes, J.keys[0], J.keys[1], J.vals[0], J.perm, (size_t)J.ne, 0u, 32u,
+                                        C.stream));
+    }
+    return;
+  }
+  if (flat) hipLaunchKernelGGL((k_morton<2, false>), tiles, block, 0, C.stream, args);
+  else hipLaunchKernelGGL((k_morton<3, false>), tiles, block, 0, C.stream, args);
+  hipLaunchKernelGGL(k_sort_move<0>, tiles, block, 0, C.stream, args);
+  hipLaunchKernelGGL(k_sort_counts, tiles, block, 0, C.stream, args, 1);
+  hipLaunchKernelGGL(k_sort_move<1>, tiles, block, 0, C.stream, args);
+  hipLaunchKernelGGL(k_sort_counts, tiles, block, 0, C.stream, args, 2);
+  hipLaunchKernelGGL(k_sort_move<2>, tiles, block, 0, C.stream, args);
+  hipLaunchKernelGGL(k_sort_counts, tiles, block, 0, C.stream, args, 3);
+  hipLaunchKernelGGL(k_sort_move<3>, tiles, block, 0, C.stream, args);
   LSM_HIP(hipGetLastError());
-  const unsigned begin_bit = 0, end_bit = 32;
-  size_t tmp_bytes = 0;
-  LSM_HIP(rocprim::radix_sort_pairs(nullptr, tmp_bytes, keys, keys2, vals, out, (size_t)ne, begin_bit,
-                                    end_bit, C.stream));
-  void* tmp = C.sort_tmp.get(tmp_bytes);
-  LSM_HIP(rocprim::radix_sort_pairs(tmp, tmp_bytes, keys, keys2, vals, out, (size_t)ne, begin_bit, end_bit,
-                                    C.stream));
 }
 
 // ---------------------------------------------------------------------------
@@ -385,50 +610,105 @@ struct LevelInfo {
   long offset[32];
 };
 
-// Level-0 boxes (node-major: [lo_0..lo_{dim-1}, hi_0..hi_{dim-1}]) in sorted order.
+// Boxes (node-major: [lo_0..lo_{dim-1}, hi_0..hi_{dim-1}]) and, in batches,
+// mesh ranges of the three levels above `l0`, and of the elements themselves
+// in sorted order if l0 is 0: a wave's 64 nodes have eight parents and one
+// grandparent, which come from shuffles, and the block's 512 one node above
+// those.  (A launch a level took 5 us each; the nodes were read again.)
+constexpr int kLevelBlock = kFanout * kFanout * kFanout;
 template <int DIM>
-__global__ void __launch_bounds__(kBlock)
-k_leaf_boxes(long ne, const double* __restrict__ bbox, const int* __restrict__ perm,
-             double* __restrict__ boxes, const int* __restrict__ group, int* __restrict__ granges) {
-  long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= ne) return;
-  long e = perm[i];
-#pragma unroll
-  for (int k = 0; k < 2 * DIM; k++) boxes[i * 2 * DIM + k] = bbox[(long)k * ne + e];
-  if (group) {
-    granges[2 * i] = group[e];
-    granges[2 * i + 1] = group[e];
-  }
-}
-
-template <int DIM>
-__global__ void __launch_bounds__(kBlock)
-k_parent_boxes(long nchild, long nparent, const double* __restrict__ child, double* __restrict__ parent,
-               const int* __restrict__ cg, int* __restrict__ pg) {
-  long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nparent) return;
+__global__ void __launch_bounds__(kLevelBlock)
+k_build_levels(LevelInfo info, int l0, long ne, const double* __restrict__ bbox, const int* __restrict__ perm,
+               const int* __restrict__ group, double* __restrict__ boxes, int* __restrict__ granges) {
+  __shared__ double top[kFanout][2 * DIM];
+  __shared__ int topg[kFanout][2];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const long i = (long)blockIdx.x * kLevelBlock + threadIdx.x;
   double b[2 * DIM];
-  long c0 = i * kFanout;
-  long c1 = c0 + kFanout < nchild ? c0 + kFanout : nchild;
 #pragma unroll
-  for (int k = 0; k < 2 * DIM; k++) b[k] = child[c0 * 2 * DIM + k];
-  for (long c = c0 + 1; c < c1; c++) {
+  for (int d = 0; d < DIM; d++) {
+    b[d] = __builtin_inf();
+    b[DIM + d] = -__builtin_inf();
+  }
+  int glo = 0x7fffffff, ghi = -1;
+  auto store = [&](int l, long node) {
+    if (l >= info.levels || node >= info.count[l]) return;
+    const long o = info.offset[l] + node;
+#pragma unroll
+    for (int k = 0; k < 2 * DIM; k++) boxes[o * 2 * DIM + k] = b[k];
+    if (granges) {
+      granges[2 * o] = glo;
+      granges[2 * o + 1] = ghi;
+    }
+  };
+  auto join = [&](int o) {
 #pragma unroll
     for (int d = 0; d < DIM; d++) {
-      b[d] = fmin_f(b[d], child[c * 2 * DIM + d]);
-      b[DIM + d] = fmax_f(b[DIM + d], child[c * 2 * DIM + DIM + d]);
+      b[d] = __builtin_fmin(b[d], __shfl_xor(b[d], o, 64));
+      b[DIM + d] = __builtin_fmax(b[DIM + d], __shfl_xor(b[DIM + d], o, 64));
+    }
+    if (granges) {
+      glo = std::min(glo, __shfl_xor(glo, o, 64));
+      ghi = std::max(ghi, __shfl_xor(ghi, o, 64));
+    }
+  };
+  if (i < info.count[l0]) {
+    if (l0 == 0) {
+      const long e = perm[i];
+#pragma unroll
+      for (int k = 0; k < 2 * DIM; k++) b[k] = bbox[(long)k * ne + e];
+      if (granges) glo = ghi = group[e];
+      store(0, i);
+    } else {
+      const long o = info.offset[l0] + i;
+#pragma unroll
+      for (int k = 0; k < 2 * DIM; k++) b[k] = boxes[o * 2 * DIM + k];
+      if (granges) {
+        glo = granges[2 * o];
+        ghi = granges[2 * o + 1];
+      }
     }
   }
+  join(1);
+  join(2);
+  join(4);
+  if ((lane & 7) == 0) store(l0 + 1, i / kFanout);
+  join(8);
+  join(16);
+  join(32);
+  if (lane == 0) {
+    store(l0 + 2, i / (kFanout * kFanout));
 #pragma unroll
-  for (int k = 0; k < 2 * DIM; k++) parent[i * 2 * DIM + k] = b[k];
-  if (cg) {
-    // children are in mesh order: the first one holds the lowest id
-    pg[2 * i] = cg[2 * c0];
-    pg[2 * i + 1] = cg[2 * (c1 - 1) + 1];
+    for (int k = 0; k < 2 * DIM; k++) top[wave][k] = b[k];
+    topg[wave][0] = glo;
+    topg[wave][1] = ghi;
   }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+#pragma unroll
+  for (int w = 1; w < kFanout; w++) {
+#pragma unroll
+    for (int d = 0; d < DIM; d++) {
+      b[d] = __builtin_fmin(b[d], top[w][d]);
+      b[DIM + d] = __builtin_fmax(b[DIM + d], top[w][DIM + d]);
+    }
+    glo = std::min(glo, topg[w][0]);
+    ghi = std::max(ghi, topg[w][1]);
+  }
+  store(l0 + 3, blockIdx.x);
 }
 
-void build_bvh(Context& C, const DevMesh& B) {
+static LevelInfo level_info(const DevBVH& H) {
+  LevelInfo info;
+  info.levels = H.levels;
+  for (int l = 0; l < 32; l++) {
+    info.count[l] = l < H.levels ? H.count[l] : 0;
+    info.offset[l] = l < H.levels ? H.offset[l] : 0;
+  }
+  return info;
+}
+
+void build_bvh(Context& C, const DevMesh& B, const DevMesh* A) {
   DevBVH& H = C.bvh;
   H.dim = B.dim;
   H.n = B.nelements;
@@ -436,7 +716,9 @@ void build_bvh(Context& C, const DevMesh& B) {
     H.levels = 0;
     return;
   }
-  morton_order(C, B, H.perm);
+  const DevMesh* meshes[2] = {&B, A};
+  DevBuf* orders[2] = {&H.perm, &C.qperm};
+  morton_order(C, A ? 2 : 1, meshes, orders);
   long n = H.n;
   int L = 0;
   long total = 0;
@@ -451,31 +733,18 @@ void build_bvh(Context& C, const DevMesh& B) {
   }
   H.levels = L;
   H.total = total;
-  int w = 2 * B.dim;
   // a walk reads whole groups of children, past the last node too
-  double* boxes = H.boxes.as<double>((size_t)(total + kFanout) * w);
+  double* boxes = H.boxes.as<double>((size_t)(total + kFanout) * 2 * B.dim);
   const double* bbox = static_cast<const double*>(B.bbox.ptr);
   const int* perm = static_cast<const int*>(H.perm.ptr);
   H.grouped = B.ngroups > 0;
   const int* group = H.grouped ? static_cast<const int*>(B.group.ptr) : nullptr;
   int* gr = H.grouped ? H.granges.as<int>((size_t)(total + kFanout) * 2) : nullptr;
-  if (B.dim == 2)
-    hipLaunchKernelGGL(k_leaf_boxes<2>, dim3(grid_for(H.n, kBlock)), dim3(kBlock), 0, C.stream, H.n,
-                       bbox, perm, boxes, group, gr);
-  else
-    hipLaunchKernelGGL(k_leaf_boxes<3>, dim3(grid_for(H.n, kBlock)), dim3(kBlock), 0, C.stream, H.n,
-                       bbox, perm, boxes, group, gr);
-  for (int l = 1; l < L; l++) {
-    const double* ch = boxes + H.offset[l - 1] * w;
-    double* pa = boxes + H.offset[l] * w;
-    const int* cg = gr ? gr + 2 * H.offset[l - 1] : nullptr;
-    int* pg = gr ? gr + 2 * H.offset[l] : nullptr;
-    if (B.dim == 2)
-      hipLaunchKernelGGL(k_parent_boxes<2>, dim3(grid_for(H.count[l], kBlock)), dim3(kBlock), 0,
-                         C.stream, H.count[l - 1], H.count[l], ch, pa, cg, pg);
-    else
-      hipLaunchKernelGGL(k_parent_boxes<3>, dim3(grid_for(H.count[l], kBlock)), dim3(kBlock), 0,
-                         C.stream, H.count[l - 1], H.count[l], ch, pa, cg, pg);
+  const LevelInfo info = level_info(H);
+  for (int l = 0; l == 0 || l + 1 < L; l += 3) {
+    const dim3 grid(grid_for(H.count[l], kLevelBlock)), block(kLevelBlock);
+    if (B.dim == 2) hipLaunchKernelGGL(k_build_levels<2>, grid, block, 0, C.stream, info, l, H.n, bbox, perm, group, boxes, gr);
+    else hipLaunchKernelGGL(k_build_levels<3>, grid, block, 0, C.stream, info, l, H.n, bbox, perm, group, boxes, gr);
   }
   LSM_HIP(hipGetLastError());
 }
@@ -882,7 +1151,7 @@ static int task_level(const LevelInfo& info, long waves, bool grouped) {
   return level < top ? level : top;
 }
 
-long find_pairs(Context& C, const DevMesh& A, const DevMesh& B, int finder, int sort_rows) {
+long find_pairs(Context& C, const DevMesh& A, const DevMesh& B, int finder, int sort_rows, bool ordered) {
   long na = A.nelements;
   long* row_count = C.row_count.as<long>(na + 1);
   long* indptr = C.indptr.as<long>(na + 1);
@@ -893,7 +1162,11 @@ long find_pairs(Context& C, const DevMesh& A, const DevMesh& B, int finder, int 
   }
   LSM_REQUIRE(A.dim == B.dim, LIBSUPERMESH_GPU_ERROR_INVALID, "Invalid dimension: meshes differ");
   const DevBVH& H = C.bvh;
-  morton_order(C, A, C.qperm);
+  if (!ordered) {
+    const DevMesh* mesh = &A;
+    DevBuf* order = &C.qperm;
+    morton_order(C, 1, &mesh, &order);
+  }
   LSM_REQUIRE((A.ngroups > 0) == H.grouped && (!H.grouped || A.ngroups == B.ngroups),
               LIBSUPERMESH_GPU_ERROR_INVALID, "batches of A and B hold different mesh counts");
   LSM_REQUIRE(H.levels <= 17, LIBSUPERMESH_GPU_ERROR_OVERFLOW, "hierarchy too deep");
@@ -907,11 +1180,7 @@ long find_pairs(Context& C, const DevMesh& A, const DevMesh& B, int finder, int 
   s.granges = H.grouped ? static_cast<const int*>(H.granges.ptr) : nullptr;
   s.boxes = static_cast<const double*>(H.boxes.ptr);
   s.perm = static_cast<const int*>(H.perm.ptr);
-  s.info.levels = H.levels;
-  for (int l = 0; l < 32; l++) {
-    s.info.count[l] = l < H.levels ? H.count[l] : 0;
-    s.info.offset[l] = l < H.levels ? H.offset[l] : 0;
-  }
+  s.info = level_info(H);
   s.row_count = row_count;
   s.indptr = indptr;
   s.level = task_level(s.info, waves, H.grouped);
@@ -1030,7 +1299,7 @@ long find_pairs_from_b(Context& C, const DevMesh& A, const DevMesh& B, int finde
   // B's elements query the hierarchy over A (built by the caller): a CSR over
   // B, in B id order, whose entries are A ids.  The overlap tests are
   // symmetric in the two boxes, so the pair set is the one A's queries find.
-  const long npairs = find_pairs(C, B, A, finder, 0);
+  const long npairs = find_pairs(C, B, A, finder, 0, true);
   const long na = A.nelements;
   long* indptr = C.indptr.as<long>(na + 1);
   if (npairs == 0) {

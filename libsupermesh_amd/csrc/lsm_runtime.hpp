@@ -184,11 +184,14 @@ int* stage_flag(Context& C);
 // Mesh id of every element of a batch from its element offsets (device,
 // [ngroups + 1]); validates the offsets.
 void stage_groups(Context& C, DevMesh& M, long ngroups, const long* offsets);
-void build_bvh(Context& C, const DevMesh& B);
+// The hierarchy over B; with A, also the order (C.qperm) that find_pairs takes
+// A's elements in, sorted in the same launches.
+void build_bvh(Context& C, const DevMesh& B, const DevMesh* A = nullptr);
 // Count / fill candidate pairs of A against the BVH of B.  Returns npairs.
-long find_pairs(Context& C, const DevMesh& A, const DevMesh& B, int finder, int sort_rows);
+// ordered: build_bvh was given A.
+long find_pairs(Context& C, const DevMesh& A, const DevMesh& B, int finder, int sort_rows, bool ordered = false);
 // The same pairs found the other way round (B's elements query a hierarchy
-// over A), regrouped as a CSR over A with every row in ascending B id order.
+// over A, built with B's order), regrouped as a CSR over A with every row in ascending B id order.
 long find_pairs_from_b(Context& C, const DevMesh& A, const DevMesh& B, int finder);
 
 // Clipping (supermesh.hip).
