@@ -61,6 +61,7 @@ static void init_context(Context& C, int device) {
   for (int i = 0; i < 16; i++) LSM_HIP(hipEventCreate(&C.ev[i]));
   C.events = true;
   LSM_HIP(hipHostMalloc(reinterpret_cast<void**>(&C.hstat), 64 * sizeof(long), hipHostMallocDefault));
+  LSM_HIP(hipMemset(C.scalars.get(1024), 0, 1024));
 }
 
 static void free_context(Context& C) {
@@ -174,13 +175,7 @@ static void run_supermesh(Context& C, const libsupermesh_gpu_mesh* a, const libs
   ph.mark();
   // the node-index check of both meshes is read back with the candidate count
   // (a bad index is clamped on the device, so the search in between is safe)
-  int* bad = stage_flag(C);
-  LSM_HIP(hipMemsetAsync(bad, 0, sizeof(int), C.stream));
-  stage_mesh(C, C.mesh_a, a->dim, loc_a, a->nnodes, a->nelements, a->positions, a->enlist, false, mass, true);
-  stage_mesh(C, C.mesh_b, b->dim, loc_b, b->nnodes, b->nelements, b->positions, b->enlist,
-             clip && !mixed, mass, true);
-  C.hstat[0] = 0;
-  LSM_HIP(hipMemcpyAsync(C.hstat, bad, sizeof(int), hipMemcpyDeviceToHost, C.stream));
+  stage_meshes(C, *a, loc_a, *b, loc_b, clip && !mixed, mass);
   stage_groups(C, C.mesh_a, ngroups, a_off);
   stage_groups(C, C.mesh_b, ngroups, b_off);
   ph.mark();
@@ -190,11 +185,10 @@ static void run_supermesh(Context& C, const libsupermesh_gpu_mesh* a, const libs
   const bool from_b = ngroups == 0 && C.mesh_a.nelements > 0 && C.mesh_a.nelements * 8 < C.mesh_b.nelements;
   build_bvh(C, from_b ? C.mesh_a : C.mesh_b, from_b ? &C.mesh_b : &C.mesh_a);
   ph.mark();
-  // find_pairs synchronises after reading the candidate count, which also
-  // completes the copy of the flag queued before it
+  // find_pairs waits for the candidate count and the staging flag
   long npairs = from_b ? find_pairs_from_b(C, C.mesh_a, C.mesh_b, finder)
                        : find_pairs(C, C.mesh_a, C.mesh_b, finder, flags & LIBSUPERMESH_GPU_SORTED, true);
-  LSM_REQUIRE(*reinterpret_cast<const int*>(C.hstat) == 0, LIBSUPERMESH_GPU_ERROR_INVALID,
+  LSM_REQUIRE((int)C.hstat[11] != C.stage_serial, LIBSUPERMESH_GPU_ERROR_INVALID,
               "Invalid node: element-node index out of range");
   ph.mark();
   out->nelements_a = a->nelements;

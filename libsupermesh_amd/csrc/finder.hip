@@ -37,21 +37,42 @@ constexpr int kBlock = 256;
 
 // Elements are simplices (LOC = DIM + 1) or, for the candidate finder only,
 // quads / hexahedra (LOC = 2^DIM): those get coordinates, boxes and scale.
+// Two meshes of one element type take one launch, A's blocks first.
+struct StageJob {
+  long ne, nnodes;
+  const double* pos;
+  const int* enl;
+  double *coords, *bbox, *sp, *scale, *planes, *affine;
+};
+struct StageArgs {
+  StageJob job[2];
+  long blocks0;  // blocks of job 0
+  int* bad;      // set to `serial` where a node index is out of range: a flag
+  int serial;    // of an earlier call says nothing, so none has to be cleared
+};
+
 template <int DIM, int LOC>
-__global__ void __launch_bounds__(kBlock)
-k_stage(long ne, long nnodes, const double* __restrict__ pos, const int* __restrict__ enl,
-        double* __restrict__ coords, double* __restrict__ bbox, double* __restrict__ sp,
-        double* __restrict__ scale, double* __restrict__ planes, double* __restrict__ affine,
-        int* __restrict__ bad) {
+__global__ void __launch_bounds__(kBlock) k_stage(StageArgs args) {
   constexpr bool SIMPLEX = LOC == DIM + 1;
-  long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const bool second = (long)blockIdx.x >= args.blocks0;
+  const StageJob& J = args.job[second ? 1 : 0];
+  const long ne = J.ne, nnodes = J.nnodes;
+  const double* __restrict__ pos = J.pos;
+  const int* __restrict__ enl = J.enl;
+  double* __restrict__ coords = J.coords;
+  double* __restrict__ bbox = J.bbox;
+  double* __restrict__ sp = J.sp;
+  double* __restrict__ scale = J.scale;
+  double* __restrict__ planes = J.planes;
+  double* __restrict__ affine = J.affine;
+  long e = ((long)blockIdx.x - (second ? args.blocks0 : 0)) * kBlock + threadIdx.x;
   if (e >= ne) return;
   double c[LOC * DIM];
 #pragma unroll
   for (int j = 0; j < LOC; j++) {
     long v = enl[e * LOC + j];
     if (v < 0 || v >= nnodes) {
-      atomicOr(bad, 1);
+      *args.bad = args.serial;
       v = 0;
     }
 #pragma unroll
@@ -134,11 +155,11 @@ k_stage(long ne, long nnodes, const double* __restrict__ pos, const int* __restr
   }
 }
 
-int* stage_flag(Context& C) { return C.scalars.as<int>(64); }
+int* stage_flag(Context& C) { return C.scalars.as<int>(256) + 36; }
 
-void stage_mesh(Context& C, DevMesh& M, int dim, int loc, long nnodes, long ne,
-                const double* positions, const int* enlist, bool need_planes, bool need_affine,
-                bool defer_check) {
+// Checks the mesh and allocates its arrays.
+static StageJob stage_job(DevMesh& M, int dim, int loc, long nnodes, long ne, const double* positions,
+                          const int* enlist, bool need_planes, bool need_affine) {
   LSM_REQUIRE(dim == 2 || dim == 3, LIBSUPERMESH_GPU_ERROR_INVALID, "Invalid dimension");
   const bool simplex = loc == dim + 1;
   LSM_REQUIRE(simplex || loc == (1 << dim), LIBSUPERMESH_GPU_ERROR_INVALID,
@@ -155,33 +176,63 @@ void stage_mesh(Context& C, DevMesh& M, int dim, int loc, long nnodes, long ne,
   M.nelements = ne;
   M.ngroups = 0;
   M.enlist_dev = enlist;
-  double* coords = M.coords.as<double>((size_t)ne * loc * dim);
-  double* bbox = M.bbox.as<double>((size_t)ne * 2 * dim);
-  double* sp = M.meas_sp.as<double>((size_t)ne);
-  double* scale = M.scale.as<double>((size_t)ne);
-  double* planes = need_planes && dim == 3 ? M.planes.as<double>((size_t)ne * 16) : nullptr;
-  double* affine = need_affine ? M.affine.as<double>((size_t)ne * (dim + dim * dim)) : nullptr;
-  int* bad = stage_flag(C);
-  if (!defer_check) LSM_HIP(hipMemsetAsync(bad, 0, sizeof(int), C.stream));
-  if (ne > 0) {
-#define LSM_STAGE(D, L)                                                                         \
-  hipLaunchKernelGGL((k_stage<D, L>), dim3(grid_for(ne, kBlock)), dim3(kBlock), 0, C.stream, ne,  \
-                     nnodes, positions, enlist, coords, bbox, sp, scale, planes, affine, bad)
-    if (dim == 2) {
-      if (simplex) LSM_STAGE(2, 3);
-      else LSM_STAGE(2, 4);
-    } else {
-      if (simplex) LSM_STAGE(3, 4);
-      else LSM_STAGE(3, 8);
-    }
-#undef LSM_STAGE
-    LSM_HIP(hipGetLastError());
+  StageJob J;
+  J.ne = ne;
+  J.nnodes = nnodes;
+  J.pos = positions;
+  J.enl = enlist;
+  J.coords = M.coords.as<double>((size_t)ne * loc * dim);
+  J.bbox = M.bbox.as<double>((size_t)ne * 2 * dim);
+  J.sp = M.meas_sp.as<double>((size_t)ne);
+  J.scale = M.scale.as<double>((size_t)ne);
+  J.planes = need_planes && dim == 3 ? M.planes.as<double>((size_t)ne * 16) : nullptr;
+  J.affine = need_affine ? M.affine.as<double>((size_t)ne * (dim + dim * dim)) : nullptr;
+  return J;
+}
+
+static void launch_stage(Context& C, int dim, int loc, const StageJob& a, const StageJob* b) {
+  StageArgs args = {};
+  args.job[0] = a;
+  if (b) args.job[1] = *b;
+  args.blocks0 = (a.ne + kBlock - 1) / kBlock;
+  args.bad = stage_flag(C);
+  args.serial = C.stage_serial;
+  const long blocks = args.blocks0 + (b ? (b->ne + kBlock - 1) / kBlock : 0);
+  if (blocks == 0) return;
+  const dim3 grid((unsigned)blocks), block(kBlock);
+  if (dim == 2) {
+    if (loc == 3) hipLaunchKernelGGL((k_stage<2, 3>), grid, block, 0, C.stream, args);
+    else hipLaunchKernelGGL((k_stage<2, 4>), grid, block, 0, C.stream, args);
+  } else {
+    if (loc == 4) hipLaunchKernelGGL((k_stage<3, 4>), grid, block, 0, C.stream, args);
+    else hipLaunchKernelGGL((k_stage<3, 8>), grid, block, 0, C.stream, args);
   }
-  if (defer_check) return;
+  LSM_HIP(hipGetLastError());
+}
+
+void stage_mesh(Context& C, DevMesh& M, int dim, int loc, long nnodes, long ne, const double* positions,
+                const int* enlist, bool need_planes, bool need_affine) {
+  const StageJob J = stage_job(M, dim, loc, nnodes, ne, positions, enlist, need_planes, need_affine);
+  C.stage_serial++;
+  launch_stage(C, dim, loc, J, nullptr);
   int hbad = 0;
-  LSM_HIP(hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, C.stream));
+  LSM_HIP(hipMemcpyAsync(&hbad, stage_flag(C), sizeof(int), hipMemcpyDeviceToHost, C.stream));
   LSM_HIP(hipStreamSynchronize(C.stream));
-  LSM_REQUIRE(hbad == 0, LIBSUPERMESH_GPU_ERROR_INVALID, "Invalid node: element-node index out of range");
+  LSM_REQUIRE(hbad != C.stage_serial, LIBSUPERMESH_GPU_ERROR_INVALID,
+              "Invalid node: element-node index out of range");
+}
+
+void stage_meshes(Context& C, const libsupermesh_gpu_mesh& a, int loc_a, const libsupermesh_gpu_mesh& b, int loc_b,
+                  bool planes_b, bool affine) {
+  const StageJob A = stage_job(C.mesh_a, a.dim, loc_a, a.nnodes, a.nelements, a.positions, a.enlist, false, affine);
+  const StageJob B = stage_job(C.mesh_b, b.dim, loc_b, b.nnodes, b.nelements, b.positions, b.enlist, planes_b, affine);
+  C.stage_serial++;
+  if (loc_a == loc_b) {
+    launch_stage(C, a.dim, loc_a, A, &B);
+  } else {
+    launch_stage(C, a.dim, loc_a, A, nullptr);
+    launch_stage(C, b.dim, loc_b, B, nullptr);
+  }
 }
 
 __global__ void __launch_bounds__(kBlock)
@@ -213,9 +264,9 @@ void stage_groups(Context& C, DevMesh& M, long ngroups, const long* offsets) {
 // ---------------------------------------------------------------------------
 
 // Bounds of the block's values b (minima, then maxima), in every lane.
-template <int DIM>
+template <int DIM, int BLOCK = kBlock>
 __device__ __forceinline__ void block_bounds(double* b) {
-  __shared__ double red[kBlock / 64][2 * DIM];
+  __shared__ double red[BLOCK / 64][2 * DIM];
   for (int o = 32; o > 0; o >>= 1) {
 #pragma unroll
     for (int d = 0; d < DIM; d++) {
@@ -229,7 +280,7 @@ __device__ __forceinline__ void block_bounds(double* b) {
   }
   __syncthreads();
 #pragma unroll
-  for (int w = 0; w < kBlock / 64; w++) {
+  for (int w = 0; w < BLOCK / 64; w++) {
 #pragma unroll
     for (int d = 0; d < DIM; d++) {
       b[d] = fmin_f(b[d], red[w][d]);
@@ -237,6 +288,9 @@ __device__ __forceinline__ void block_bounds(double* b) {
     }
   }
 }
+
+// The search's words: [0] longest row, [1] tasks.
+static long* search_words(Context& C) { return C.scalars.as<long>(128) + 16; }
 
 // A sort of one mesh's elements by Morton code, or of two meshes' (the
 // hierarchy's and the queries') in the same launches.
@@ -272,11 +326,13 @@ struct OrderJob {
 
 struct OrderArgs {
   OrderJob job[2];
+  long* words;        // the search's [0] longest row, [1] tasks: cleared here
 };
 
 template <int DIM>
 __global__ void __launch_bounds__(kBlock) k_center_bounds(OrderArgs args) {
   const OrderJob& J = args.job[blockIdx.y];
+  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 2) args.words[threadIdx.x] = 0;
   for (long k = (long)blockIdx.x * kBlock + threadIdx.x; k < (long)kSortPasses * J.groups * kDigits;
        k += (long)gridDim.x * kBlock)
     J.sums[k] = 0;
@@ -410,6 +466,22 @@ __global__ void __launch_bounds__(kBlock) k_sort_counts(OrderArgs args, int pass
   write_counts(J, tile, pass, hist[threadIdx.x]);
 }
 
+// Rank of this lane's key among the wave's keys of the same digit d, those of
+// earlier calls first; `counts`, the wave's, go on from call to call.
+__device__ __forceinline__ int rank_digit(unsigned d, bool live, unsigned* counts) {
+  const int lane = threadIdx.x & 63;
+  unsigned long long m = __ballot(live);
+#pragma unroll
+  for (int b = 0; b < 8; b++) {
+    const unsigned long long v = __ballot((d >> b) & 1u);
+    m &= (d >> b) & 1u ? v : ~v;
+  }
+  const int lower = __builtin_popcountll(m & ((1ULL << lane) - 1));
+  unsigned old = 0;
+  if (live && lower == 0) old = atomicAdd(counts + d, (unsigned)__builtin_popcountll(m));
+  return (int)__shfl(old, live ? __builtin_ctzll(m) : lane, 64) + lower;
+}
+
 // Moves a tile's keys and element ids to their places for one digit.  A wave
 // ranks 64 keys at a time among its own (the lanes of equal digit by eight
 // ballots), the tile is put in digit order in LDS, and neighbouring lanes
@@ -457,18 +529,7 @@ __global__ void __launch_bounds__(kBlock) k_sort_move(OrderArgs args) {
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < kSortItems; i++) {
-    const bool live = (wave * kSortItems + i) * 64 + lane < n;
-    const unsigned d = (key[i] >> (8 * PASS)) & (kDigits - 1);
-    unsigned long long m = __ballot(live);
-#pragma unroll
-    for (int b = 0; b < 8; b++) {
-      const unsigned long long v = __ballot((d >> b) & 1u);
-      m &= (d >> b) & 1u ? v : ~v;
-    }
-    const int lower = __builtin_popcountll(m & ((1ULL << lane) - 1));
-    unsigned old = 0;
-    if (live && lower == 0) old = atomicAdd(&hist[wave][d], (unsigned)__builtin_popcountll(m));
-    rank[i] = (int)__shfl(old, live ? __builtin_ctzll(m) : lane, 64) + lower;
+    rank[i] = rank_digit((key[i] >> (8 * PASS)) & (kDigits - 1), (wave * kSortItems + i) * 64 + lane < n, hist[wave]);
   }
   __syncthreads();
   unsigned mine = 0;  // digit t's keys in this tile; each wave's first place among them
@@ -525,12 +586,267 @@ __global__ void __launch_bounds__(kBlock) k_sort_move(OrderArgs args) {
 // reads more counts than keys.
 constexpr long kOrderMax = 1L << 23;
 
+// ---------------------------------------------------------------------------
+// Implicit hierarchy
+// ---------------------------------------------------------------------------
+
+struct LevelInfo {
+  int levels;
+  long count[32];
+  long offset[32];
+};
+
+static LevelInfo level_info(const DevBVH& H) {
+  LevelInfo info;
+  info.levels = H.levels;
+  for (int l = 0; l < 32; l++) {
+    info.count[l] = l < H.levels ? H.count[l] : 0;
+    info.offset[l] = l < H.levels ? H.offset[l] : 0;
+  }
+  return info;
+}
+
+// A node's box [lo_0..lo_{dim-1}, hi_0..hi_{dim-1}] and, in batches, its mesh
+// range.
+template <int DIM>
+struct NodeBox {
+  double b[2 * DIM];
+  int glo, ghi;
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int d = 0; d < DIM; d++) {
+      b[d] = __builtin_inf();
+      b[DIM + d] = -__builtin_inf();
+    }
+    glo = 0x7fffffff;
+    ghi = -1;
+  }
+  __device__ __forceinline__ void element(long e, long ne, const double* __restrict__ bbox,
+                                          const int* __restrict__ group) {
+#pragma unroll
+    for (int k = 0; k < 2 * DIM; k++) b[k] = bbox[(long)k * ne + e];
+    if (group) glo = ghi = group[e];
+  }
+  __device__ __forceinline__ void store(const LevelInfo& info, int l, long node, double* __restrict__ boxes,
+                                        int* __restrict__ granges) const {
+    if (l >= info.levels || node >= info.count[l]) return;
+    const long o = info.offset[l] + node;
+#pragma unroll
+    for (int k = 0; k < 2 * DIM; k++) boxes[o * 2 * DIM + k] = b[k];
+    if (granges) {
+      granges[2 * o] = glo;
+      granges[2 * o + 1] = ghi;
+    }
+  }
+  __device__ __forceinline__ void add(const NodeBox& x) {
+#pragma unroll
+    for (int d = 0; d < DIM; d++) {
+      b[d] = __builtin_fmin(b[d], x.b[d]);
+      b[DIM + d] = __builtin_fmax(b[DIM + d], x.b[DIM + d]);
+    }
+    glo = std::min(glo, x.glo);
+    ghi = std::max(ghi, x.ghi);
+  }
+  // the union with the lanes whose number differs in bit o
+  __device__ __forceinline__ void join(int o) {
+    NodeBox x;
+#pragma unroll
+    for (int k = 0; k < 2 * DIM; k++) x.b[k] = __shfl_xor(b[k], o, 64);
+    x.glo = __shfl_xor(glo, o, 64);
+    x.ghi = __shfl_xor(ghi, o, 64);
+    add(x);
+  }
+};
+
+// Boxes of the three levels above `l0`, and of the elements themselves in
+// sorted order if l0 is 0: a wave's 64 nodes have eight parents and one
+// grandparent, which come from shuffles, and the block's 512 one node above
+// those.  (A launch a level took 5 us each; the nodes were read again.)
+constexpr int kLevelBlock = kFanout * kFanout * kFanout;
+template <int DIM>
+__global__ void __launch_bounds__(kLevelBlock)
+k_build_levels(LevelInfo info, int l0, long ne, const double* __restrict__ bbox, const int* __restrict__ perm,
+               const int* __restrict__ group, double* __restrict__ boxes, int* __restrict__ granges) {
+  __shared__ NodeBox<DIM> top[kFanout];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const long i = (long)blockIdx.x * kLevelBlock + threadIdx.x;
+  NodeBox<DIM> x;
+  x.clear();
+  if (i < info.count[l0]) {
+    if (l0 == 0) {
+      x.element(perm[i], ne, bbox, group);
+      x.store(info, 0, i, boxes, granges);
+    } else {
+      const long o = info.offset[l0] + i;
+#pragma unroll
+      for (int k = 0; k < 2 * DIM; k++) x.b[k] = boxes[o * 2 * DIM + k];
+      if (granges) {
+        x.glo = granges[2 * o];
+        x.ghi = granges[2 * o + 1];
+      }
+    }
+  }
+  for (int o = 1; o < kFanout; o <<= 1) x.join(o);
+  if ((lane & 7) == 0) x.store(info, l0 + 1, i / kFanout, boxes, granges);
+  for (int o = kFanout; o < 64; o <<= 1) x.join(o);
+  if (lane == 0) {
+    x.store(info, l0 + 2, i / (kFanout * kFanout), boxes, granges);
+    top[wave] = x;
+  }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  for (int w = 1; w < kFanout; w++) x.add(top[w]);
+  x.store(info, l0 + 3, blockIdx.x, boxes, granges);
+}
+
+// Small meshes, a block each: order and, for the first, the hierarchy in one
+// launch (nine to eleven otherwise, each a few microseconds of latency with
+// next to no work).  A thread holds up to kSmallItems keys through the four
+// passes, exchanged in LDS; the 64 boxes of a wave give two levels by
+// shuffles, the at most 128 boxes of the second level the rest.
+constexpr int kSmallBlock = 1024;
+constexpr int kSmallItems = 8;
+constexpr long kSmallMax = (long)kSmallBlock * kSmallItems;
+template <int DIM>
+__global__ void __launch_bounds__(kSmallBlock)
+k_small_order(OrderArgs args, LevelInfo info, double* __restrict__ boxes, int* __restrict__ granges) {
+  constexpr int kWaves = kSmallBlock / 64;
+  constexpr int kTops = (int)(kSmallMax / (kFanout * kFanout));
+  struct Sort {
+    unsigned hist[kWaves][kDigits], wsum[kDigits / 64];
+    uint32_t key[kSmallMax];
+    int val[kSmallMax];
+  };
+  __shared__ union {
+    Sort sort;
+    NodeBox<DIM> top[kTops];
+  } mem;
+  const OrderJob& J = args.job[blockIdx.x];
+  if (blockIdx.x == 0 && threadIdx.x < 2) args.words[threadIdx.x] = 0;
+  const int n = (int)J.ne, t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  if (n == 0) return;
+  const int items = (n + kSmallBlock - 1) / kSmallBlock;
+  double b[2 * DIM];
+#pragma unroll
+  for (int d = 0; d < DIM; d++) {
+    b[d] = __builtin_inf();
+    b[DIM + d] = -__builtin_inf();
+  }
+  for (int e = t; e < n; e += kSmallBlock) {
+#pragma unroll
+    for (int d = 0; d < DIM; d++) {
+      const double c = 0.5 * (J.bbox[d * n + e] + J.bbox[(DIM + d) * n + e]);
+      b[d] = fmin_f(b[d], c);
+      b[DIM + d] = fmax_f(b[DIM + d], c);
+    }
+  }
+  block_bounds<DIM, kSmallBlock>(b);
+  uint32_t key[kSmallItems];
+  int val[kSmallItems], rank[kSmallItems];
+  auto at = [&](int i) { return (wave * items + i) * 64 + lane; };  // this lane's i-th place
+#pragma unroll
+  for (int i = 0; i < kSmallItems; i++) {
+    if (i >= items) break;
+    val[i] = at(i);
+    key[i] = at(i) < n ? morton_key<DIM>(J, b, at(i)) : 0;
+  }
+  for (int pass = 0; pass < kSortPasses; pass++) {
+    const int shift = 8 * pass;
+#pragma unroll
+    for (int k = 0; k < kWaves * kDigits / kSmallBlock; k++) (&mem.sort.hist[0][0])[k * kSmallBlock + t] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kSmallItems; i++) {
+      if (i >= items) break;
+      rank[i] = rank_digit((key[i] >> shift) & (kDigits - 1), at(i) < n, mem.sort.hist[wave]);
+    }
+    __syncthreads();
+    unsigned mine = 0, sum = 0;
+    if (t < kDigits) {
+#pragma unroll
+      for (int w = 0; w < kWaves; w++) {
+        const unsigned c = mem.sort.hist[w][t];
+        mem.sort.hist[w][t] = mine;
+        mine += c;
+      }
+      sum = mine;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const unsigned x = __shfl_up(sum, o, 64);
+        if (lane >= o) sum += x;
+      }
+      if (lane == 63) mem.sort.wsum[wave] = sum;
+    }
+    __syncthreads();
+    if (t < kDigits) {
+      for (int w = 0; w < wave; w++) sum += mem.sort.wsum[w];
+#pragma unroll
+      for (int w = 0; w < kWaves; w++) mem.sort.hist[w][t] += sum - mine;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kSmallItems; i++) {
+      if (i >= items) break;
+      if (at(i) < n) {
+        const unsigned o = mem.sort.hist[wave][(key[i] >> shift) & (kDigits - 1)] + (unsigned)rank[i];
+        mem.sort.key[o] = key[i];
+        mem.sort.val[o] = val[i];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kSmallItems; i++) {
+      if (i >= items) break;
+      if (at(i) < n) {
+        key[i] = mem.sort.key[at(i)];
+        val[i] = mem.sort.val[at(i)];
+      }
+    }
+  }
+  __syncthreads();
+  const bool build = blockIdx.x == 0 && boxes != nullptr;
+  NodeBox<DIM> x;
+#pragma unroll
+  for (int i = 0; i < kSmallItems; i++) {
+    if (i >= items) break;
+    const int p = at(i);
+    if (p < n) J.perm[p] = val[i];
+    if (!build) continue;
+    x.clear();
+    if (p < n) {
+      x.element(val[i], n, J.bbox, J.group);
+      x.store(info, 0, p, boxes, granges);
+    }
+    for (int o = 1; o < kFanout; o <<= 1) x.join(o);
+    if ((lane & 7) == 0) x.store(info, 1, p / kFanout, boxes, granges);
+    for (int o = kFanout; o < 64; o <<= 1) x.join(o);
+    if (lane == 0) {
+      x.store(info, 2, p / (kFanout * kFanout), boxes, granges);
+      mem.top[wave * items + i] = x;
+    }
+  }
+  if (!build) return;
+  __syncthreads();
+  if (t >= kTops) return;  // whole waves
+  x.clear();
+  if (t < kWaves * items) x = mem.top[t];
+  for (int o = 1; o < kFanout; o <<= 1) x.join(o);
+  if ((lane & 7) == 0) x.store(info, 3, t / kFanout, boxes, granges);
+  for (int o = kFanout; o < 64; o <<= 1) x.join(o);
+  if (lane == 0) x.store(info, 4, wave, boxes, granges);
+  if (t != 0 || info.levels <= 5) return;
+  for (int k = 64; k < kWaves * items; k++) x.add(mem.top[k]);
+  x.store(info, 5, 0, boxes, granges);
+}
+
 // Sorts the elements of M[0], and of M[1] if it is given, by Morton code:
 // perm[j] gets the permutation.
-static void morton_order(Context& C, int n, const DevMesh* const* M, DevBuf* const* perm) {
+// With H (set up but for its boxes), the boxes of its levels over M[0] too.
+static void morton_order(Context& C, int n, const DevMesh* const* M, DevBuf* const* perm, const DevBVH* H) {
   OrderArgs args = {};
+  args.words = search_words(C);
   size_t total = 0, words = 0;
-  bool large = false;
+  bool large = false, small = true;
   for (int j = 0; j < n; j++) {
     OrderJob& J = args.job[j];
     J.ne = M[j]->nelements;
@@ -545,6 +861,24 @@ static void morton_order(Context& C, int n, const DevMesh* const* M, DevBuf* con
     total += (size_t)J.ne;
     words += (size_t)(J.tiles + kSortPasses * J.groups) * kDigits;
     large = large || J.ne > kOrderMax;
+    small = small && J.ne <= kSmallMax;
+  }
+  const bool flat = M[0]->dim == 2;
+  const dim3 block(kBlock);
+  LevelInfo info = {};
+  double* boxes = nullptr;
+  int* granges = nullptr;
+  if (H) {
+    info = level_info(*H);
+    boxes = static_cast<double*>(H->boxes.ptr);
+    granges = H->grouped ? static_cast<int*>(H->granges.ptr) : nullptr;
+  }
+  if (small) {
+    const dim3 grid((unsigned)n), threads(kSmallBlock);
+    if (flat) hipLaunchKernelGGL(k_small_order<2>, grid, threads, 0, C.stream, args, info, boxes, granges);
+    else hipLaunchKernelGGL(k_small_order<3>, grid, threads, 0, C.stream, args, info, boxes, granges);
+    LSM_HIP(hipGetLastError());
+    return;
   }
   double* part = C.partials.as<double>((size_t)n * kBoundParts * 6);
   uint32_t* keys[2] = {C.keys.as<uint32_t>(total), C.keys_alt.as<uint32_t>(total)};
@@ -567,9 +901,8 @@ static void morton_order(Context& C, int n, const DevMesh* const* M, DevBuf* con
     J.sums = table + (size_t)J.tiles * kDigits;
     table += (size_t)(J.tiles + kSortPasses * J.groups) * kDigits;
   }
-  const dim3 block(kBlock), parts((unsigned)std::max(1, std::max(args.job[0].nparts, args.job[1].nparts)), (unsigned)n);
+  const dim3 parts((unsigned)std::max(1, std::max(args.job[0].nparts, args.job[1].nparts)), (unsigned)n);
   const dim3 tiles((unsigned)std::max(1, args.job[0].tiles + args.job[1].tiles));
-  const bool flat = M[0]->dim == 2;
   if (flat) hipLaunchKernelGGL(k_center_bounds<2>, parts, block, 0, C.stream, args);
   else hipLaunchKernelGGL(k_center_bounds<3>, parts, block, 0, C.stream, args);
   if (large) {
@@ -586,126 +919,24 @@ static void morton_order(Context& C, int n, const DevMesh* const* M, DevBuf* con
       LSM_HIP(rocprim::radix_sort_pairs(tmp, bytes, J.keys[0], J.keys[1], J.vals[0], J.perm, (size_t)J.ne, 0u, 32u,
                                         C.stream));
     }
-    return;
+  } else {
+    if (flat) hipLaunchKernelGGL((k_morton<2, false>), tiles, block, 0, C.stream, args);
+    else hipLaunchKernelGGL((k_morton<3, false>), tiles, block, 0, C.stream, args);
+    hipLaunchKernelGGL(k_sort_move<0>, tiles, block, 0, C.stream, args);
+    hipLaunchKernelGGL(k_sort_counts, tiles, block, 0, C.stream, args, 1);
+    hipLaunchKernelGGL(k_sort_move<1>, tiles, block, 0, C.stream, args);
+    hipLaunchKernelGGL(k_sort_counts, tiles, block, 0, C.stream, args, 2);
+    hipLaunchKernelGGL(k_sort_move<2>, tiles, block, 0, C.stream, args);
+    hipLaunchKernelGGL(k_sort_counts, tiles, block, 0, C.stream, args, 3);
+    hipLaunchKernelGGL(k_sort_move<3>, tiles, block, 0, C.stream, args);
   }
-  if (flat) hipLaunchKernelGGL((k_morton<2, false>), tiles, block, 0, C.stream, args);
-  else hipLaunchKernelGGL((k_morton<3, false>), tiles, block, 0, C.stream, args);
-  hipLaunchKernelGGL(k_sort_move<0>, tiles, block, 0, C.stream, args);
-  hipLaunchKernelGGL(k_sort_counts, tiles, block, 0, C.stream, args, 1);
-  hipLaunchKernelGGL(k_sort_move<1>, tiles, block, 0, C.stream, args);
-  hipLaunchKernelGGL(k_sort_counts, tiles, block, 0, C.stream, args, 2);
-  hipLaunchKernelGGL(k_sort_move<2>, tiles, block, 0, C.stream, args);
-  hipLaunchKernelGGL(k_sort_counts, tiles, block, 0, C.stream, args, 3);
-  hipLaunchKernelGGL(k_sort_move<3>, tiles, block, 0, C.stream, args);
+  for (int l = 0; H && (l == 0 || l + 1 < H->levels); l += 3) {
+    const dim3 grid(grid_for(H->count[l], kLevelBlock)), threads(kLevelBlock);
+    const OrderJob& J = args.job[0];
+    if (flat) hipLaunchKernelGGL(k_build_levels<2>, grid, threads, 0, C.stream, info, l, J.ne, J.bbox, J.perm, J.group, boxes, granges);
+    else hipLaunchKernelGGL(k_build_levels<3>, grid, threads, 0, C.stream, info, l, J.ne, J.bbox, J.perm, J.group, boxes, granges);
+  }
   LSM_HIP(hipGetLastError());
-}
-
-// ---------------------------------------------------------------------------
-// Implicit hierarchy
-// ---------------------------------------------------------------------------
-
-struct LevelInfo {
-  int levels;
-  long count[32];
-  long offset[32];
-};
-
-// Boxes (node-major: [lo_0..lo_{dim-1}, hi_0..hi_{dim-1}]) and, in batches,
-// mesh ranges of the three levels above `l0`, and of the elements themselves
-// in sorted order if l0 is 0: a wave's 64 nodes have eight parents and one
-// grandparent, which come from shuffles, and the block's 512 one node above
-// those.  (A launch a level took 5 us each; the nodes were read again.)
-constexpr int kLevelBlock = kFanout * kFanout * kFanout;
-template <int DIM>
-__global__ void __launch_bounds__(kLevelBlock)
-k_build_levels(LevelInfo info, int l0, long ne, const double* __restrict__ bbox, const int* __restrict__ perm,
-               const int* __restrict__ group, double* __restrict__ boxes, int* __restrict__ granges) {
-  __shared__ double top[kFanout][2 * DIM];
-  __shared__ int topg[kFanout][2];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const long i = (long)blockIdx.x * kLevelBlock + threadIdx.x;
-  double b[2 * DIM];
-#pragma unroll
-  for (int d = 0; d < DIM; d++) {
-    b[d] = __builtin_inf();
-    b[DIM + d] = -__builtin_inf();
-  }
-  int glo = 0x7fffffff, ghi = -1;
-  auto store = [&](int l, long node) {
-    if (l >= info.levels || node >= info.count[l]) return;
-    const long o = info.offset[l] + node;
-#pragma unroll
-    for (int k = 0; k < 2 * DIM; k++) boxes[o * 2 * DIM + k] = b[k];
-    if (granges) {
-      granges[2 * o] = glo;
-      granges[2 * o + 1] = ghi;
-    }
-  };
-  auto join = [&](int o) {
-#pragma unroll
-    for (int d = 0; d < DIM; d++) {
-      b[d] = __builtin_fmin(b[d], __shfl_xor(b[d], o, 64));
-      b[DIM + d] = __builtin_fmax(b[DIM + d], __shfl_xor(b[DIM + d], o, 64));
-    }
-    if (granges) {
-      glo = std::min(glo, __shfl_xor(glo, o, 64));
-      ghi = std::max(ghi, __shfl_xor(ghi, o, 64));
-    }
-  };
-  if (i < info.count[l0]) {
-    if (l0 == 0) {
-      const long e = perm[i];
-#pragma unroll
-      for (int k = 0; k < 2 * DIM; k++) b[k] = bbox[(long)k * ne + e];
-      if (granges) glo = ghi = group[e];
-      store(0, i);
-    } else {
-      const long o = info.offset[l0] + i;
-#pragma unroll
-      for (int k = 0; k < 2 * DIM; k++) b[k] = boxes[o * 2 * DIM + k];
-      if (granges) {
-        glo = granges[2 * o];
-        ghi = granges[2 * o + 1];
-      }
-    }
-  }
-  join(1);
-  join(2);
-  join(4);
-  if ((lane & 7) == 0) store(l0 + 1, i / kFanout);
-  join(8);
-  join(16);
-  join(32);
-  if (lane == 0) {
-    store(l0 + 2, i / (kFanout * kFanout));
-#pragma unroll
-    for (int k = 0; k < 2 * DIM; k++) top[wave][k] = b[k];
-    topg[wave][0] = glo;
-    topg[wave][1] = ghi;
-  }
-  __syncthreads();
-  if (threadIdx.x != 0) return;
-#pragma unroll
-  for (int w = 1; w < kFanout; w++) {
-#pragma unroll
-    for (int d = 0; d < DIM; d++) {
-      b[d] = __builtin_fmin(b[d], top[w][d]);
-      b[DIM + d] = __builtin_fmax(b[DIM + d], top[w][DIM + d]);
-    }
-    glo = std::min(glo, topg[w][0]);
-    ghi = std::max(ghi, topg[w][1]);
-  }
-  store(l0 + 3, blockIdx.x);
-}
-
-static LevelInfo level_info(const DevBVH& H) {
-  LevelInfo info;
-  info.levels = H.levels;
-  for (int l = 0; l < 32; l++) {
-    info.count[l] = l < H.levels ? H.count[l] : 0;
-    info.offset[l] = l < H.levels ? H.offset[l] : 0;
-  }
-  return info;
 }
 
 void build_bvh(Context& C, const DevMesh& B, const DevMesh* A) {
@@ -716,9 +947,6 @@ void build_bvh(Context& C, const DevMesh& B, const DevMesh* A) {
     H.levels = 0;
     return;
   }
-  const DevMesh* meshes[2] = {&B, A};
-  DevBuf* orders[2] = {&H.perm, &C.qperm};
-  morton_order(C, A ? 2 : 1, meshes, orders);
   long n = H.n;
   int L = 0;
   long total = 0;
@@ -733,20 +961,13 @@ void build_bvh(Context& C, const DevMesh& B, const DevMesh* A) {
   }
   H.levels = L;
   H.total = total;
-  // a walk reads whole groups of children, past the last node too
-  double* boxes = H.boxes.as<double>((size_t)(total + kFanout) * 2 * B.dim);
-  const double* bbox = static_cast<const double*>(B.bbox.ptr);
-  const int* perm = static_cast<const int*>(H.perm.ptr);
   H.grouped = B.ngroups > 0;
-  const int* group = H.grouped ? static_cast<const int*>(B.group.ptr) : nullptr;
-  int* gr = H.grouped ? H.granges.as<int>((size_t)(total + kFanout) * 2) : nullptr;
-  const LevelInfo info = level_info(H);
-  for (int l = 0; l == 0 || l + 1 < L; l += 3) {
-    const dim3 grid(grid_for(H.count[l], kLevelBlock)), block(kLevelBlock);
-    if (B.dim == 2) hipLaunchKernelGGL(k_build_levels<2>, grid, block, 0, C.stream, info, l, H.n, bbox, perm, group, boxes, gr);
-    else hipLaunchKernelGGL(k_build_levels<3>, grid, block, 0, C.stream, info, l, H.n, bbox, perm, group, boxes, gr);
-  }
-  LSM_HIP(hipGetLastError());
+  // a walk reads whole groups of children, past the last node too
+  H.boxes.as<double>((size_t)(total + kFanout) * 2 * B.dim);
+  if (H.grouped) H.granges.as<int>((size_t)(total + kFanout) * 2);
+  const DevMesh* meshes[2] = {&B, A};
+  DevBuf* orders[2] = {&H.perm, &C.qperm};
+  morton_order(C, A ? 2 : 1, meshes, orders, &H);
 }
 
 // ---------------------------------------------------------------------------
@@ -1129,13 +1350,60 @@ k_sort_rows(long na, const long* __restrict__ indptr, int* __restrict__ indices)
 }
 
 // The words that the host waits for, in its own memory: [0] the pairs, [1]
-// the longest row, [2] the tasks.
-__global__ void k_publish(const long* __restrict__ npairs, const long* __restrict__ maxrow,
-                          const unsigned* __restrict__ ntasks, long* __restrict__ host) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    host[0] = *npairs;
-    host[1] = *maxrow;
-    host[2] = ntasks ? (long)*ntasks : 0L;
+// the longest row, [2] the tasks, [3] the staging flag.
+__device__ __forceinline__ void publish(long npairs, const long* maxrow, const unsigned* ntasks, const int* bad,
+                                        long* host) {
+  host[0] = npairs;
+  host[1] = *maxrow;
+  host[2] = ntasks ? (long)*ntasks : 0L;
+  host[3] = *bad;
+}
+
+__global__ void k_publish(long na, long* __restrict__ indptr, const long* __restrict__ maxrow,
+                          const unsigned* __restrict__ ntasks, const int* __restrict__ bad, long* __restrict__ host) {
+  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+  indptr[0] = 0;
+  publish(indptr[na], maxrow, ntasks, bad, host);
+}
+
+// Row offsets of up to kScanMax rows, and the host's words, in one launch of
+// one block (three launches with the library's scan).
+constexpr int kScanBlock = 1024;
+constexpr int kScanItems = 16;
+constexpr long kScanMax = (long)kScanBlock * kScanItems;
+__global__ void __launch_bounds__(kScanBlock)
+k_scan_rows(int na, const long* __restrict__ row_count, long* __restrict__ indptr, const long* __restrict__ maxrow,
+            const unsigned* __restrict__ ntasks, const int* __restrict__ bad, long* __restrict__ host) {
+  __shared__ long wsum[kScanBlock / 64];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int items = (na + kScanBlock - 1) / kScanBlock;
+  long n[kScanItems], run = 0;
+#pragma unroll
+  for (int i = 0; i < kScanItems; i++) {
+    if (i >= items) break;
+    const int k = t * items + i;
+    n[i] = k < na ? row_count[k] : 0;
+    run += n[i];
+  }
+  long sum = run;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const long x = __shfl_up(sum, o, 64);
+    if (lane >= o) sum += x;
+  }
+  if (lane == 63) wsum[wave] = sum;
+  __syncthreads();
+  for (int w = 0; w < wave; w++) sum += wsum[w];
+  sum -= run;
+#pragma unroll
+  for (int i = 0; i < kScanItems; i++) {
+    if (i >= items) break;
+    const int k = t * items + i;
+    if (k >= na) break;
+    if (k == 0) indptr[0] = 0;
+    sum += n[i];
+    indptr[k + 1] = sum;
+    if (k == na - 1) publish(sum, maxrow, ntasks, bad, host);
   }
 }
 
@@ -1144,10 +1412,13 @@ __global__ void k_publish(const long* __restrict__ npairs, const long* __restric
 // node on an idle card, so a search with few query waves is cut until the
 // card is full of tasks: nodes of 8^level elements.  In a batch, where a mesh
 // of a few elements may face one of tens of thousands, always to 512 elements.
+// A hierarchy of at most 64 elements is walked in less time than the two
+// launches that cut it take.
 static int task_level(const LevelInfo& info, long waves, bool grouped) {
   const int top = info.levels - 1;
   int level = waves >= 8192 ? top : (waves >= 2048 ? 3 : (waves >= 256 ? 2 : 1));
   if (grouped && level > 3) level = 3;
+  if (top <= 2) level = top;
   return level < top ? level : top;
 }
 
@@ -1155,8 +1426,11 @@ long find_pairs(Context& C, const DevMesh& A, const DevMesh& B, int finder, int 
   long na = A.nelements;
   long* row_count = C.row_count.as<long>(na + 1);
   long* indptr = C.indptr.as<long>(na + 1);
-  LSM_HIP(hipMemsetAsync(indptr, 0, sizeof(long) * (na + 1), C.stream));
+  volatile long* host = C.hstat + 8;
   if (na == 0 || B.nelements == 0) {
+    host[3] = 0;
+    LSM_HIP(hipMemsetAsync(indptr, 0, sizeof(long) * (na + 1), C.stream));
+    LSM_HIP(hipMemcpyAsync(C.hstat + 11, stage_flag(C), sizeof(int), hipMemcpyDeviceToHost, C.stream));
     LSM_HIP(hipStreamSynchronize(C.stream));
     return 0;
   }
@@ -1165,7 +1439,7 @@ long find_pairs(Context& C, const DevMesh& A, const DevMesh& B, int finder, int 
   if (!ordered) {
     const DevMesh* mesh = &A;
     DevBuf* order = &C.qperm;
-    morton_order(C, 1, &mesh, &order);
+    morton_order(C, 1, &mesh, &order, nullptr);
   }
   LSM_REQUIRE((A.ngroups > 0) == H.grouped && (!H.grouped || A.ngroups == B.ngroups),
               LIBSUPERMESH_GPU_ERROR_INVALID, "batches of A and B hold different mesh counts");
@@ -1210,13 +1484,11 @@ long find_pairs(Context& C, const DevMesh& A, const DevMesh& B, int finder, int 
 #define LSM_TASKS(D, CL, G) k_search_tasks<D, CL, G>
 #define LSM_COUNT(D, CL, G) k_search<D, CL, G, false>
 #define LSM_FILL(D, CL, G) k_search<D, CL, G, true>
-  long* words = C.scalars.as<long>(64) + 16;  // [0] longest row, [1] tasks
+  long* words = search_words(C);  // cleared by the order's first kernel
   s.maxrow = words;
-  volatile long* host = C.hstat + 8;
   dim3 grid = wave_grid;
   long room = 16 * waves + 16384;
   while (true) {
-    hipLaunchKernelGGL(k_clear_words, dim3(1), dim3(64), 0, C.stream, 2, words);
     if (split) {
       s.cap = (unsigned)room;
       int2* tasks = C.ftasks.as<int2>(room);
@@ -1234,19 +1506,26 @@ long find_pairs(Context& C, const DevMesh& A, const DevMesh& B, int finder, int 
     } else {
       LSM_SEARCH(LSM_COUNT, s);
     }
-    size_t tmp_bytes = 0;
-    LSM_HIP(rocprim::inclusive_scan(nullptr, tmp_bytes, row_count, indptr + 1, (size_t)na,
-                                    rocprim::plus<long>(), C.stream));
-    void* tmp = C.scan_tmp.get(tmp_bytes);
-    LSM_HIP(rocprim::inclusive_scan(tmp, tmp_bytes, row_count, indptr + 1, (size_t)na,
-                                    rocprim::plus<long>(), C.stream));
-    hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, C.stream, indptr + na, s.maxrow, split ? s.ntasks : nullptr,
-                       C.hstat + 8);
+    const unsigned* ntasks = split ? s.ntasks : nullptr;
+    if (na <= kScanMax) {
+      hipLaunchKernelGGL(k_scan_rows, dim3(1), dim3(kScanBlock), 0, C.stream, (int)na, row_count, indptr, s.maxrow, ntasks,
+                         stage_flag(C), C.hstat + 8);
+    } else {
+      size_t tmp_bytes = 0;
+      LSM_HIP(rocprim::inclusive_scan(nullptr, tmp_bytes, row_count, indptr + 1, (size_t)na,
+                                      rocprim::plus<long>(), C.stream));
+      void* tmp = C.scan_tmp.get(tmp_bytes);
+      LSM_HIP(rocprim::inclusive_scan(tmp, tmp_bytes, row_count, indptr + 1, (size_t)na,
+                                      rocprim::plus<long>(), C.stream));
+      hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, C.stream, na, indptr, s.maxrow, ntasks, stage_flag(C),
+                         C.hstat + 8);
+    }
     LSM_HIP(hipGetLastError());
     LSM_HIP(hipStreamSynchronize(C.stream));
     if (!split || host[2] <= room) break;
     LSM_REQUIRE(host[2] < (1L << 31), LIBSUPERMESH_GPU_ERROR_OVERFLOW, "too many search tasks");
     room = host[2] + host[2] / 8;
+    hipLaunchKernelGGL(k_clear_words, dim3(1), dim3(64), 0, C.stream, 2, words);
   }
   const long npairs = host[0], maxrow = host[1];
   LSM_REQUIRE(npairs < (1L << 40), LIBSUPERMESH_GPU_ERROR_OVERFLOW, "too many candidate pairs");

@@ -150,9 +150,11 @@ struct Context {
   // batches: per-mesh pair offsets and measure sums
   DevBuf gpairs, gsum, gparts;
   // pinned status words the pipeline copies back asynchronously and reads
-  // after its next synchronisation: [0] staging flag, [1] longest mass row,
-  // [8..10] the search's pairs, longest row and tasks
+  // after its next synchronisation: [1] longest mass row, [8..11] the
+  // search's pairs, longest row, tasks and the staging flag, [16..21] the
+  // totals over the pairs
   long* hstat = nullptr;
+  int stage_serial = 0;  // of the latest staging
   Predictor predictor;
   // 2D mixed mass: rows laid out before the clip and filled by it
   bool mass_rows_ready = false;
@@ -175,11 +177,13 @@ struct Context {
 Context* default_context();
 
 // Mesh staging + BVH (finder.hip).
-// With defer_check the node-index check is left to the caller: it clears the
-// flag (stage_flag) before staging and reads it back later.
+// A node index out of range sets the flag (stage_flag) to the context's
+// stage_serial and is clamped: stage_mesh waits and checks it; after
+// stage_meshes find_pairs brings it to hstat[11], where the caller looks.
 void stage_mesh(Context& C, DevMesh& M, int dim, int loc, long nnodes, long nelements,
-                const double* positions, const int* enlist, bool need_planes, bool need_affine,
-                bool defer_check = false);
+                const double* positions, const int* enlist, bool need_planes, bool need_affine);
+void stage_meshes(Context& C, const libsupermesh_gpu_mesh& a, int loc_a, const libsupermesh_gpu_mesh& b, int loc_b,
+                  bool planes_b, bool affine);
 int* stage_flag(Context& C);
 // Mesh id of every element of a batch from its element offsets (device,
 // [ngroups + 1]); validates the offsets.

@@ -36,6 +36,10 @@ struct Partial {
   long long maxc, pad;
 };
 
+// Where k_reduce_partials leaves the totals for the host: pinned memory, so
+// that no copy follows it.
+static Partial* host_totals(Context& C) { return reinterpret_cast<Partial*>(C.hstat + 16); }
+
 __device__ __forceinline__ void two_sum(double a, double b, double& s, double& e) {
   s = a + b;
   double bb = s - a;
@@ -1145,7 +1149,7 @@ k_reduce_pairs(long npairs, const long* __restrict__ npairs_dev, const int* __re
   if (threadIdx.x == 0) partials[blockIdx.x] = red[0];
 }
 
-__global__ void __launch_bounds__(kClipBlock) k_reduce_partials(int n, Partial* __restrict__ parts) {
+__global__ void __launch_bounds__(kClipBlock) k_reduce_partials(int n, Partial* __restrict__ parts, Partial* __restrict__ host) {
   __shared__ Partial red[kClipBlock];
   Partial t = {0.0, 0.0, 0, 0, 0, 0};
   for (int i = threadIdx.x; i < n; i += kClipBlock) {
@@ -1167,7 +1171,10 @@ __global__ void __launch_bounds__(kClipBlock) k_reduce_partials(int n, Partial* 
     }
     __syncthreads();
   }
-  if (threadIdx.x == 0) parts[0] = red[0];
+  if (threadIdx.x == 0) {
+    parts[0] = red[0];
+    if (host) *host = red[0];
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1478,11 +1485,10 @@ void clip_pairs_mixed(Context& C, const DevMesh& A, const DevMesh& B, long npair
   Partial* parts = C.partials.as<Partial>(kClipGrid);
   hipLaunchKernelGGL(k_reduce_pairs, dim3(kClipGrid), dim3(kClipBlock), 0, C.stream, npairs, nullptr, g.counts, g.measure,
                      parts);
-  hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(kClipBlock), 0, C.stream, kClipGrid, parts);
+  hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(kClipBlock), 0, C.stream, kClipGrid, parts, host_totals(C));
   LSM_HIP(hipGetLastError());
-  Partial tot;
-  LSM_HIP(hipMemcpyAsync(&tot, parts, sizeof(Partial), hipMemcpyDeviceToHost, C.stream));
   LSM_HIP(hipStreamSynchronize(C.stream));
+  const Partial tot = *host_totals(C);
   out->counts = g.counts;
   out->measure = g.measure;
   out->blocks = nullptr;
@@ -2201,11 +2207,10 @@ void clip_pairs(Context& C, const DevMesh& A, const DevMesh& B, long npairs, int
   if (C.timing) LSM_HIP(hipEventRecord(C.ev[15], C.stream));
   hipLaunchKernelGGL(k_reduce_pairs, dim3(kClipGrid), dim3(kClipBlock), 0, C.stream, npairs, nullptr, g.counts,
                      g.measure, parts);
-  hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(kClipBlock), 0, C.stream, kClipGrid, parts);
+  hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(kClipBlock), 0, C.stream, kClipGrid, parts, host_totals(C));
   LSM_HIP(hipGetLastError());
-  Partial tot;
-  LSM_HIP(hipMemcpyAsync(&tot, parts, sizeof(Partial), hipMemcpyDeviceToHost, C.stream));
   LSM_HIP(hipStreamSynchronize(C.stream));
+  const Partial tot = *host_totals(C);
   if (C.timing) {
     float ms = 0.f;
     LSM_HIP(hipEventElapsedTime(&ms, C.ev[14], C.ev[15]));
@@ -2443,7 +2448,7 @@ static void enqueue_count_pass(Context& C, ClipArgs& g, int dim, long cap, const
   }
   hipLaunchKernelGGL(k_reduce_pairs, dim3(kClipGrid), dim3(kClipBlock), 0, C.stream, g.npairs, g.npairs_dev,
                      g.counts, g.measure, parts);
-  hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(kClipBlock), 0, C.stream, kClipGrid, parts);
+  hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(kClipBlock), 0, C.stream, kClipGrid, parts, nullptr);
   LSM_HIP(hipGetLastError());
   if (ngroups > 0) batch_sums(C, ngroups, a_off, indptr, g.measure);
 }
@@ -2831,7 +2836,7 @@ void clip_pairs_noalloc(int device, hipStream_t stream, const libsupermesh_gpu_m
     hipLaunchKernelGGL(k_clip_direct_tet, dim3(grid_for(npairs, kWalkBlock / 4)), dim3(kWalkBlock), 0, stream, g);
   }
   hipLaunchKernelGGL(k_reduce_pairs, dim3(kClipGrid), dim3(kClipBlock), 0, stream, npairs, nullptr, counts, measure, parts);
-  hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(kClipBlock), 0, stream, kClipGrid, parts);
+  hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(kClipBlock), 0, stream, kClipGrid, parts, nullptr);
   hipLaunchKernelGGL(k_noalloc_sum, dim3(1), dim3(64), 0, stream, parts, sum);
   LSM_HIP(hipGetLastError());
 }

@@ -1,7 +1,8 @@
 """The sort of the elements by Morton code: rows of an unsorted search come in
 the order of the hierarchy's leaves, which numpy's stable sort of the same
-codes gives, for element counts at the edges of the sort's tiles (2048 keys),
-of its groups of tiles and of the hierarchy's blocks (512 leaves)."""
+codes gives, for element counts at the edges of the one-block sort (8192 keys,
+1024 a round), of the tiles (2048 keys) and groups of the other, of the
+hierarchy's blocks (512 leaves) and of the one-block scan (16384 rows)."""
 import numpy as np
 import pytest
 
@@ -46,18 +47,24 @@ def loose(dim, n, seed, ties):
 
 
 @pytest.mark.parametrize("dim", [2, 3])
-@pytest.mark.parametrize("n", [1, 8, 63, 64, 65, 511, 512, 513, 2047, 2048, 2049, 4096 + 1, 8 * 2048 + 5, 33 * 2048 - 1])
-def test_rows_come_in_leaf_order(dim, n):
+@pytest.mark.parametrize("na, nb", [
+    # both within a block
+    (1, 1), (3, 8), (20, 63), (21, 64), (22, 65), (200, 511), (200, 512), (200, 513), (1025, 1023), (400, 1024),
+    (1024, 1025), (3000, 8191), (8192, 8192),
+    # one beyond
+    (9000, 1), (9000, 513), (9000, 2047), (9000, 2048), (9000, 2049), (3000, 8193), (2049, 8 * 2048 + 5),
+    (16384, 4096 + 1), (16385, 4096), (20000, 33 * 2048 - 1)])
+def test_rows_come_in_leaf_order(dim, na, nb):
     ctx = gpu.Context(0)
-    pb, eb = loose(dim, n, n, False)
-    pa, ea = loose(dim, max(n // 3, 1), n + 1, False)
+    pb, eb = loose(dim, nb, nb, False)
+    pa, ea = loose(dim, na, nb + 1, False)
     r = ctx.supermesh(gpu.DeviceMesh(pa, ea), gpu.DeviceMesh(pb, eb), flags=0)
     out = gpu.fetch(r, dim)
     rank = morton_rank(pb, eb)
     rows, cols = O.csr_to_pairs(out["indptr"], out["indices"])
     same = rows[1:] == rows[:-1]
     assert (np.diff(rank[cols])[same] > 0).all()
-    if n <= 20000:
+    if nb <= 20000:
         ip, ix = O.brute_force(pa, ea, pb, eb)
         assert np.array_equal(out["indptr"], ip)
         order = np.lexsort((cols, rows))
