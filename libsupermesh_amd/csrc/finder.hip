@@ -418,7 +418,7 @@ __device__ __forceinline__ void write_counts(const OrderJob& J, int tile, int pa
 }
 
 // Keys of a tile's elements, and the counts of their lowest digit.  With
-// `vals`, element ids beside the keys, for the library's sort.
+// VALS, element ids beside the keys instead, for the other sorts.
 template <int DIM, bool VALS>
 __global__ void __launch_bounds__(kBlock) k_morton(OrderArgs args) {
   __shared__ unsigned hist[kDigits];
@@ -699,19 +699,18 @@ k_build_levels(LevelInfo info, int l0, long ne, const double* __restrict__ bbox,
   x.store(info, l0 + 3, blockIdx.x, boxes, granges);
 }
 
-// Small meshes, a block each: order and, for the first, the hierarchy in one
-// launch (nine to eleven otherwise, each a few microseconds of latency with
-// next to no work).  A thread holds up to kSmallItems keys through the four
-// passes, exchanged in LDS; the 64 boxes of a wave give two levels by
-// shuffles, the at most 128 boxes of the second level the rest.
+// Tiny meshes, a block each: order and, for the first, the hierarchy in one
+// launch (five otherwise, each a few microseconds of latency with next to no
+// work).  A thread holds a key through the four passes, exchanged in LDS; the
+// 64 boxes of a wave give two levels by shuffles, the at most 16 boxes of the
+// second level the rest.  With eight keys a thread a block took 73 us for
+// 8192 elements: k_rank does those on the whole card.
 constexpr int kSmallBlock = 1024;
-constexpr int kSmallItems = 8;
-constexpr long kSmallMax = (long)kSmallBlock * kSmallItems;
+constexpr long kSmallMax = kSmallBlock;
 template <int DIM>
 __global__ void __launch_bounds__(kSmallBlock)
 k_small_order(OrderArgs args, LevelInfo info, double* __restrict__ boxes, int* __restrict__ granges) {
   constexpr int kWaves = kSmallBlock / 64;
-  constexpr int kTops = (int)(kSmallMax / (kFanout * kFanout));
   struct Sort {
     unsigned hist[kWaves][kDigits], wsum[kDigits / 64];
     uint32_t key[kSmallMax];
@@ -719,47 +718,32 @@ k_small_order(OrderArgs args, LevelInfo info, double* __restrict__ boxes, int* _
   };
   __shared__ union {
     Sort sort;
-    NodeBox<DIM> top[kTops];
+    NodeBox<DIM> top[kWaves];
   } mem;
   const OrderJob& J = args.job[blockIdx.x];
   if (blockIdx.x == 0 && threadIdx.x < 2) args.words[threadIdx.x] = 0;
   const int n = (int)J.ne, t = threadIdx.x, lane = t & 63, wave = t >> 6;
   if (n == 0) return;
-  const int items = (n + kSmallBlock - 1) / kSmallBlock;
+  const bool live = t < n;
   double b[2 * DIM];
 #pragma unroll
   for (int d = 0; d < DIM; d++) {
     b[d] = __builtin_inf();
     b[DIM + d] = -__builtin_inf();
   }
-  for (int e = t; e < n; e += kSmallBlock) {
+  if (live) {
 #pragma unroll
-    for (int d = 0; d < DIM; d++) {
-      const double c = 0.5 * (J.bbox[d * n + e] + J.bbox[(DIM + d) * n + e]);
-      b[d] = fmin_f(b[d], c);
-      b[DIM + d] = fmax_f(b[DIM + d], c);
-    }
+    for (int d = 0; d < DIM; d++) b[d] = b[DIM + d] = 0.5 * (J.bbox[d * n + t] + J.bbox[(DIM + d) * n + t]);
   }
   block_bounds<DIM, kSmallBlock>(b);
-  uint32_t key[kSmallItems];
-  int val[kSmallItems], rank[kSmallItems];
-  auto at = [&](int i) { return (wave * items + i) * 64 + lane; };  // this lane's i-th place
-#pragma unroll
-  for (int i = 0; i < kSmallItems; i++) {
-    if (i >= items) break;
-    val[i] = at(i);
-    key[i] = at(i) < n ? morton_key<DIM>(J, b, at(i)) : 0;
-  }
+  uint32_t key = live ? morton_key<DIM>(J, b, t) : 0;
+  int val = t;
   for (int pass = 0; pass < kSortPasses; pass++) {
     const int shift = 8 * pass;
 #pragma unroll
     for (int k = 0; k < kWaves * kDigits / kSmallBlock; k++) (&mem.sort.hist[0][0])[k * kSmallBlock + t] = 0;
     __syncthreads();
-#pragma unroll
-    for (int i = 0; i < kSmallItems; i++) {
-      if (i >= items) break;
-      rank[i] = rank_digit((key[i] >> shift) & (kDigits - 1), at(i) < n, mem.sort.hist[wave]);
-    }
+    const int rank = rank_digit((key >> shift) & (kDigits - 1), live, mem.sort.hist[wave]);
     __syncthreads();
     unsigned mine = 0, sum = 0;
     if (t < kDigits) {
@@ -784,59 +768,92 @@ k_small_order(OrderArgs args, LevelInfo info, double* __restrict__ boxes, int* _
       for (int w = 0; w < kWaves; w++) mem.sort.hist[w][t] += sum - mine;
     }
     __syncthreads();
-#pragma unroll
-    for (int i = 0; i < kSmallItems; i++) {
-      if (i >= items) break;
-      if (at(i) < n) {
-        const unsigned o = mem.sort.hist[wave][(key[i] >> shift) & (kDigits - 1)] + (unsigned)rank[i];
-        mem.sort.key[o] = key[i];
-        mem.sort.val[o] = val[i];
-      }
+    if (live) {
+      const unsigned o = mem.sort.hist[wave][(key >> shift) & (kDigits - 1)] + (unsigned)rank;
+      mem.sort.key[o] = key;
+      mem.sort.val[o] = val;
     }
     __syncthreads();
+    if (live) {
+      key = mem.sort.key[t];
+      val = mem.sort.val[t];
+    }
+  }
+  __syncthreads();
+  if (live) J.perm[t] = val;
+  if (blockIdx.x != 0 || boxes == nullptr) return;
+  NodeBox<DIM> x;
+  x.clear();
+  if (live) {
+    x.element(val, n, J.bbox, J.group);
+    x.store(info, 0, t, boxes, granges);
+  }
+  for (int o = 1; o < kFanout; o <<= 1) x.join(o);
+  if ((lane & 7) == 0) x.store(info, 1, t / kFanout, boxes, granges);
+  for (int o = kFanout; o < 64; o <<= 1) x.join(o);
+  if (lane == 0) {
+    x.store(info, 2, wave, boxes, granges);
+    mem.top[wave] = x;
+  }
+  __syncthreads();
+  if (wave != 0) return;
+  x.clear();
+  if (lane < kWaves) x = mem.top[lane];
+  for (int o = 1; o < kFanout; o <<= 1) x.join(o);
+  if ((lane & 7) == 0) x.store(info, 3, lane / kFanout, boxes, granges);
+  x.join(kFanout);  // kWaves is two groups
+  if (lane == 0) x.store(info, 4, 0, boxes, granges);
+}
+
+// The order of a small mesh's keys by counting: an element's place is the
+// number of smaller keys, and of equal ones before it.  64 elements to a
+// block, a lane each; each wave goes through every sixteenth 64 keys.  n^2
+// compares, but one launch on the whole card where the sort's seven wait for
+// each other: up to 8192 elements that is the shorter (the sort costs about
+// 45 us whatever the size).
+constexpr int kRankBlock = 1024;
+constexpr long kRankMax = 8192;
+__global__ void __launch_bounds__(kRankBlock) k_rank(OrderArgs args, int blocks0) {
+  constexpr int kWaves = kRankBlock / 64;
+  __shared__ __align__(16) uint32_t keys[kRankMax];
+  __shared__ int part[kWaves][64];
+  const bool second = (int)blockIdx.x >= blocks0;
+  const OrderJob& J = args.job[second ? 1 : 0];
+  const int mine = (int)blockIdx.x - (second ? blocks0 : 0);
+  const int n = (int)J.ne, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int chunks = (n + 63) / 64;
+  for (int k = threadIdx.x; k < chunks * 64; k += kRankBlock) keys[k] = k < n ? J.keys[0][k] : 0xffffffffu;
+  __syncthreads();
+  const uint32_t key = keys[mine * 64 + lane];
+  int place = 0;
+  for (int c = wave; c < chunks; c += kWaves) {
+    const uint4* k = reinterpret_cast<const uint4*>(keys + c * 64);
+    if (c < mine) {
 #pragma unroll
-    for (int i = 0; i < kSmallItems; i++) {
-      if (i >= items) break;
-      if (at(i) < n) {
-        key[i] = mem.sort.key[at(i)];
-        val[i] = mem.sort.val[at(i)];
+      for (int j = 0; j < 16; j++) {
+        const uint4 x = k[j];
+        place += (x.x <= key) + (x.y <= key) + (x.z <= key) + (x.w <= key);
+      }
+    } else if (c > mine) {
+#pragma unroll
+      for (int j = 0; j < 16; j++) {
+        const uint4 x = k[j];
+        place += (x.x < key) + (x.y < key) + (x.z < key) + (x.w < key);
+      }
+    } else {
+      for (int j = 0; j < 64; j++) {
+        const uint32_t x = keys[c * 64 + j];
+        place += x < key || (x == key && j < lane);
       }
     }
   }
+  part[wave][lane] = place;
   __syncthreads();
-  const bool build = blockIdx.x == 0 && boxes != nullptr;
-  NodeBox<DIM> x;
+  if (wave != 0 || mine * 64 + lane >= n) return;
+  place = 0;
 #pragma unroll
-  for (int i = 0; i < kSmallItems; i++) {
-    if (i >= items) break;
-    const int p = at(i);
-    if (p < n) J.perm[p] = val[i];
-    if (!build) continue;
-    x.clear();
-    if (p < n) {
-      x.element(val[i], n, J.bbox, J.group);
-      x.store(info, 0, p, boxes, granges);
-    }
-    for (int o = 1; o < kFanout; o <<= 1) x.join(o);
-    if ((lane & 7) == 0) x.store(info, 1, p / kFanout, boxes, granges);
-    for (int o = kFanout; o < 64; o <<= 1) x.join(o);
-    if (lane == 0) {
-      x.store(info, 2, p / (kFanout * kFanout), boxes, granges);
-      mem.top[wave * items + i] = x;
-    }
-  }
-  if (!build) return;
-  __syncthreads();
-  if (t >= kTops) return;  // whole waves
-  x.clear();
-  if (t < kWaves * items) x = mem.top[t];
-  for (int o = 1; o < kFanout; o <<= 1) x.join(o);
-  if ((lane & 7) == 0) x.store(info, 3, t / kFanout, boxes, granges);
-  for (int o = kFanout; o < 64; o <<= 1) x.join(o);
-  if (lane == 0) x.store(info, 4, wave, boxes, granges);
-  if (t != 0 || info.levels <= 5) return;
-  for (int k = 64; k < kWaves * items; k++) x.add(mem.top[k]);
-  x.store(info, 5, 0, boxes, granges);
+  for (int w = 0; w < kWaves; w++) place += part[w][lane];
+  J.perm[place] = mine * 64 + lane;
 }
 
 // Sorts the elements of M[0], and of M[1] if it is given, by Morton code:
@@ -846,7 +863,7 @@ static void morton_order(Context& C, int n, const DevMesh* const* M, DevBuf* con
   OrderArgs args = {};
   args.words = search_words(C);
   size_t total = 0, words = 0;
-  bool large = false, small = true;
+  bool large = false, small = true, count = true;
   for (int j = 0; j < n; j++) {
     OrderJob& J = args.job[j];
     J.ne = M[j]->nelements;
@@ -862,6 +879,7 @@ static void morton_order(Context& C, int n, const DevMesh* const* M, DevBuf* con
     words += (size_t)(J.tiles + kSortPasses * J.groups) * kDigits;
     large = large || J.ne > kOrderMax;
     small = small && J.ne <= kSmallMax;
+    count = count && J.ne <= kRankMax;
   }
   const bool flat = M[0]->dim == 2;
   const dim3 block(kBlock);
@@ -883,7 +901,7 @@ static void morton_order(Context& C, int n, const DevMesh* const* M, DevBuf* con
   double* part = C.partials.as<double>((size_t)n * kBoundParts * 6);
   uint32_t* keys[2] = {C.keys.as<uint32_t>(total), C.keys_alt.as<uint32_t>(total)};
   int* vals[2] = {C.vals.as<int>(total), C.vals_alt.as<int>(total)};
-  unsigned* table = large ? nullptr : C.sort_tmp.as<unsigned>(words);
+  unsigned* table = large || count ? nullptr : C.sort_tmp.as<unsigned>(words);
   size_t at = 0;
   for (int j = 0; j < n; j++) {
     OrderJob& J = args.job[j];
@@ -893,7 +911,7 @@ static void morton_order(Context& C, int n, const DevMesh* const* M, DevBuf* con
       J.vals[k] = vals[k] + at;
     }
     at += (size_t)J.ne;
-    if (large) {
+    if (large || count) {
       J.groups = 0;
       continue;
     }
@@ -905,7 +923,12 @@ static void morton_order(Context& C, int n, const DevMesh* const* M, DevBuf* con
   const dim3 tiles((unsigned)std::max(1, args.job[0].tiles + args.job[1].tiles));
   if (flat) hipLaunchKernelGGL(k_center_bounds<2>, parts, block, 0, C.stream, args);
   else hipLaunchKernelGGL(k_center_bounds<3>, parts, block, 0, C.stream, args);
-  if (large) {
+  if (count) {
+    if (flat) hipLaunchKernelGGL((k_morton<2, true>), tiles, block, 0, C.stream, args);
+    else hipLaunchKernelGGL((k_morton<3, true>), tiles, block, 0, C.stream, args);
+    const int blocks0 = (int)((args.job[0].ne + 63) / 64), blocks1 = (int)((args.job[1].ne + 63) / 64);
+    hipLaunchKernelGGL(k_rank, dim3((unsigned)(blocks0 + blocks1)), dim3(kRankBlock), 0, C.stream, args, blocks0);
+  } else if (large) {
     if (flat) hipLaunchKernelGGL((k_morton<2, true>), tiles, block, 0, C.stream, args);
     else hipLaunchKernelGGL((k_morton<3, true>), tiles, block, 0, C.stream, args);
     LSM_HIP(hipGetLastError());
@@ -1309,11 +1332,16 @@ __global__ void __launch_bounds__(kBlock) k_task_rows(SearchArgs s, const uint2*
   long run = 0;
   if (t < s.na) {
     const uint2 sp = span[t / kQueries];
-    for (unsigned k = 0; k < sp.y; k++) {
-      int* c = s.tcount + ((long)sp.x + k) * kQueries + t % kQueries;
-      const int n = *c;
-      *c = (int)run;
-      run += n;
+    int* c = s.tcount + (long)sp.x * kQueries + t % kQueries;
+    for (unsigned k = 0; k < sp.y; k += 8) {  // eight loads in flight
+      int n[8];
+#pragma unroll
+      for (unsigned j = 0; j < 8; j++) n[j] = k + j < sp.y ? c[(long)(k + j) * kQueries] : 0;
+#pragma unroll
+      for (unsigned j = 0; j < 8; j++) {
+        if (k + j < sp.y) c[(long)(k + j) * kQueries] = (int)run;
+        run += n[j];
+      }
     }
     s.row_count[s.qperm[t]] = run;
   }
@@ -1409,17 +1437,18 @@ k_scan_rows(int na, const long* __restrict__ row_count, long* __restrict__ indpt
 
 // Level of the hierarchy at which walks are cut into tasks, levels - 1 for
 // none.  A wave walks its part of the tree by itself, a few microseconds per
-// node on an idle card, so a search with few query waves is cut until the
-// card is full of tasks: nodes of 8^level elements.  In a batch, where a mesh
-// of a few elements may face one of tens of thousands, always to 512 elements.
-// A hierarchy of at most 64 elements is walked in less time than the two
-// launches that cut it take.
+// node on an idle card, so a search of few query waves is cut at nodes of 64
+// elements (tet 11^3 vs 10^3, 250 waves: the call 359 us, 422 uncut, 403 at
+// nodes of 8, 376 at 512).  From 2048 waves, eight per CU, the walks hide each
+// other and the two launches and the larger union are only a loss (tet 32^3 vs
+// 29^3, 6144 waves: 3.40 ms uncut, 3.63 at 512).  In a batch, where a mesh of
+// a few elements may face one of tens of thousands, always at 512 elements
+// (192 uneven mesh pairs: 6.5 ms, 10.8 uncut).  A hierarchy of at most 64
+// elements is walked in less time than the launches that cut it take.
 static int task_level(const LevelInfo& info, long waves, bool grouped) {
   const int top = info.levels - 1;
-  int level = waves >= 8192 ? top : (waves >= 2048 ? 3 : (waves >= 256 ? 2 : 1));
-  if (grouped && level > 3) level = 3;
-  if (top <= 2) level = top;
-  return level < top ? level : top;
+  if (top <= 2) return top;
+  return std::min(top, grouped ? 3 : (waves >= 2048 ? top : 2));
 }
 
 long find_pairs(Context& C, const DevMesh& A, const DevMesh& B, int finder, int sort_rows, bool ordered) {

@@ -1,7 +1,8 @@
 """The sort of the elements by Morton code: rows of an unsorted search come in
 the order of the hierarchy's leaves, which numpy's stable sort of the same
-codes gives, for element counts at the edges of the one-block sort (8192 keys,
-1024 a round), of the tiles (2048 keys) and groups of the other, of the
+codes gives, for element counts at the edges of the one-block sort (1024 keys), of
+the sort by counting (64 keys a block, up to 8192),
+of the tiles (2048 keys) and groups of tiles of the other, of the
 hierarchy's blocks (512 leaves) and of the one-block scan (16384 rows)."""
 import numpy as np
 import pytest
@@ -48,9 +49,9 @@ def loose(dim, n, seed, ties):
 
 @pytest.mark.parametrize("dim", [2, 3])
 @pytest.mark.parametrize("na, nb", [
-    # both within a block
+    # one block each (to 1024), counting (to 8192)
     (1, 1), (3, 8), (20, 63), (21, 64), (22, 65), (200, 511), (200, 512), (200, 513), (1025, 1023), (400, 1024),
-    (1024, 1025), (3000, 8191), (8192, 8192),
+    (1024, 1025), (1024, 1024), (300, 1025), (2000, 4095), (3000, 8191), (8192, 8192),
     # one beyond
     (9000, 1), (9000, 513), (9000, 2047), (9000, 2048), (9000, 2049), (3000, 8193), (2049, 8 * 2048 + 5),
     (16384, 4096 + 1), (16385, 4096), (20000, 33 * 2048 - 1)])
