@@ -64,6 +64,83 @@ static void init_context(Context& C, int device) {
   LSM_HIP(hipMemset(C.scalars.get(1024), 0, 1024));
 }
 
+constexpr size_t kHostChunk = 2 << 20;
+
+static void free_chunks(Context& C) {
+  for (int h = 0; h < 2; h++) {
+    if (C.chunk_ev[h]) (void)hipEventDestroy(C.chunk_ev[h]);
+    if (C.chunk[h]) (void)hipHostFree(C.chunk[h]);
+    C.chunk_ev[h] = nullptr;
+    C.chunk[h] = nullptr;
+    C.chunk_busy[h] = false;
+  }
+  C.chunk_bytes = 0;
+}
+
+// Halves for a transfer of `bytes`: its size, within 4 kB and kHostChunk.
+static void need_chunks(Context& C, size_t bytes) {
+  size_t want = 4096;
+  while (want < bytes && want < kHostChunk) want *= 2;
+  if (want <= C.chunk_bytes) return;
+  LSM_HIP(hipStreamSynchronize(C.stream));
+  free_chunks(C);
+  for (int h = 0; h < 2; h++) {
+    LSM_HIP(hipHostMalloc(reinterpret_cast<void**>(&C.chunk[h]), want, hipHostMallocDefault));
+    LSM_HIP(hipEventCreateWithFlags(&C.chunk_ev[h], hipEventDisableTiming));
+  }
+  C.chunk_bytes = want;
+}
+
+static void wait_chunk(Context& C, int h) {
+  if (C.chunk_busy[h]) LSM_HIP(hipEventSynchronize(C.chunk_ev[h]));
+  C.chunk_busy[h] = false;
+}
+
+static void mark_chunk(Context& C, int h) {
+  LSM_HIP(hipEventRecord(C.chunk_ev[h], C.stream));
+  C.chunk_busy[h] = true;
+}
+
+// n values to the device; put(first, count, out) writes `count` of them from
+// `first` on into pinned memory.  The copy of one half runs while the other
+// is written; nothing refers to the caller's arrays afterwards.
+template <class T, class Put>
+static void upload_chunks(Context& C, T* dst, size_t n, Put&& put) {
+  if (n == 0) return;
+  need_chunks(C, n * sizeof(T));
+  const size_t per = C.chunk_bytes / sizeof(T);
+  for (size_t i = 0; i < n; i += per) {
+    const size_t m = std::min(per, n - i);
+    const int h = C.chunk_next;
+    C.chunk_next ^= 1;
+    wait_chunk(C, h);
+    put(i, m, reinterpret_cast<T*>(C.chunk[h]));
+    LSM_HIP(hipMemcpyAsync(dst + i, C.chunk[h], m * sizeof(T), hipMemcpyHostToDevice, C.stream));
+    mark_chunk(C, h);
+  }
+}
+
+// n values from the device; take(first, count, in) reads them from pinned
+// memory, while the next ones are on their way.
+template <class T, class Take>
+static void download_chunks(Context& C, const T* src, size_t n, Take&& take) {
+  if (n == 0) return;
+  need_chunks(C, n * sizeof(T));
+  const size_t per = C.chunk_bytes / sizeof(T);
+  auto begin = [&](size_t i, int h) {
+    wait_chunk(C, h);
+    LSM_HIP(hipMemcpyAsync(C.chunk[h], src + i, std::min(per, n - i) * sizeof(T), hipMemcpyDeviceToHost, C.stream));
+    mark_chunk(C, h);
+  };
+  int h = C.chunk_next;
+  begin(0, h);
+  for (size_t i = 0; i < n; i += per, h ^= 1) {
+    if (i + per < n) begin(i + per, h ^ 1);
+    wait_chunk(C, h);
+    take(i, std::min(per, n - i), reinterpret_cast<const T*>(C.chunk[h]));
+  }
+}
+
 static void free_context(Context& C) {
   hipSetDevice(C.device);
   if (C.stream) hipStreamSynchronize(C.stream);
@@ -87,6 +164,7 @@ static void free_context(Context& C) {
   for (DevBuf* b : bufs) b->release();
   if (C.hstat) hipHostFree(C.hstat);
   C.hstat = nullptr;
+  free_chunks(C);
   if (C.events)
     for (int i = 0; i < 16; i++) hipEventDestroy(C.ev[i]);
   C.events = false;
@@ -453,6 +531,13 @@ struct FinderState {
   long nelements_a = 0;
   std::vector<long> indptr;
   std::vector<int> indices;
+  // a device search's results wait on the device for get_output, which brings
+  // them to the caller's arrays through pinned memory, and its buffers then
+  // go back to the context (a host copy in between was filled, read and
+  // freed on every call)
+  bool on_device = false;
+  long npairs = 0;
+  DevBuf dindptr, dindices;
 };
 
 static FinderState g_tree, g_rtree, g_sort, g_front;
@@ -505,24 +590,37 @@ static void host_mesh_to_device(Context& C, DevMesh& M, long nnodes, int dim, lo
               "Unsupported element type: simplices, quads or hexahedra only");
   LSM_REQUIRE(nnodes >= 0 && ne >= 0 && nnodes < (1L << 31) && ne < (1L << 31),
               LIBSUPERMESH_GPU_ERROR_INVALID, "Invalid mesh size");
-  std::vector<int> e32((size_t)ne * loc);
-  for (size_t i = 0; i < e32.size(); i++) {
-    long v = enl[i];
-    LSM_REQUIRE(v >= 0 && v < nnodes, LIBSUPERMESH_GPU_ERROR_INVALID, "Invalid node");
-    e32[i] = (int)v;
-  }
   double* dpos = M.pos_copy.as<double>((size_t)nnodes * dim);
   int* denl = M.enl_copy.as<int>((size_t)ne * loc);
-  if (nnodes > 0)
-    LSM_HIP(hipMemcpyAsync(dpos, pos, sizeof(double) * nnodes * dim, hipMemcpyHostToDevice, C.stream));
-  if (ne > 0)
-    LSM_HIP(hipMemcpyAsync(denl, e32.data(), sizeof(int) * ne * loc, hipMemcpyHostToDevice, C.stream));
-  LSM_HIP(hipStreamSynchronize(C.stream));
+  upload_chunks(C, denl, (size_t)ne * loc, [&](size_t i, size_t m, int* out) {
+    // the sign bit of v or of nnodes - 1 - v is set where v is out of range:
+    // no branch, so that the loop is vectorised
+    unsigned long bad = 0;
+    for (size_t k = 0; k < m; k++) {
+      const unsigned long v = (unsigned long)enl[i + k];
+      bad |= v | ((unsigned long)nnodes - 1 - v);
+      out[k] = (int)v;
+    }
+    LSM_REQUIRE((long)bad >= 0, LIBSUPERMESH_GPU_ERROR_INVALID, "Invalid node");
+  });
+  upload_chunks(C, dpos, (size_t)nnodes * dim,
+                [&](size_t i, size_t m, double* out) { std::memcpy(out, pos + i, m * sizeof(double)); });
   view.dim = dim;
   view.nnodes = nnodes;
   view.nelements = ne;
   view.positions = dpos;
   view.enlist = denl;
+}
+
+// The buffers of S's results to the context, if it has none by now: results
+// of a later call on it stay where they are.
+static void give_back(FinderState& S, Context& C) {
+  S.on_device = false;
+  if (!C.indptr.ptr) std::swap(S.dindptr, C.indptr);
+  if (!C.indices.ptr) std::swap(S.dindices, C.indices);
+  if (S.dindptr.ptr || S.dindices.ptr) LSM_HIP(hipStreamSynchronize(C.stream));
+  S.dindptr.release();
+  S.dindices.release();
 }
 
 static void finder_set_input(FinderState& S, int finder, long nnodes_a, int dim_a, long ne_a,
@@ -531,12 +629,11 @@ static void finder_set_input(FinderState& S, int finder, long nnodes_a, int dim_
                              const long* enl_b) {
   std::lock_guard<std::mutex> lk(S.mu);
   S.ready = false;
-  S.indptr.clear();
-  S.indices.clear();
   LSM_REQUIRE(dim_a == dim_b, LIBSUPERMESH_GPU_ERROR_INVALID, "Invalid dimension");
   Context& C = *default_context();
   std::lock_guard<std::mutex> lk2(C.mu);
   LSM_HIP(hipSetDevice(C.device));
+  give_back(S, C);  // results that nobody asked for
   libsupermesh_gpu_mesh va, vb;
   host_mesh_to_device(C, C.mesh_a, nnodes_a, dim_a, ne_a, loc_a, pos_a, enl_a, va);
   host_mesh_to_device(C, C.mesh_b, nnodes_b, dim_b, ne_b, loc_b, pos_b, enl_b, vb);
@@ -544,26 +641,39 @@ static void finder_set_input(FinderState& S, int finder, long nnodes_a, int dim_
   run_supermesh(C, &va, &vb, finder, LIBSUPERMESH_GPU_SORTED, false, &r, 0, nullptr, nullptr, loc_a,
                 loc_b);
   S.nelements_a = ne_a;
-  S.indptr.resize((size_t)ne_a + 1);
-  S.indices.resize((size_t)r.npairs);
-  LSM_HIP(hipMemcpy(S.indptr.data(), r.indptr, sizeof(long) * (ne_a + 1), hipMemcpyDeviceToHost));
-  if (r.npairs > 0)
-    LSM_HIP(hipMemcpy(S.indices.data(), r.indices, sizeof(int) * r.npairs, hipMemcpyDeviceToHost));
+  S.npairs = r.npairs;
+  std::swap(S.dindptr, C.indptr);
+  std::swap(S.dindices, C.indices);
+  S.on_device = true;
   S.ready = true;
 }
 
 static void finder_query_output(FinderState& S, long* nindices) {
   std::lock_guard<std::mutex> lk(S.mu);
   LSM_REQUIRE(S.ready, LIBSUPERMESH_GPU_ERROR_STATE, "query_output called before set_input");
-  *nindices = (long)S.indices.size();
+  *nindices = S.on_device ? S.npairs : (long)S.indices.size();
 }
 
 static void finder_get_output(FinderState& S, long nelements, long nindices, long* indices,
                               long* ind_ptr) {
   std::lock_guard<std::mutex> lk(S.mu);
   LSM_REQUIRE(S.ready, LIBSUPERMESH_GPU_ERROR_STATE, "get_output called before set_input");
-  LSM_REQUIRE(nelements == S.nelements_a && nindices == (long)S.indices.size(),
+  LSM_REQUIRE(nelements == S.nelements_a && nindices == (S.on_device ? S.npairs : (long)S.indices.size()),
               LIBSUPERMESH_GPU_ERROR_INVALID, "get_output sizes differ from query_output");
+  if (S.on_device) {
+    Context& C = *default_context();
+    std::lock_guard<std::mutex> lk2(C.mu);
+    LSM_HIP(hipSetDevice(C.device));
+    download_chunks(C, static_cast<const int*>(S.dindices.ptr), (size_t)nindices, [&](size_t i, size_t m, const int* in) {
+      for (size_t k = 0; k < m; k++) indices[i + k] = in[k];
+    });
+    download_chunks(C, static_cast<const long*>(S.dindptr.ptr), (size_t)nelements + 1, [&](size_t i, size_t m, const long* in) {
+      std::memcpy(ind_ptr + i, in, m * sizeof(long));
+    });
+    S.ready = false;
+    give_back(S, C);
+    return;
+  }
   for (long i = 0; i <= nelements; i++) ind_ptr[i] = S.indptr[i];
   for (long i = 0; i < nindices; i++) indices[i] = S.indices[i];
   S.ready = false;

@@ -155,6 +155,13 @@ struct Context {
   // totals over the pairs
   long* hstat = nullptr;
   int stage_serial = 0;  // of the latest staging
+  // pinned halves that host arrays pass through on their way to and from the
+  // device, at most kHostChunk bytes each; an event says when a half is free
+  char* chunk[2] = {nullptr, nullptr};
+  size_t chunk_bytes = 0;
+  hipEvent_t chunk_ev[2] = {nullptr, nullptr};
+  bool chunk_busy[2] = {false, false};
+  int chunk_next = 0;
   Predictor predictor;
   // 2D mixed mass: rows laid out before the clip and filled by it
   bool mass_rows_ready = false;
