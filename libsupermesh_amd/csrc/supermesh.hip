@@ -3395,7 +3395,10 @@ k_mass_rows_tet(long nn, const long* __restrict__ nptr, int* __restrict__ nlist,
 // ...; while a row is reduced, the next row's entries (up to 64 * PF) and the
 // one after's bounds are already being loaded.  Rows hold at most CAP entries
 // and the hash table 1 << HBITS slots: the smaller variant takes less LDS, so
-// more waves share a CU.
+// more waves share a CU.  A slot's value is loaded with its key, also where the
+// key then says that the pair is empty (never written, never used): waiting for
+// the key first left nothing in flight while a row was reduced (tri 1024^2 vs
+// 1000^2: 1.17 -> 1.02 ms, 2.1 GB of slots).
 template <int CAP, int PF, int HBITS>
 __global__ void __launch_bounds__(64)
 k_mass_rows_slots(long nn, const long* __restrict__ raw_off, int* __restrict__ tkey, double* __restrict__ tval,
@@ -3415,7 +3418,7 @@ k_mass_rows_slots(long nn, const long* __restrict__ raw_off, int* __restrict__ t
   for (int q = 0; q < PF; q++) {
     const long r = a0 + lane + 64 * q;
     ck[q] = r < a1 ? tkey[r] : -1;
-    cv[q] = ck[q] >= 0 ? tval[r] : 0.0;
+    cv[q] = r < a1 ? tval[r] : 0.0;
   }
   long j = i + stride;
   long b0 = 0, b1 = 0;
@@ -3439,7 +3442,7 @@ k_mass_rows_slots(long nn, const long* __restrict__ raw_off, int* __restrict__ t
     for (long rb = a0 + 64 * PF; rb < a1; rb += 64) {  // the rest of a long row
       const long r = rb + lane;
       const int key = r < a1 ? tkey[r] : -1;
-      const double v = key >= 0 ? tval[r] : 0.0;
+      const double v = r < a1 ? tval[r] : 0.0;
       const unsigned long long m = __ballot(key >= 0);
       if (key >= 0) {
         const int pos = n + __popcll(m & ((1ULL << lane) - 1));
@@ -3456,7 +3459,7 @@ k_mass_rows_slots(long nn, const long* __restrict__ raw_off, int* __restrict__ t
       for (int q = 0; q < PF; q++) {
         const long r = b0 + lane + 64 * q;
         ck[q] = r < b1 ? tkey[r] : -1;
-        cv[q] = ck[q] >= 0 ? tval[r] : 0.0;
+        cv[q] = r < b1 ? tval[r] : 0.0;
       }
       if (jn < nn) {
         c0 = raw_off[jn];
