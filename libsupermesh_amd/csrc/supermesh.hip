@@ -2203,7 +2203,7 @@ void clip_pairs(Context& C, const DevMesh& A, const DevMesh& B, long npairs, int
   if (C.timing) LSM_HIP(hipEventRecord(C.ev[14], C.stream));
   if (dim == 2) launch_clip<2>(C, g, mass, false);
   else if (learned) launch_tet_walk(C, g, mass ? 4 : 3);
-  else launch_tet_walk(C, g, mass, false);
+  else if (npairs > 0) launch_tet_walk(C, g, mass, false);  // without pairs there is no work list to read
   if (C.timing) LSM_HIP(hipEventRecord(C.ev[15], C.stream));
   hipLaunchKernelGGL(k_reduce_pairs, dim3(kClipGrid), dim3(kClipBlock), 0, C.stream, npairs, nullptr, g.counts,
                      g.measure, parts);
