@@ -385,27 +385,30 @@ static void run_callback_driver(Context& C, const libsupermesh_gpu_mesh* a, int 
   }
 }
 
-// Flags (bit 0) any pair whose A id is outside [0, na) or B id outside
-// [0, nb).
+// Sets *flag to `serial` where a pair's A id is outside [0, na) or its B id
+// outside [0, nb).
 __global__ void __launch_bounds__(256) k_check_pair_ids(long n, const int* __restrict__ pa,
                                                         const int* __restrict__ pb, long na, long nb,
-                                                        int* __restrict__ flag) {
+                                                        int* __restrict__ flag, int serial) {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n && (pa[i] < 0 || pa[i] >= na || pb[i] < 0 || pb[i] >= nb)) *flag = 1;
+  if (i < n && (pa[i] < 0 || pa[i] >= na || pb[i] < 0 || pb[i] >= nb)) *flag = serial;
 }
 
 // Checks caller-supplied pair lists against the mesh sizes before any kernel
-// reads coordinates through them.
+// reads coordinates through them.  The flag is the staging's and is marked the
+// same way, with a number of its own: any other mark would be taken for that
+// of the staging that gets its number.
 static void check_pair_ids(Context& C, long n, const int* pa, const int* pb, long na, long nb) {
   if (n <= 0) return;
   int* flag = stage_flag(C);
-  LSM_HIP(hipMemsetAsync(flag, 0, sizeof(int), C.stream));
-  hipLaunchKernelGGL(k_check_pair_ids, dim3(grid_for(n, 256)), dim3(256), 0, C.stream, n, pa, pb, na, nb, flag);
+  C.stage_serial++;
+  hipLaunchKernelGGL(k_check_pair_ids, dim3(grid_for(n, 256)), dim3(256), 0, C.stream, n, pa, pb, na, nb, flag,
+                     C.stage_serial);
   LSM_HIP(hipGetLastError());
   int h = 0;
   LSM_HIP(hipMemcpyAsync(&h, flag, sizeof(int), hipMemcpyDeviceToHost, C.stream));
   LSM_HIP(hipStreamSynchronize(C.stream));
-  LSM_REQUIRE(h == 0, LIBSUPERMESH_GPU_ERROR_INVALID, "Invalid element: pair id out of range");
+  LSM_REQUIRE(h != C.stage_serial, LIBSUPERMESH_GPU_ERROR_INVALID, "Invalid element: pair id out of range");
 }
 
 __global__ void __launch_bounds__(256) k_low_byte(long n, int* __restrict__ v) {

@@ -154,7 +154,7 @@ struct Context {
   // search's pairs, longest row, tasks and the staging flag, [16..21] the
   // totals over the pairs
   long* hstat = nullptr;
-  int stage_serial = 0;  // of the latest staging
+  int stage_serial = 0;  // of the latest staging or check of a pair list
   // pinned halves that host arrays pass through on their way to and from the
   // device, at most kHostChunk bytes each; an event says when a half is free
   char* chunk[2] = {nullptr, nullptr};
