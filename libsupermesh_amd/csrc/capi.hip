@@ -61,7 +61,9 @@ static void init_context(Context& C, int device) {
   for (int i = 0; i < 16; i++) LSM_HIP(hipEventCreate(&C.ev[i]));
   C.events = true;
   LSM_HIP(hipHostMalloc(reinterpret_cast<void**>(&C.hstat), 64 * sizeof(long), hipHostMallocDefault));
-  LSM_HIP(hipMemset(C.scalars.get(1024), 0, 1024));
+  // on the context's own stream, which does not wait for the null stream: a
+  // clear queued there could land between the kernels of the first call
+  LSM_HIP(hipMemsetAsync(C.scalars.get(1024), 0, 1024, C.stream));
 }
 
 constexpr size_t kHostChunk = 2 << 20;
