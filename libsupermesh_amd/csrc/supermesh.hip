@@ -1538,16 +1538,17 @@ k_batch_pairs(long ngroups, const long* __restrict__ a_off, const long* __restri
   if (g <= ngroups) gpairs[g] = indptr[a_off[g]];
 }
 
-// ... and its measure sum, double-double in a fixed order: kSumParts blocks a
-// mesh, then one wave adds their parts.  (One block a mesh was a chain of
-// thousands of dependent loads and adds on the largest mesh: 2.0 ms of a batch
-// of ~100 mesh pairs of up to 50 000 tets.)
+// ... and its measure sum, double-double in a fixed order: `parts` blocks a
+// mesh, then, if there is more than one, a wave adds their sums.  (One block a
+// mesh was a chain of thousands of dependent loads and adds on the largest
+// mesh: 2.0 ms of a batch of ~100 mesh pairs of up to 50 000 tets.)
 constexpr int kSumParts = 64;
 __global__ void __launch_bounds__(kClipBlock)
-k_batch_sum(const long* __restrict__ gpairs, const double* __restrict__ measure, double2* __restrict__ parts) {
-  const long g = blockIdx.y, first = gpairs[g], n = gpairs[g + 1] - first;
+k_batch_sum(const long* __restrict__ gpairs, const double* __restrict__ measure, int parts, double2* __restrict__ sums,
+            double* __restrict__ gsum) {
+  const long g = blockIdx.x / parts, first = gpairs[g], n = gpairs[g + 1] - first;
   double hi = 0.0, lo = 0.0;
-  for (long p = (long)blockIdx.x * kClipBlock + threadIdx.x; p < n; p += kSumParts * kClipBlock)
+  for (long p = (long)(blockIdx.x % parts) * kClipBlock + threadIdx.x; p < n; p += (long)parts * kClipBlock)
     dd_add(hi, lo, measure[first + p]);
   __shared__ double rh[kClipBlock], rl[kClipBlock];
   rh[threadIdx.x] = hi;
@@ -1562,20 +1563,42 @@ k_batch_sum(const long* __restrict__ gpairs, const double* __restrict__ measure,
     }
     __syncthreads();
   }
-  if (threadIdx.x == 0) parts[g * kSumParts + blockIdx.x] = make_double2(rh[0], rl[0]);
+  if (threadIdx.x != 0) return;
+  if (parts == 1) gsum[g] = rh[0] + rl[0];
+  else sums[blockIdx.x] = make_double2(rh[0], rl[0]);
 }
 
 __global__ void __launch_bounds__(64)
-k_batch_total(const double2* __restrict__ parts, double* __restrict__ gsum) {
+k_batch_total(int parts, const double2* __restrict__ sums, double* __restrict__ gsum) {
   static_assert(kSumParts == 64, "a lane per part");
-  const double2 x = parts[(long)blockIdx.x * kSumParts + threadIdx.x];
-  double hi = x.x, lo = x.y;
+  double hi = 0.0, lo = 0.0;
+  if ((int)threadIdx.x < parts) {
+    const double2 x = sums[(long)blockIdx.x * parts + threadIdx.x];
+    hi = x.x;
+    lo = x.y;
+  }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
     const double h2 = __shfl_down(hi, o, 64), l2 = __shfl_down(lo, o, 64);
     dd_merge(hi, lo, h2, l2);
   }
   if (threadIdx.x == 0) gsum[blockIdx.x] = hi + lo;
+}
+
+// Blocks per mesh of a batch's sums: 64 up to 128 meshes, then as many as give
+// 8192 blocks, four times what the card holds at once, and one from 8192
+// meshes on, which fill it by themselves (64 for any number of them were 1.3 M
+// nearly empty blocks and 20 MB of parts for 20 000 mesh pairs of 8 and 18
+// triangles: the call 1.50 ms, 0.62 with one).  A rule on the number of meshes
+// alone: a recorded count pass serves other numbers of pairs.
+static int batch_parts(long ngroups) {
+  return (int)std::max(1L, std::min<long>(kSumParts, 8192 / std::max(1L, ngroups)));
+}
+
+// The parts' sums of a batch, if there is more than one per mesh.
+static double2* batch_part_sums(Context& C, long ngroups) {
+  const int parts = batch_parts(ngroups);
+  return parts > 1 ? C.gparts.as<double2>((size_t)ngroups * parts) : nullptr;
 }
 
 // Order-sensitive 64-bit checksum of a device buffer: sum over its 32-bit
@@ -1626,12 +1649,13 @@ void batch_sums(Context& C, long ngroups, const long* a_offsets, const long* ind
   double* gs = C.gsum.as<double>((size_t)ngroups);
   hipLaunchKernelGGL(k_batch_pairs, dim3(grid_for(ngroups + 1, kClipBlock)), dim3(kClipBlock), 0,
                      C.stream, ngroups, a_offsets, indptr, gp);
-  // the grid's second dimension holds 65535 meshes
-  double2* parts = C.gparts.as<double2>((size_t)ngroups * kSumParts);
-  for (long g0 = 0; g0 < ngroups; g0 += 65535)
-    hipLaunchKernelGGL(k_batch_sum, dim3(kSumParts, (unsigned)std::min<long>(65535, ngroups - g0)), dim3(kClipBlock), 0,
-                       C.stream, gp + g0, measure, parts + g0 * kSumParts);
-  if (ngroups > 0) hipLaunchKernelGGL(k_batch_total, dim3((unsigned)ngroups), dim3(64), 0, C.stream, parts, gs);
+  const int parts = batch_parts(ngroups);
+  double2* sums = batch_part_sums(C, ngroups);
+  if (ngroups > 0)
+    hipLaunchKernelGGL(k_batch_sum, dim3((unsigned)(ngroups * parts)), dim3(kClipBlock), 0, C.stream, gp, measure, parts,
+                       sums, gs);
+  if (ngroups > 0 && parts > 1)
+    hipLaunchKernelGGL(k_batch_total, dim3((unsigned)ngroups), dim3(64), 0, C.stream, parts, sums, gs);
   LSM_HIP(hipGetLastError());
 }
 
@@ -2544,7 +2568,7 @@ void count_pass_graph(Context& C, const DevMesh& A, const DevMesh& B, long npair
   if (ngroups > 0) {
     C.gpairs.as<long>((size_t)ngroups + 1);
     C.gsum.as<double>((size_t)ngroups);
-    C.gparts.as<double2>((size_t)ngroups * kSumParts);
+    batch_part_sums(C, ngroups);
   }
   if (dim == 2) {
     g.olist = static_cast<int*>(C.work.ptr);
