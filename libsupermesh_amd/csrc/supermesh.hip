@@ -857,73 +857,79 @@ static unsigned long long* walk_queues(Context& C) {
   return q;
 }
 
-// The P1 x P1 mass of a pair from its kept tets' moments, one row of the block
-// per lane.  add() takes a kept tet in coordinates local to o, a vertex of the
-// pair's first output (inside both elements, so that the basis functions at o
-// lie in [0, 1] and nothing cancels); its integrals of 1, d_i and d_i d_j are
-// V, V/4 sum_v d_v and V/20 (sum_v d_v d_v' + (sum d)(sum d)'), exact for the
-// quadratic products, where the reference sums its 4-point rule, exact for
-// them too, over the tets (test_parallel_p1_inner_product_3d.F90:226-337).
-struct TetMoments {
-  double m[10];  // 1, x, y, z, xx, xy, xz, yy, yz, zz
-  double o[3];
+// The P1 x P1 mass of a pair, a share of it per lane: m[4 i + j] is the integral
+// over this lane's kept tets of f_i g_j, f = (1, A's basis functions 1 to 3), g
+// likewise of B.  A tet's is closed in its vertex values,
+// int f g = V / 20 (sum_v f_v g_v + (sum_v f_v)(sum_v g_v)), where the reference
+// sums its 4-point rule, exact for these products too
+// (test_parallel_p1_inner_product_3d.F90:226-337).  The functions are evaluated
+// vertex by vertex, so that the large gradients of thin elements cost each of
+// two factors its own digits and their product no more: moments in x, y, z
+// contracted with both gradients lost the digits of both (median over pairs of
+// tilted tets 1e-3 thick: 4e-13 of the pair's mass instead of 2e-14; the call
+// at tet 32^3 vs 30^3 3.47 ms instead of 3.74).
+struct TetMass {
+  double m[16];
   __device__ __forceinline__ void clear() {
 #pragma unroll
-    for (int i = 0; i < 10; i++) m[i] = 0.0;
+    for (int i = 0; i < 16; i++) m[i] = 0.0;
   }
-  __device__ __forceinline__ void add(const double* t, double vol) {
-    double d[4][3], s[3];
+  static __device__ __forceinline__ void values(const double* __restrict__ aff, const double* x, double* f) {
+    const double dx = x[0] - aff[0], dy = x[1] - aff[1], dz = x[2] - aff[2];
 #pragma unroll
-    for (int k = 0; k < 3; k++) {
+    for (int r = 0; r < 3; r++)
+      f[r] = __builtin_fma(aff[5 + 3 * r], dz, __builtin_fma(aff[4 + 3 * r], dy, aff[3 + 3 * r] * dx));
+  }
+  __device__ __forceinline__ void add(const double* t, double vol, const double* __restrict__ affa,
+                                      const double* __restrict__ affb) {
+    const double w = 0.05 * vol, w5 = 0.25 * vol;
+    double sa[3] = {0.0, 0.0, 0.0}, sb[3] = {0.0, 0.0, 0.0};
 #pragma unroll
-      for (int v = 0; v < 4; v++) d[v][k] = t[3 * v + k] - o[k];
-      s[k] = (d[0][k] + d[1][k]) + (d[2][k] + d[3][k]);
+    for (int v = 0; v < 4; v++) {
+      double f[3], g[3];
+      values(affa, t + 3 * v, f);
+      values(affb, t + 3 * v, g);
+#pragma unroll
+      for (int i = 0; i < 3; i++) {
+        sa[i] += f[i];
+        sb[i] += g[i];
+        const double wf = w * f[i];
+#pragma unroll
+        for (int j = 0; j < 3; j++) m[5 + 4 * i + j] = __builtin_fma(wf, g[j], m[5 + 4 * i + j]);
+      }
     }
-    const double w4 = 0.25 * vol, w20 = 0.05 * vol;
     m[0] += vol;
 #pragma unroll
-    for (int k = 0; k < 3; k++) m[1 + k] = __builtin_fma(w4, s[k], m[1 + k]);
-    int n = 4;
+    for (int i = 0; i < 3; i++) {
+      m[1 + i] = __builtin_fma(w5, sb[i], m[1 + i]);
+      m[4 + 4 * i] = __builtin_fma(w5, sa[i], m[4 + 4 * i]);
+      const double wf = w * sa[i];
 #pragma unroll
-    for (int i = 0; i < 3; i++)
-#pragma unroll
-      for (int j = i; j < 3; j++) {
-        double x = s[i] * s[j];
-#pragma unroll
-        for (int v = 0; v < 4; v++) x = __builtin_fma(d[v][i], d[v][j], x);
-        m[n] = __builtin_fma(w20, x, m[n]);
-        n++;
-      }
+      for (int j = 0; j < 3; j++) m[5 + 4 * i + j] = __builtin_fma(wf, sb[j], m[5 + 4 * i + j]);
+    }
   }
-  // Row q of the block: int phi^A_q phi^B_j, j = 0..3 (whole quad).
-  __device__ __forceinline__ void row(int q, const double* __restrict__ affa, const double* __restrict__ affb,
-                                      double* out) {
-    double M[10];
+  // Row q of the quad's block, int phi^A_q phi^B_j (whole quad).  Each lane
+  // hands the two rows that the other pair of lanes is to have to that pair,
+  // then one row to its neighbour.
+  __device__ __forceinline__ void row(int q, double* out) {
+    double half[8], r[4];
 #pragma unroll
-    for (int i = 0; i < 10; i++) M[i] = quad_sum(m[i]);
-    double fa[4], fb[4], ga[3], alpha;
-    basis<3>(affa, o, fa);
-    basis<3>(affb, o, fb);
-    alpha = q == 0 ? fa[0] : (q == 1 ? fa[1] : (q == 2 ? fa[2] : fa[3]));
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-      const double g1 = affa[3 + k], g2 = affa[6 + k], g3 = affa[9 + k];
-      ga[k] = q == 0 ? -((g1 + g2) + g3) : (q == 1 ? g1 : (q == 2 ? g2 : g3));
+    for (int i = 0; i < 8; i++) {
+      const double keep = q & 2 ? m[8 + i] : m[i], give = q & 2 ? m[i] : m[8 + i];
+      half[i] = keep + quad_xor<2>(give);
     }
-    // int phi^A_q and int phi^A_q d
-    const double i0 = alpha * M[0] + (ga[0] * M[1] + ga[1] * M[2] + ga[2] * M[3]);
-    const double ix = alpha * M[1] + (ga[0] * M[4] + ga[1] * M[5] + ga[2] * M[6]);
-    const double iy = alpha * M[2] + (ga[0] * M[5] + ga[1] * M[7] + ga[2] * M[8]);
-    const double iz = alpha * M[3] + (ga[0] * M[6] + ga[1] * M[8] + ga[2] * M[9]);
-    double rest = 0.0;
 #pragma unroll
-    for (int j = 1; j < 4; j++) {
-      const double* h = affb + 3 * j;
-      const double g = h[0] * ix + h[1] * iy + h[2] * iz;
-      out[j] = fb[j] * i0 + g;
-      rest += g;
+    for (int i = 0; i < 4; i++) {
+      const double keep = q & 1 ? half[4 + i] : half[i], give = q & 1 ? half[i] : half[4 + i];
+      r[i] = keep + quad_xor<1>(give);
     }
-    out[0] = fb[0] * i0 - rest;
+    // basis function 0: one minus the others, of B and then of A
+    r[0] -= (r[1] + r[2]) + r[3];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const double rest = (quad_lane<1>(r[j]) + quad_lane<2>(r[j])) + quad_lane<3>(r[j]);
+      out[j] = q == 0 ? r[j] - rest : r[j];
+    }
   }
 };
 
@@ -939,7 +945,10 @@ k_clip_tet_walk(ClipArgs g) {
   __shared__ uint4 table[256];
   for (int i = threadIdx.x; i < 256; i += BLOCK) table[i] = reinterpret_cast<const uint4*>(kSplitTable.e)[i];
   __syncthreads();
-  QuadClip<4> W;
+  // the mass needs the registers that the planes would take (tet 32^3 vs 30^3
+  // with the mass: 3.74 ms; planes in registers and two waves per SIMD 3.88,
+  // three waves and spills 5.24)
+  QuadClip<4, !MASS> W;
   W.init(&lds[threadIdx.x >> 6], table);
   const int q = W.q;
   // blocks go to the XCDs round robin: each XCD takes one contiguous share
@@ -979,7 +988,7 @@ k_clip_tet_walk(ClipArgs g) {
   bool lost = false;
   unsigned nsplit = 0, nlost = 0;  // this quad's split runs and pairs to clip again
   double tol = 0.0, m = 0.0;
-  TetMoments mom;
+  TetMass mass;
   auto start = [&]() {
     p = np;
     a = na;
@@ -991,7 +1000,7 @@ k_clip_tet_walk(ClipArgs g) {
     m = 0.0;
     k = 0;
     lost = false;
-    if (MASS) mom.clear();
+    if (MASS) mass.clear();
     W.set_plane(q, nP);
     W.begin(nv);
     active = true;
@@ -1018,7 +1027,7 @@ k_clip_tet_walk(ClipArgs g) {
         }
         if (MASS) {
           double row[4] = {0.0, 0.0, 0.0, 0.0};
-          if (k > 0) mom.row(q, g.aaff + (long)a * 12, g.baff + (long)b * 12, row);
+          if (k > 0) mass.row(q, row);
 #pragma unroll
           for (int j = 0; j < 4; j++) g.blocks[(long)p * 16 + 4 * q + j] = row[j];
         }
@@ -1068,17 +1077,7 @@ k_clip_tet_walk(ClipArgs g) {
       m = m + quad_lane<1>(vr);
       m = m + quad_lane<2>(vr);
       const uint32_t kept = quad_or((keep ? 1u : 0u) << q);
-      if (MASS) {
-        // the origin: the first output's first vertex
-        const uint32_t first = lead & -lead;
-#pragma unroll
-        for (int i = 0; i < 3; i++) {
-          const double x0 = quad_lane<0>(t[i]), x1 = quad_lane<1>(t[i]), x2 = quad_lane<2>(t[i]);
-          const double x = first == 1u ? x0 : (first == 2u ? x1 : x2);
-          mom.o[i] = k == 0 ? x : mom.o[i];
-        }
-        if (keep) mom.add(t, vr);
-      }
+      if (MASS && keep) mass.add(t, vr, g.aaff + (long)a * 12, g.baff + (long)b * 12);
       if (FILL || LEARNED) {
         const int at = k + __builtin_popcount(kept & ((1u << q) - 1u));
         if (keep && at < cap) {

@@ -213,10 +213,16 @@ __device__ __forceinline__ uint32_t quad_or(uint32_t x) {
   x |= (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x4e, 0xf, 0xf, true);  // lanes 2 3 0 1
   return x;
 }
-// Sum over the quad, the same in its four lanes.
-__device__ __forceinline__ double quad_sum(double x) {
-  const double a = quad_lane<0>(x) + quad_lane<1>(x);
-  return a + (quad_lane<2>(x) + quad_lane<3>(x));
+// The value of the lane whose number differs by X (1 or 2).
+template <int X>
+__device__ __forceinline__ double quad_xor(double x) {
+  constexpr int kPerm = X == 1 ? 0xb1 : 0x4e;
+  uint64_t b;
+  __builtin_memcpy(&b, &x, 8);
+  b = (uint64_t)(uint32_t)__builtin_amdgcn_mov_dpp((int)(b >> 32), kPerm, 0xf, 0xf, true) << 32 |
+      (uint32_t)__builtin_amdgcn_mov_dpp((int)b, kPerm, 0xf, 0xf, true);
+  __builtin_memcpy(&x, &b, 8);
+  return x;
 }
 
 // The wave's lanes exchange data through LDS in program order; only the
@@ -241,8 +247,9 @@ struct QuadLds {
   uint32_t stack[kEntries][kWords][16];
 };
 
-// One quad's clip: begin() with a tet, then step() until done().
-template <int NP>
+// One quad's clip: begin() with a tet, then step() until done().  With REGS the
+// planes are kept in registers.
+template <int NP, bool REGS = true>
 struct QuadClip {
   static constexpr int kRows = QuadLds<NP>::kRows, kWords = QuadLds<NP>::kWords, SW = code_words(NP);
   double* pool;
@@ -257,7 +264,7 @@ struct QuadClip {
   bool cur;         // T is to be done
   // planes 1..NP-1, which every new vertex is classified against (in LDS they
   // took a fifth of its traffic, which bounds the step beside the VALU)
-  double P[NP - 1][4];
+  double P[REGS ? NP - 1 : 1][4];
 
   __device__ __forceinline__ void init(QuadLds<NP>* lds, const uint4* tab) {
     const int lane = threadIdx.x & 63, g = lane >> 2;
@@ -296,7 +303,12 @@ struct QuadClip {
 #pragma unroll
       for (int j = w == 0 ? 1 : 0; j < 4; j++) {
         const int p = 4 * w + j;
-        const unsigned s = p < NP ? side_code(plane_distance(P[p < NP ? p - 1 : 0], v)) : 1u;
+        unsigned s = 1u;
+        if (p < NP) {
+          double pl[4];
+          if (!REGS) get_plane(p, pl);
+          s = side_code(plane_distance(REGS ? P[REGS && p < NP ? p - 1 : 0] : pl, v));
+        }
         c[w] |= s << (2 * j);
       }
     }
@@ -313,7 +325,7 @@ struct QuadClip {
     for (int k = 0; k < 3; k++) pool[k * kRows + q] = v[k];
     quad_fence();
 #pragma unroll
-    for (int j = 1; j < NP; j++) get_plane(j, P[j - 1]);
+    for (int j = 1; j < (REGS ? NP : 1); j++) get_plane(j, P[j - 1]);
     double P0[4];
     get_plane(0, P0);
     uint32_t c[SW];
