@@ -3277,6 +3277,21 @@ k_mass_rows_long(long nn, const long* __restrict__ raw_off, int* __restrict__ tk
   }
 }
 
+// Columns that row i of the 3D mass can have at most: four per candidate pair of
+// its elements, and no more than the row kernel takes.
+__global__ void __launch_bounds__(256)
+k_tet_row_bounds(long nn, const long* __restrict__ nptr, const int* __restrict__ nlist, const long* __restrict__ indptr,
+                 long* __restrict__ bound) {
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= nn) return;
+  long n = 0;
+  for (long x = nptr[i]; x < nptr[i + 1]; x++) {
+    const long e = nlist[x] >> 2;
+    n += 4 * (indptr[e + 1] - indptr[e]);
+  }
+  bound[i] = n < kMaxDistinct ? n : kMaxDistinct;
+}
+
 // 3D rows, one wave each, from the per-pair blocks: the wave takes the node's
 // elements in ascending order, an element's candidate pairs 64 at a time, and
 // its non-empty pairs sixteen at a time, four lanes a pair (a B node each).
@@ -3290,8 +3305,8 @@ k_mass_rows_long(long nn, const long* __restrict__ raw_off, int* __restrict__ tk
 __global__ void __launch_bounds__(256)
 k_mass_rows_tet(long nn, const long* __restrict__ nptr, int* __restrict__ nlist, const long* __restrict__ indptr,
                 const int* __restrict__ cols, const int* __restrict__ counts, const double* __restrict__ blocks,
-                const int* __restrict__ enlb, int* __restrict__ tkey, double* __restrict__ tval,
-                long* __restrict__ ucount, int* __restrict__ overflow) {
+                const int* __restrict__ enlb, const long* __restrict__ raw_off, int* __restrict__ tkey,
+                double* __restrict__ tval, long* __restrict__ ucount, int* __restrict__ overflow) {
   __shared__ int s_key[4][kHashSlots];
   __shared__ double s_sum[4][kHashSlots];
   const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 3;
@@ -3398,8 +3413,9 @@ k_mass_rows_tet(long nn, const long* __restrict__ nptr, int* __restrict__ nlist,
     return;
   }
   // each lane's columns, packed across the wave through the output row
-  int* out_key = tkey + i * kMaxDistinct;
-  double* out_val = tval + i * kMaxDistinct;
+  const long out = raw_off ? raw_off[i] : i * kMaxDistinct;
+  int* out_key = tkey + out;
+  double* out_val = tval + out;
   int done = 0;
 #pragma unroll
   for (int s0 = 0; s0 < kHashSlots; s0 += 64) {
@@ -3725,13 +3741,29 @@ void assemble_mass(Context& C, const DevMesh& A, const DevMesh& B, long npairs,
   int* nlist = C.ukeys.as<int>(nent + 1);
   hipLaunchKernelGGL(k_node_fill, dim3(grid_for(nent, 256)), dim3(256), 0, C.stream, na, loc,
                      A.enlist_dev, nptr, cursor, nlist);
-  int* tkey = C.mkeys.as<int>((size_t)nn * kMaxDistinct);
-  double* tval = C.mvals.as<double>((size_t)nn * kMaxDistinct);
+  // The rows' columns before they are packed: the most that a row may hold, one
+  // row after another.  A pair adds to four rows, four columns each, so where
+  // that is less (nodes without elements, an A that B covers in part) the rows
+  // lie by their own bounds: never more than 16 columns, 192 bytes, per pair,
+  // whose block took 128.
+  size_t room = (size_t)nn * kMaxDistinct;
+  long* raw_off = nullptr;
+  if (room > 16 * (size_t)npairs) {
+    room = 16 * (size_t)npairs;
+    long* bound = C.mslot.as<long>(2 * (size_t)nn + 1);
+    raw_off = bound + nn;
+    hipLaunchKernelGGL(k_tet_row_bounds, dim3(grid_for(nn, 256)), dim3(256), 0, C.stream, nn, nptr, nlist, out->indptr,
+                       bound);
+    LSM_HIP(hipMemsetAsync(raw_off, 0, sizeof(long), C.stream));
+    inclusive_scan_long(C, bound, raw_off + 1, nn);
+  }
+  int* tkey = C.mkeys.as<int>(room);
+  double* tval = C.mvals.as<double>(room);
   long* ucount = C.mvals_alt.as<long>(nn + 1);
   int* ovf = C.scalars.as<int>(64) + 4;
   LSM_HIP(hipMemsetAsync(ovf, 0, sizeof(int), C.stream));
   hipLaunchKernelGGL(k_mass_rows_tet, dim3(grid_for(nn, 4)), dim3(256), 0, C.stream, nn, nptr, nlist, out->indptr,
-                     out->indices, out->counts, out->blocks, B.enlist_dev, tkey, tval, ucount, ovf);
+                     out->indices, out->counts, out->blocks, B.enlist_dev, raw_off, tkey, tval, ucount, ovf);
   LSM_HIP(hipGetLastError());
   // scanned before the overflow flag is known: one read-back for both
   inclusive_scan_long(C, ucount, mindptr + 1, nn);
@@ -3746,7 +3778,7 @@ void assemble_mass(Context& C, const DevMesh& A, const DevMesh& B, long npairs,
   const long nnz = C.hstat[3];
   int* mind = C.mindices.as<int>(nnz);
   double* mval = C.uvals.as<double>(nnz);
-  hipLaunchKernelGGL(k_mass_copy, dim3(grid_for(nn, 256 / kCopyLanes)), dim3(256), 0, C.stream, nn, nullptr, mindptr,
+  hipLaunchKernelGGL(k_mass_copy, dim3(grid_for(nn, 256 / kCopyLanes)), dim3(256), 0, C.stream, nn, raw_off, mindptr,
                      tkey, tval, mind, mval);
   LSM_HIP(hipGetLastError());
   out->mass_nnz = nnz;
