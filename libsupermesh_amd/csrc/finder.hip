@@ -1023,7 +1023,7 @@ struct SearchArgs {
   // tasks: (query wave, node at `level`) pairs; without them, every wave
   // starts at the root
   const int2* tasks;
-  const unsigned* ntasks;
+  const unsigned long long* ntasks;
   unsigned cap;         // tasks that the arrays hold
   int level;
   int* tcount;          // [cap][kQueries]: results of the wave's queries below the task's node, then their prefix sums
@@ -1237,7 +1237,8 @@ __device__ __forceinline__ long grid_wave() {
 // order; first[w] and count[w] say which.
 template <int DIM, bool CLOSED, bool GROUPED>
 __global__ void __launch_bounds__(kBlock)
-k_search_tasks(SearchArgs s, int2* __restrict__ tasks, unsigned* __restrict__ ntasks, uint2* __restrict__ span) {
+k_search_tasks(SearchArgs s, int2* __restrict__ tasks, unsigned long long* __restrict__ ntasks,
+               uint2* __restrict__ span) {
   const long w = grid_wave();
   if (w * kQueries >= s.na) return;
   const Queries<DIM, GROUPED> Q(s, w);
@@ -1246,13 +1247,17 @@ k_search_tasks(SearchArgs s, int2* __restrict__ tasks, unsigned* __restrict__ nt
   walk_union<DIM, CLOSED, GROUPED>(s, Q, top, 0, s.level, [&](long, const unsigned long long* m) {
     n += __builtin_popcount(any_query(m));
   });
+  // the first task's place: one beyond the arrays is not written, and all of a
+  // total beyond them is unused (the host sees it and calls again with room),
+  // so that the places below need no more than 32 bits
   unsigned at = 0;
   if (lane == 0) {
-    if (n) at = atomicAdd(ntasks, n);
+    const unsigned long long first = n ? atomicAdd(ntasks, (unsigned long long)n) : 0;
+    at = first < s.cap ? (unsigned)first : s.cap;
     span[w] = make_uint2(at, n);
   }
   at = (unsigned)__builtin_amdgcn_readfirstlane((int)at);
-  if (at + n > s.cap) return;  // the host sees the total and calls again with room
+  if (n > s.cap - at) return;
   walk_union<DIM, CLOSED, GROUPED>(s, Q, top, 0, s.level, [&](long first, const unsigned long long* m) {
     const unsigned u = any_query(m);
     if (lane < kFanout && ((u >> lane) & 1u))
@@ -1328,7 +1333,7 @@ __global__ void __launch_bounds__(kBlock) k_search(SearchArgs s) {
 // queries' rows.  A lane per query.
 __global__ void __launch_bounds__(kBlock) k_task_rows(SearchArgs s, const uint2* __restrict__ span) {
   const long t = (long)blockIdx.x * kBlock + threadIdx.x;
-  if (*s.ntasks > s.cap) return;
+  if (*s.ntasks > (unsigned long long)s.cap) return;
   long run = 0;
   if (t < s.na) {
     const uint2 sp = span[t / kQueries];
@@ -1379,7 +1384,7 @@ k_sort_rows(long na, const long* __restrict__ indptr, int* __restrict__ indices)
 
 // The words that the host waits for, in its own memory: [0] the pairs, [1]
 // the longest row, [2] the tasks, [3] the staging flag.
-__device__ __forceinline__ void publish(long npairs, const long* maxrow, const unsigned* ntasks, const int* bad,
+__device__ __forceinline__ void publish(long npairs, const long* maxrow, const unsigned long long* ntasks, const int* bad,
                                         long* host) {
   host[0] = npairs;
   host[1] = *maxrow;
@@ -1388,7 +1393,8 @@ __device__ __forceinline__ void publish(long npairs, const long* maxrow, const u
 }
 
 __global__ void k_publish(long na, long* __restrict__ indptr, const long* __restrict__ maxrow,
-                          const unsigned* __restrict__ ntasks, const int* __restrict__ bad, long* __restrict__ host) {
+                          const unsigned long long* __restrict__ ntasks, const int* __restrict__ bad,
+            long* __restrict__ host) {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
   indptr[0] = 0;
   publish(indptr[na], maxrow, ntasks, bad, host);
@@ -1401,7 +1407,8 @@ constexpr int kScanItems = 16;
 constexpr long kScanMax = (long)kScanBlock * kScanItems;
 __global__ void __launch_bounds__(kScanBlock)
 k_scan_rows(int na, const long* __restrict__ row_count, long* __restrict__ indptr, const long* __restrict__ maxrow,
-            const unsigned* __restrict__ ntasks, const int* __restrict__ bad, long* __restrict__ host) {
+            const unsigned long long* __restrict__ ntasks, const int* __restrict__ bad,
+            long* __restrict__ host) {
   __shared__ long wsum[kScanBlock / 64];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int items = (na + kScanBlock - 1) / kScanBlock;
@@ -1523,7 +1530,7 @@ long find_pairs(Context& C, const DevMesh& A, const DevMesh& B, int finder, int 
       int2* tasks = C.ftasks.as<int2>(room);
       uint2* span = C.fspan.as<uint2>(waves);
       s.tcount = C.fcount.as<int>((size_t)room * kQueries);
-      unsigned* ntasks = reinterpret_cast<unsigned*>(words + 1);
+      unsigned long long* ntasks = reinterpret_cast<unsigned long long*>(words + 1);
       s.tasks = nullptr;
       grid = wave_grid;
       LSM_SEARCH(LSM_TASKS, s, tasks, ntasks, span);
@@ -1535,7 +1542,7 @@ long find_pairs(Context& C, const DevMesh& A, const DevMesh& B, int finder, int 
     } else {
       LSM_SEARCH(LSM_COUNT, s);
     }
-    const unsigned* ntasks = split ? s.ntasks : nullptr;
+    const unsigned long long* ntasks = split ? s.ntasks : nullptr;
     if (na <= kScanMax) {
       hipLaunchKernelGGL(k_scan_rows, dim3(1), dim3(kScanBlock), 0, C.stream, (int)na, row_count, indptr, s.maxrow, ntasks,
                          stage_flag(C), C.hstat + 8);
