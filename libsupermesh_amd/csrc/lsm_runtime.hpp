@@ -157,11 +157,13 @@ struct Context {
   int stage_serial = 0;  // of the latest staging or check of a pair list
   // pinned halves that host arrays pass through on their way to and from the
   // device, at most kHostChunk bytes each; an event says when a half is free
+  char* chunk_block = nullptr;  // their memory, where it is not hstat's page
   char* chunk[2] = {nullptr, nullptr};
   size_t chunk_bytes = 0;
   hipEvent_t chunk_ev[2] = {nullptr, nullptr};
   bool chunk_busy[2] = {false, false};
   int chunk_next = 0;
+  bool uploads_once = false;    // a tree's context: large arrays come once, when it is built
   Predictor predictor;
   // 2D mixed mass: rows laid out before the clip and filled by it
   bool mass_rows_ready = false;
