@@ -33,7 +33,11 @@ extern "C" {
 /* Tree (quadtree / octree) candidate finder, strict AABB overlap.
  * set_input runs the whole search; query_output returns the number of pairs;
  * get_output fills indices[nindices] (B ids, ascending within each row) and
- * ind_ptr[nelements + 1] and releases the result.
+ * ind_ptr[nelements + 1] and releases the result, which lies in device memory
+ * until then or until the next set_input of the same finder (tree or R-tree).
+ * get_output brings it to the host, and waits meanwhile for calls of other
+ * threads that run on the library's own context (any finder's set_input, the
+ * mesh adjacency functions).
  * Replaces src/C_bindings.F90:346-391 (declared at include/libsupermesh-c.h:21-23). */
 void libsupermesh_tree_intersection_finder_set_input(long* nnodes_a, int* dim_a, long* nelements_a, int* loc_a, long* nnodes_b, int* dim_b, long* nelements_b, int* loc_b, c_kind* positions_a, long* enlist_a, c_kind* positions_b, long* enlist_b);
 void libsupermesh_tree_intersection_finder_query_output(long* nindices);

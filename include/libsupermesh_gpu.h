@@ -166,7 +166,8 @@ int libsupermesh_gpu_synchronize(int device);
 
 /* The count pass's launch shape the context measured fastest for dimension
  * dim (LIBSUPERMESH_GPU_GRAPH; zeros before the first such call): threads per
- * block, blocks in the grid (3D: the walk's persistent lanes / block; 2D:
+ * block, blocks in the grid (3D: the walk's persistent lanes / block, four
+ * lanes to a pair; 2D:
  * blocks of the grid-stride loop, i.e. the pairs each wave takes, or 0: one
  * block per `block` pairs, each lane one pair), the tet depths whose stack
  * lives in LDS (3D: 3, all of them; 2D: 0) and the time of that shape on the
@@ -279,8 +280,8 @@ int libsupermesh_gpu_predictor_get(libsupermesh_gpu_context* ctx, float* params)
 int libsupermesh_gpu_predictor_quantile(libsupermesh_gpu_context* ctx, float q);
 /* Outputs beyond a pair's budget go to an arena of fraction x the predicted
  * output plus min_tets tets (defaults 0.25 and 2^20; 0 and 0: no arena)
- * split among the clip's lanes; such runs are then joined in the spill
- * reserve, and pairs that find their lane's share full (every pair beyond
+ * split among the clip's quads of lanes; such runs are then joined in the
+ * spill reserve, and pairs that find their quad's share full (every pair beyond
  * its budget, without an arena) are clipped again into it. */
 int libsupermesh_gpu_predictor_arena(libsupermesh_gpu_context* ctx, float fraction, long min_tets);
 /* The spill reserve: fraction x the predicted output plus min_tets tets
