@@ -1,8 +1,9 @@
 // lsm_geometry.hpp -- FP64 element geometry and the per-pair clippers.
 //
-// Every routine here runs one candidate pair per lane with its whole state in
-// VGPRs: no per-lane arrays are indexed with run-time values, so nothing goes
-// to scratch.  The library is compiled with -ffp-contract=off and the code
+// What the kernels use of it runs one candidate pair per lane (or, for tets, as a
+// quad's lane) with its whole state in VGPRs: no per-lane arrays are indexed with
+// run-time values, so nothing goes to scratch.  clip_tet and the walk further
+// down clip one pair in one thread, for the one-pair functions.  The library is compiled with -ffp-contract=off and the code
 // spells out each operation in the reference's order, so every result rounds
 // exactly as the reference's Fortran does (IEEE double, no FMA, correctly
 // rounded division and square root).
@@ -385,13 +386,6 @@ LSM_HD double in_reg(double x) {
   return x;
 }
 
-LSM_HD int in_reg_i(int x) {
-#ifdef __HIP_DEVICE_COMPILE__
-  asm volatile("" : "+v"(x));
-#endif
-  return x;
-}
-
 LSM_HD double sel4(const double* a, int k) {
   const double a0 = in_reg(a[0]), a1 = in_reg(a[1]), a2 = in_reg(a[2]), a3 = in_reg(a[3]);
   double r = a3;
@@ -588,12 +582,10 @@ LSM_HD Tet make_child(const Tet& T, const Split& s, int ci) {
 }
 
 // ---------------------------------------------------------------------------
-// Flat depth-first walk: the same clip as clip_tet, written as a loop whose
-// body always does the same work -- build one child, then classify it (or
-// measure it, at the last plane) -- so that lanes of a wave at different
-// depths, in different split cases, or on different pairs run in lockstep.
-// A child is built from a recipe (up to three split points, then a source for
-// each of the four output slots) that reproduces clip_buf's vertex order.
+// Flat depth-first walk, for one pair in one thread: the same clip as clip_tet,
+// written as a loop over any number of planes.  A child is built from a recipe
+// (up to three split points, then a source for each of the four output slots)
+// that reproduces clip_buf's vertex order.
 // ---------------------------------------------------------------------------
 
 // Packed classification: bits 0-2 kind (0 discard, 1 keep, 2 +++-, 3 ++--,
@@ -731,21 +723,13 @@ LSM_HD void build_child(const double* T, const double* d, const Recipe& r, doubl
   }
 }
 
-// Depth-first walk over the clip tree of one pair and NP planes, in which
-// every step builds exactly one child: the next child is built (and, at depth
-// NP, handed to the sink; otherwise pushed and classified against the next
-// plane), then the walk climbs over every depth whose children are all done.
-// The lanes of a wave stay in lockstep: the work of a step does not depend on
-// the depth, the split case or whether the child is a leaf.  State: the class
-// of the current tet at each depth 0..NP-1 against the plane below it, the
-// depth of the next child to build (0 once the walk is over) and the index
-// of the next child at each depth 1..NP (2 bits each).  Tets at depths
-// 1..NREG live in the caller's registers R (depth d at R[(d - 1) * 12 + i]),
-// and those at depths NREG+1..NP-1 in the caller's stack: depth d at
-// stk[((d - NREG - 1) * 12 + i) * STRIDE], so a wave's lanes can interleave
-// their stacks in LDS (STRIDE = lanes) or a host caller use a plain array
-// (STRIDE = 1).  Register depths cost a select per coordinate and step; each
-// takes 96 bytes per lane off the stack.
+// Depth-first walk over the clip tree of one pair and NP planes: each step
+// builds the next child (and, at depth NP, hands it to the sink; otherwise
+// pushes it and classifies it against the next plane), then climbs over every
+// depth whose children are all done.  State: the class of the current tet at
+// each depth 0..NP-1 against the plane below it, the depth of the next child to
+// build (0 once the walk is over) and the index of the next child at each depth
+// 1..NP (2 bits each).  The tet at depth d is at stk[(d - 1) * 12].
 template <int NP>
 struct WalkState {
   int cls[NP];
@@ -779,66 +763,32 @@ LSM_HD void walk_begin(WalkState<NP>& W, int cls0) {
   walk_climb(W);
 }
 
-// One step (W.level >= 1).  plane(j, out) gives plane j (0..NP-1) as
-// [n0 n1 n2 c].  Calls sink(tet, vol_tet, keep) once per step: keep is true
-// for the kept output tets, in the reference's order, and false otherwise
-// (the tet is then not an output).
-template <int NP, int STRIDE, int NREG = 0, class PlaneFn, class Sink>
-LSM_HD void walk_next(WalkState<NP>& W, const double* A, double* R, double* stk, PlaneFn&& plane,
-                      double tol, Sink&& sink) {
-  static_assert(NREG >= 0 && NREG < NP, "register depths 1..NREG, NREG < NP");
+// One step (W.level >= 1).  Calls sink(tet, vol_tet) for a kept output tet.
+template <int NP, class Sink>
+LSM_HD void walk_next(WalkState<NP>& W, const double* A, double* stk, const double* planes, double tol, Sink&& sink) {
   const int k = W.level;
   const int ci = (W.digits >> (2 * k)) & 3;
-  int c = in_reg_i(W.cls[0]);
-#pragma unroll
-  for (int j = 1; j < NP; j++) c = k == j + 1 ? in_reg_i(W.cls[j]) : c;
-  // the parent (depth k-1): A at depth 0, a register tet at depths 1..NREG,
-  // else the stack's; the stack word is read in any case so that the loads
-  // are issued together
-  const int sd = k - 2 - NREG;
-  const double* src = stk + (sd > 0 ? sd : 0) * 12 * STRIDE;
-  double parent[12];
-#pragma unroll
-  for (int i = 0; i < 12; i++) {
-    double v = in_reg(src[i * STRIDE]);
-#pragma unroll
-    for (int r = NREG; r >= 1; r--) v = k == r + 1 ? in_reg(R[(r - 1) * 12 + i]) : v;
-    parent[i] = k == 1 ? in_reg(A[i]) : v;
-  }
-  double pl[4], pd[4];
-  plane(k - 1, pl);
-  walk_distances(parent, pl, pd);
-  double child[12];
-  build_child(parent, pd, make_recipe(c, ci), child);
+  const double* parent = k == 1 ? A : stk + (k - 2) * 12;
+  double pd[4], child[12];
+  walk_distances(parent, planes + 4 * (k - 1), pd);
+  build_child(parent, pd, make_recipe(W.cls[k - 1], ci), child);
   W.digits += 1 << (2 * k);
-  const bool leaf = k == NP;
-  const double vol = tet_volume_tet(child);
-  sink(child, vol, leaf && vol >= tol);
-  // the child's class against the next plane (computed at depth NP too, and
-  // unused there)
-  double cp[4], dc[4];
-  plane(k < NP ? k : NP - 1, cp);
-  walk_distances(child, cp, dc);
-  const int cc = pack_class(dc);
-#pragma unroll
-  for (int r = 1; r <= NREG; r++) {
-#pragma unroll
-    for (int i = 0; i < 12; i++) R[(r - 1) * 12 + i] = k == r ? child[i] : R[(r - 1) * 12 + i];
+  if (k == NP) {
+    const double vol = tet_volume_tet(child);
+    if (vol >= tol) sink(child, vol);
+  } else {
+    double dc[4];
+    walk_distances(child, planes + 4 * k, dc);
+    W.cls[k] = pack_class(dc);
+    for (int i = 0; i < 12; i++) stk[(k - 1) * 12 + i] = child[i];
+    W.digits &= ~(3 << (2 * (k + 1)));
+    W.level = k + 1;
   }
-  if (!leaf && k > NREG) {
-    double* dst = stk + (k - 1 - NREG) * 12 * STRIDE;
-#pragma unroll
-    for (int i = 0; i < 12; i++) dst[i * STRIDE] = child[i];
-  }
-#pragma unroll
-  for (int j = 1; j < NP; j++) W.cls[j] = !leaf && k == j ? cc : W.cls[j];
-  W.digits = leaf ? W.digits : (W.digits & ~(3 << (2 * (k + 1))));
-  W.level = leaf ? k : k + 1;
   walk_climb(W);
 }
 
-// Whole walk of one pair on the host or in a single lane: sink(tet, vol_tet)
-// for each kept output tet; returns how many.  planes: NP x [n0 n1 n2 c].
+// Whole walk of one pair: sink(tet, vol_tet) for each kept output tet; returns
+// how many.  planes: NP x [n0 n1 n2 c].
 template <int NP, class Sink>
 LSM_HD int walk_whole(const double* A, const double* planes, double tol, Sink&& sink) {
   double stk[12 * (NP - 1)];
@@ -847,31 +797,13 @@ LSM_HD int walk_whole(const double* A, const double* planes, double tol, Sink&& 
   WalkState<NP> W;
   walk_begin(W, pack_class(d0));
   int kept = 0;
-  auto plane = [&](int j, double* o) {
-#pragma unroll
-    for (int i = 0; i < 4; i++) o[i] = planes[4 * j + i];
-  };
   while (W.level > 0)
-    walk_next<NP, 1>(W, A, nullptr, stk, plane, tol, [&](const double* t, double v, bool keep) {
-      if (keep) {
-        sink(t, v);
-        kept++;
-      }
+    walk_next<NP>(W, A, stk, planes, tol, [&](const double* t, double v) {
+      sink(t, v);
+      kept++;
     });
   return kept;
 }
-
-// Whole clip of one pair with the walk (host checks).
-template <class Sink>
-LSM_HD int clip_tet_walk(const double* A, const Planes& P, double tol, Sink&& sink) {
-  double planes[16];
-  for (int i = 0; i < 4; i++) {
-    for (int k = 0; k < 3; k++) planes[4 * i + k] = P.n[i][k];
-    planes[4 * i + 3] = P.c[i];
-  }
-  return walk_whole<4>(A, planes, tol, sink);
-}
-
 
 // The six face planes of a hexahedron in Gmsh node order, normals from
 // unit_cross as written in intersect_tet_hex (Supermesh.F90:269-280); no

@@ -1,6 +1,7 @@
 // supermesh.hip -- clipping kernels, reductions and P1 x P1 mixed mass.
 //
-// One candidate pair per lane.  The kernels read element vertex coordinates
+// One candidate pair per lane in 2D, per quad of lanes in 3D (tet_quad.hpp).  The
+// kernels read element vertex coordinates
 // from the element-major arrays staged by finder.hip (48 B per triangle,
 // 96 B per tet) and, for tets, B's four planes precomputed once per element
 // (get_planes_tet is a pure function of the element, so this is bitwise the
@@ -60,98 +61,45 @@ __device__ __forceinline__ void dd_merge(double& hi, double& lo, double hi2, dou
   lo = lo + (e + lo2);
 }
 
-// Quadrature rules of the reference's mixed-mass tests: Dunavant degree 2 on
-// triangles (barycentric (4,1,1)/6, weights 1/3; test_parallel_p1_inner_product_2d.F90:59-68)
-// and the 4-point Stroud rule on tets (..._3d.F90:61-80).
-__constant__ double kQ2[3][3] = {{4.0 / 6.0, 1.0 / 6.0, 1.0 / 6.0},
-                                 {1.0 / 6.0, 4.0 / 6.0, 1.0 / 6.0},
-                                 {1.0 / 6.0, 1.0 / 6.0, 4.0 / 6.0}};
-#define LSM_QA 5.8541019662496852e-1
-#define LSM_QB 1.3819660112501050e-1
-__constant__ double kQ3[4][4] = {{LSM_QA, LSM_QB, LSM_QB, LSM_QB},
-                                 {LSM_QB, LSM_QA, LSM_QB, LSM_QB},
-                                 {LSM_QB, LSM_QB, LSM_QA, LSM_QB},
-                                 {LSM_QB, LSM_QB, LSM_QB, LSM_QA}};
-
-template <int DIM>
+// Values at x of the basis functions of a triangle's barycentric map.
 __device__ __forceinline__ void basis(const double* __restrict__ aff, const double* x, double* f) {
-  if constexpr (DIM == 2) {
-    double dx = x[0] - aff[0], dy = x[1] - aff[1];
-    double f2 = aff[2] * dx;
-    f2 = f2 + aff[3] * dy;
-    double f3 = aff[4] * dx;
-    f3 = f3 + aff[5] * dy;
-    f[1] = f2;
-    f[2] = f3;
-    f[0] = 1.0 - f2 - f3;
-  } else {
-    double dx = x[0] - aff[0], dy = x[1] - aff[1], dz = x[2] - aff[2];
-    double s = 0.0;
-#pragma unroll
-    for (int r = 0; r < 3; r++) {
-      double v = aff[3 + 3 * r] * dx;
-      v = v + aff[4 + 3 * r] * dy;
-      v = v + aff[5 + 3 * r] * dz;
-      f[1 + r] = v;
-    }
-    s = 1.0 - f[1] - f[2] - f[3];
-    f[0] = s;
-  }
+  double dx = x[0] - aff[0], dy = x[1] - aff[1];
+  double f2 = aff[2] * dx;
+  f2 = f2 + aff[3] * dy;
+  double f3 = aff[4] * dx;
+  f3 = f3 + aff[5] * dy;
+  f[1] = f2;
+  f[2] = f3;
+  f[0] = 1.0 - f2 - f3;
 }
 
-// Adds the element's contributions to blk[LOC][LOC].  2D: the product of two
-// P1 functions is quadratic, so the 3-point rule of the reference tests
+// Adds a triangle's contributions to blk[3][3].  The product of two P1 functions
+// is quadratic, so the 3-point rule of the reference tests
 // (test_parallel_p1_inner_product_2d.F90:59-68) equals the closed form
 // int_c f g = |c|/12 (sum_v f_v g_v + (sum_v f_v)(sum_v g_v)) over c's
 // vertex values; this evaluates the latter (about half the operations; sums
 // may use fused multiply-adds: the mass is compared within 1e-12, not
-// bitwise).  3D: the reference's 4-point rule as written.
-template <int DIM>
-__device__ __forceinline__ void mass_element(const double* el, double meas, const double* affa,
-                                             const double* affb, double* blk) {
-  if constexpr (DIM == 2) {
-    double fa[3][3], fb[3][3];  // [vertex][basis]
+// bitwise).
+__device__ __forceinline__ void mass_triangle(const double* el, double meas, const double* affa, const double* affb,
+                                              double* blk) {
+  double fa[3][3], fb[3][3];  // [vertex][basis]
 #pragma unroll
-    for (int v = 0; v < 3; v++) {
-      basis<2>(affa, el + 2 * v, fa[v]);
-      basis<2>(affb, el + 2 * v, fb[v]);
-    }
-    const double w = meas * (1.0 / 12.0);
-#pragma unroll
-    for (int i = 0; i < 3; i++) {
-      const double sa = fa[0][i] + fa[1][i] + fa[2][i];
-#pragma unroll
-      for (int j = 0; j < 3; j++) {
-        const double sb = fb[0][j] + fb[1][j] + fb[2][j];
-        double d = __builtin_fma(fa[0][i], fb[0][j], sa * sb);
-        d = __builtin_fma(fa[1][i], fb[1][j], d);
-        d = __builtin_fma(fa[2][i], fb[2][j], d);
-        blk[i * 3 + j] = __builtin_fma(w, d, blk[i * 3 + j]);
-      }
-    }
-    return;
+  for (int v = 0; v < 3; v++) {
+    basis(affa, el + 2 * v, fa[v]);
+    basis(affb, el + 2 * v, fb[v]);
   }
-  constexpr int LOC = DIM + 1;
-  constexpr int NQ = DIM == 2 ? 3 : 4;
-  const double wq = DIM == 2 ? 1.0 / 3.0 : 0.25;
-  const double wm = wq * meas;
+  const double w = meas * (1.0 / 12.0);
 #pragma unroll
-  for (int q = 0; q < NQ; q++) {
-    double x[DIM];
+  for (int i = 0; i < 3; i++) {
+    const double sa = fa[0][i] + fa[1][i] + fa[2][i];
 #pragma unroll
-    for (int d = 0; d < DIM; d++) {
-      double s = 0.0;
-#pragma unroll
-      for (int v = 0; v < LOC; v++) s = s + (DIM == 2 ? kQ2[q][v] : kQ3[q][v]) * el[v * DIM + d];
-      x[d] = s;
+    for (int j = 0; j < 3; j++) {
+      const double sb = fb[0][j] + fb[1][j] + fb[2][j];
+      double d = __builtin_fma(fa[0][i], fb[0][j], sa * sb);
+      d = __builtin_fma(fa[1][i], fb[1][j], d);
+      d = __builtin_fma(fa[2][i], fb[2][j], d);
+      blk[i * 3 + j] = __builtin_fma(w, d, blk[i * 3 + j]);
     }
-    double fa[LOC], fb[LOC];
-    basis<DIM>(affa, x, fa);
-    basis<DIM>(affb, x, fb);
-#pragma unroll
-    for (int i = 0; i < LOC; i++)
-#pragma unroll
-      for (int j = 0; j < LOC; j++) blk[i * LOC + j] = blk[i * LOC + j] + wm * fa[i] * fb[j];
   }
 }
 
@@ -177,7 +125,7 @@ __device__ __forceinline__ void tri_moments(double x0, double y0, double x1, dou
 // A's first vertex, where phi^A = (1, 0, 0)): with phi^A_i = alpha_i + g_i.d
 // and phi^B_j = beta_j + h_j.d, the integral is alpha_i beta_j I + alpha_i
 // h_j.Id + beta_j g_i.Id + g_i^T Idd h_j.  The same integral as summing
-// mass_element<2> over the fan, in exact arithmetic.
+// mass_triangle over the fan, in exact arithmetic.
 __device__ __forceinline__ void mass_from_moments(const double* mom, const double* affa, const double* affb,
                                                   double* blk) {
   double g[3][2], h[3][2], beta[3];
@@ -194,7 +142,7 @@ __device__ __forceinline__ void mass_from_moments(const double* mom, const doubl
   h[0][0] = -(h[1][0] + h[2][0]);
   h[0][1] = -(h[1][1] + h[2][1]);
   const double o[2] = {affa[0], affa[1]};
-  basis<2>(affb, o, beta);
+  basis(affb, o, beta);
 #pragma unroll
   for (int j = 0; j < 3; j++) {
     const double hd = h[j][0] * mom[1] + h[j][1] * mom[2];            // h_j . Id
@@ -234,13 +182,13 @@ struct ClipArgs {
   // run starts at offsets[p] (the budgets laid end to end)
   const unsigned* budget;  // packed budget levels; this call uses byte bshift / 8
   int bshift;
-  // outputs beyond a budget continue in the walking lane's own arena region
-  // (no atomics: a lane finishes one pair before the next), elements
-  // [arena_base + lane * arena_per_lane, + arena_per_lane); aoff[w] = where
+  // outputs beyond a budget continue in the walking quad's own arena region
+  // (no atomics: a quad finishes one pair before the next), elements
+  // [arena_base + quad * arena_per_quad, + arena_per_quad); aoff[w] = where
   // work item w's continue.  dropped[w]: 1 the run is split (budget, then
-  // arena), 2 the lane's arena ran out (the pair is clipped again)
+  // arena), 2 the quad's arena ran out (the pair is clipped again)
   long arena_base;
-  long arena_per_lane;
+  long arena_per_quad;
   long* aoff;
   unsigned char* dropped;
   unsigned long long* ndropped;  // [0] split runs, [1] pairs clipped again
@@ -398,14 +346,14 @@ __global__ void __launch_bounds__(1024) k_scan_blocks(const long* __restrict__ c
   }
 }
 
-template <int DIM, bool MASS, bool FILL>
-__global__ void __launch_bounds__(kClipBlock) k_clip(ClipArgs g) {
-  constexpr int LOC = DIM + 1;
-  constexpr int ESZ = LOC * DIM;
+// Streaming 2D clipper (clip_tri) of the listed pairs work[0 .. *nwork), those that
+// outgrew the LDS one's polygons.
+template <bool MASS, bool FILL>
+__global__ void __launch_bounds__(kClipBlock) k_clip_listed(ClipArgs g) {
   const long stride = (long)gridDim.x * blockDim.x;
-  const long n = g.work ? (long)*g.nwork : pair_count(g);
+  const long n = (long)*g.nwork;
   for (long w = (long)blockIdx.x * blockDim.x + threadIdx.x; w < n; w += stride) {
-    const long p = g.work ? g.work[w] : w;
+    const long p = g.work[w];
     const long a = g.rows[p], b = g.cols[p];
     long off = 0;
     int cap = 0;  // fill pass: the count pass's result bounds the writes
@@ -414,59 +362,38 @@ __global__ void __launch_bounds__(kClipBlock) k_clip(ClipArgs g) {
       if (cap == 0) continue;
       off = g.offsets[p];
     }
-    double A[ESZ];
+    double A[6], Bv[6];
 #pragma unroll
-    for (int k = 0; k < ESZ; k++) A[k] = g.acoords[a * ESZ + k];
+    for (int k = 0; k < 6; k++) A[k] = g.acoords[a * 6 + k];
+#pragma unroll
+    for (int k = 0; k < 6; k++) Bv[k] = g.bcoords[b * 6 + k];
     const double tol = 10.0 * fmin_f(g.asp[a], g.bsp[b]);
     double m = 0.0;
-    double blk[LOC * LOC];
-    double affa[DIM + DIM * DIM], affb[DIM + DIM * DIM];
+    double blk[9];
+    double affa[6], affb[6];
     if (MASS) {
 #pragma unroll
-      for (int k = 0; k < LOC * LOC; k++) blk[k] = 0.0;
+      for (int k = 0; k < 9; k++) blk[k] = 0.0;
 #pragma unroll
-      for (int k = 0; k < DIM + DIM * DIM; k++) {
-        affa[k] = g.aaff[a * (DIM + DIM * DIM) + k];
-        affb[k] = g.baff[b * (DIM + DIM * DIM) + k];
+      for (int k = 0; k < 6; k++) {
+        affa[k] = g.aaff[a * 6 + k];
+        affb[k] = g.baff[b * 6 + k];
       }
     }
-    int nk;
-    if constexpr (DIM == 2) {
-      double Bv[ESZ];
-#pragma unroll
-      for (int k = 0; k < ESZ; k++) Bv[k] = g.bcoords[b * ESZ + k];
-      Line L[3];
-      tri_lines(Bv, L);
-      int k = 0;
-      nk = clip_tri(A, L, tol, [&](double x0, double y0, double x1, double y1, double x2, double y2,
-                                   double ar) {
-        m = m + ar;
-        if (MASS) {
-          double el[6] = {x0, y0, x1, y1, x2, y2};
-          mass_element<2>(el, ar, affa, affb, blk);
-        }
-        if (FILL && k < cap) {
-          stream_tri(g.elements + (off + k) * 6, x0, y0, x1, y1, x2, y2);
-        }
-        k++;
-      });
-    } else {
-      Planes P;
-      load_planes(g.bplanes, b, P);
-      Tet TA;
-#pragma unroll
-      for (int kk = 0; kk < 12; kk++) TA.v[kk] = A[kk];
-      int k = 0;
-      nk = clip_tet(TA, P, tol, [&](const Tet& T, double) {
-        double vr = tet_volume_real(T.v);
-        m = m + vr;
-        if (MASS) mass_element<3>(T.v, vr, affa, affb, blk);
-        if (FILL && k < cap) {
-          write_tet(g.elements + (off + k) * 12, T.v);
-        }
-        k++;
-      });
-    }
+    Line L[3];
+    tri_lines(Bv, L);
+    int k = 0;
+    const int nk = clip_tri(A, L, tol, [&](double x0, double y0, double x1, double y1, double x2, double y2, double ar) {
+      m = m + ar;
+      if (MASS) {
+        double el[6] = {x0, y0, x1, y1, x2, y2};
+        mass_triangle(el, ar, affa, affb, blk);
+      }
+      if (FILL && k < cap) {
+        stream_tri(g.elements + (off + k) * 6, x0, y0, x1, y1, x2, y2);
+      }
+      k++;
+    });
     if (FILL) continue;
     if (nk == 0) m = 0.0;
     g.counts[p] = nk;
@@ -474,18 +401,18 @@ __global__ void __launch_bounds__(kClipBlock) k_clip(ClipArgs g) {
     if (MASS) {
       if (g.blocks) {
 #pragma unroll
-        for (int k = 0; k < LOC * LOC; k++) g.blocks[p * LOC * LOC + k] = nk == 0 ? 0.0 : blk[k];
+        for (int k = 0; k < 9; k++) g.blocks[p * 9 + k] = nk == 0 ? 0.0 : blk[k];
       }
       if (g.rkey) {
-        const long r = (p - g.indptr[a]) * LOC;
+        const long r = (p - g.indptr[a]) * 3;
 #pragma unroll
-        for (int li = 0; li < LOC; li++) {
-          const long o = g.rbase[a * LOC + li] + r;
+        for (int li = 0; li < 3; li++) {
+          const long o = g.rbase[a * 3 + li] + r;
 #pragma unroll
-          for (int j = 0; j < LOC; j++) g.rkey[o + j] = nk == 0 ? -1 : g.enlb[b * LOC + j];
+          for (int j = 0; j < 3; j++) g.rkey[o + j] = nk == 0 ? -1 : g.enlb[b * 3 + j];
           if (nk > 0) {
 #pragma unroll
-            for (int j = 0; j < LOC; j++) g.rval[o + j] = blk[li * LOC + j];
+            for (int j = 0; j < 3; j++) g.rval[o + j] = blk[li * 3 + j];
           }
         }
       }
@@ -605,8 +532,8 @@ static unsigned one_round_grid(long n, int block = kTriBlock) {
 }
 
 // 2D pairs, one per lane: the count pass (counts, measures, mass blocks and
-// mass row slots) or the fill pass, as k_clip<2, ...>, on clip_poly_lds.
-// Pairs that outgrow the LDS polygon go to g.olist for k_clip.
+// mass row slots) or the fill pass, as k_clip_listed, on clip_poly_lds.
+// Pairs that outgrow the LDS polygon go to g.olist for k_clip_listed.
 template <bool MASS, bool FILL, int BLOCK = kTriBlock>
 __global__ void __launch_bounds__(BLOCK) k_clip_tri(ClipArgs g) {
   __shared__ double poly[LdsPoly<3, 3>::kPoints * 2 * BLOCK];
@@ -983,7 +910,7 @@ k_clip_tet_walk(ClipArgs g) {
   // single pass: this quad's arena region, its fill level, and whether the
   // current pair's output outgrew budget and arena
   const long abase =
-      LEARNED ? g.arena_base + (((long)blockIdx.x * BLOCK + threadIdx.x) >> 2) * g.arena_per_lane : 0;
+      LEARNED ? g.arena_base + (((long)blockIdx.x * BLOCK + threadIdx.x) >> 2) * g.arena_per_quad : 0;
   long atop = 0;
   bool lost = false;
   unsigned nsplit = 0, nlost = 0;  // this quad's split runs and pairs to clip again
@@ -1085,7 +1012,7 @@ k_clip_tet_walk(ClipArgs g) {
         } else if (LEARNED && keep) {
           // beyond the budget: the run continues in this quad's arena
           const long e = atop + (at - cap);
-          if (e < g.arena_per_lane) {
+          if (e < g.arena_per_quad) {
             write_tet(g.elements + (abase + e) * 12, t);
           } else {
             lost = true;
@@ -1178,7 +1105,7 @@ __global__ void __launch_bounds__(kClipBlock) k_reduce_partials(int n, Partial* 
 
 // ---------------------------------------------------------------------------
 // Mixed element types in bulk: the dispatch of intersect_elements
-// (Supermesh.F90:162-209) for one pair per lane.  2D: tri x quad clips the
+// (Supermesh.F90:162-209).  2D, a pair per lane: tri x quad clips the
 // triangle by the quad's lines (tol from the triangle), quad x tri clips B's
 // triangle by A's lines, quad x quad clips A's quad by B's lines (tol 10*tiny);
 // 3D: tet x hex clips the tet by the hex's 6 planes, hex x tet the reverse,
@@ -1662,42 +1589,29 @@ __global__ void k_zero_u64(unsigned long long* __restrict__ p) {
   if (threadIdx.x == 0 && blockIdx.x == 0) *p = 0;
 }
 
-template <int DIM>
-static void launch_clip(Context& C, const ClipArgs& args, bool mass, bool fill) {
-  dim3 grid(kClipGrid), block(kClipBlock);
-  if (DIM == 2 && args.work == nullptr) {
-    // LDS clipper over all pairs, then the streaming clipper over the pairs
-    // it handed back (a device-side count: usually none, no host sync)
-    ClipArgs g = args;
-    g.olist = C.work.as<int>((size_t)(args.npairs > 0 ? args.npairs : 1));
-    g.nolist = C.scalars.as<unsigned long long>(16) + 2;
-    if (!fill) hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, C.stream, g.nolist);
-    const dim3 tgrid(one_round_grid(args.npairs)), tblock(kTriBlock);
-    if (fill) hipLaunchKernelGGL((k_clip_tri<false, true>), tgrid, tblock, 0, C.stream, g);
-    else if (mass) hipLaunchKernelGGL((k_clip_tri<true, false>), tgrid, tblock, 0, C.stream, g);
-    else hipLaunchKernelGGL((k_clip_tri<false, false>), tgrid, tblock, 0, C.stream, g);
-    LSM_HIP(hipGetLastError());
-    g.work = g.olist;
-    g.nwork = g.nolist;
-    const dim3 fgrid(64);
-    if (fill) hipLaunchKernelGGL((k_clip<DIM, false, true>), fgrid, block, 0, C.stream, g);
-    else if (mass) hipLaunchKernelGGL((k_clip<DIM, true, false>), fgrid, block, 0, C.stream, g);
-    else hipLaunchKernelGGL((k_clip<DIM, false, false>), fgrid, block, 0, C.stream, g);
-    LSM_HIP(hipGetLastError());
-    return;
-  }
-  if (fill) {
-    hipLaunchKernelGGL((k_clip<DIM, false, true>), grid, block, 0, C.stream, args);
-  } else if (mass) {
-    hipLaunchKernelGGL((k_clip<DIM, true, false>), grid, block, 0, C.stream, args);
-  } else {
-    hipLaunchKernelGGL((k_clip<DIM, false, false>), grid, block, 0, C.stream, args);
-  }
+// 2D: the LDS clipper over all pairs, then the streaming clipper over the pairs
+// it handed back (a device-side count: usually none, no host sync).
+static void launch_clip_tri(Context& C, const ClipArgs& args, bool mass, bool fill) {
+  ClipArgs g = args;
+  g.olist = C.work.as<int>((size_t)(args.npairs > 0 ? args.npairs : 1));
+  g.nolist = C.scalars.as<unsigned long long>(16) + 2;
+  if (!fill) hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, C.stream, g.nolist);
+  const dim3 tgrid(one_round_grid(args.npairs)), tblock(kTriBlock);
+  if (fill) hipLaunchKernelGGL((k_clip_tri<false, true>), tgrid, tblock, 0, C.stream, g);
+  else if (mass) hipLaunchKernelGGL((k_clip_tri<true, false>), tgrid, tblock, 0, C.stream, g);
+  else hipLaunchKernelGGL((k_clip_tri<false, false>), tgrid, tblock, 0, C.stream, g);
+  LSM_HIP(hipGetLastError());
+  g.work = g.olist;
+  g.nwork = g.nolist;
+  const dim3 fgrid(64), block(kClipBlock);
+  if (fill) hipLaunchKernelGGL((k_clip_listed<false, true>), fgrid, block, 0, C.stream, g);
+  else if (mass) hipLaunchKernelGGL((k_clip_listed<true, false>), fgrid, block, 0, C.stream, g);
+  else hipLaunchKernelGGL((k_clip_listed<false, false>), fgrid, block, 0, C.stream, g);
   LSM_HIP(hipGetLastError());
 }
 
 // which: 0 count, 1 count + mass, 2 fill, 3 single pass, 4 single pass + mass.
-// Persistent lanes: one full wave of resident blocks.
+// Persistent quads: one full wave of resident blocks.
 static unsigned tet_walk_blocks(Context& C, int which) {
   static int blocks_per_cu[5] = {0, 0, 0, 0, 0};
   static const void* kernels[5] = {
@@ -2133,7 +2047,7 @@ void clip_pairs(Context& C, const DevMesh& A, const DevMesh& B, long npairs, int
   if (dim == 3 && npairs > 0) triage_tets(C, g, mass, npairs);
   bool learned = elems && dim == 3 && (flags & LIBSUPERMESH_GPU_LEARNED) && npairs > 0;
   const bool dense = flags & LIBSUPERMESH_GPU_DENSE;
-  long nwork = 0, nslots = 0, nspill = 0, capacity = 0, arena_per_lane = 0, gap = 0;
+  long nwork = 0, nslots = 0, nspill = 0, capacity = 0, arena_per_quad = 0, gap = 0;
   long* offs = nullptr;
   C.runs_layout = false;
   out->dense_route = 0;
@@ -2170,8 +2084,8 @@ void clip_pairs(Context& C, const DevMesh& A, const DevMesh& B, long npairs, int
     // the highest quantile level whose runs, with the arena and the spill
     // reserve behind them, fit in the device memory left.  The arena takes
     // the outputs beyond a budget (a fraction of the expected output, spread
-    // over the walk's lanes), the spill reserve the joined runs of those
-    // pairs (run layout only) and the runs of the pairs whose lane's arena
+    // over the walk's quads), the spill reserve the joined runs of those
+    // pairs (run layout only) and the runs of the pairs whose quad's arena
     // ran out (clipped again).  The dense layout is moved into place in the
     // same buffer afterwards; its runs start a gap into the buffer, so that
     // the pairs ahead of their budgets do not reach runs not yet moved.
@@ -2182,14 +2096,14 @@ void clip_pairs(Context& C, const DevMesh& A, const DevMesh& B, long npairs, int
     LSM_HIP(hipMemGetInfo(&free_b, &total_b));
     const double avail = (double)free_b + (double)C.elements.bytes - 4e9;
     const double expect = (double)hs[4] / 1024.0;
-    const long lanes = tet_walk_quads(C, mass ? 4 : 3);  // the grid of the single-pass launch
-    arena_per_lane = ((long)(P.arena_fraction * expect) + P.arena_min) / lanes;
+    const long quads = tet_walk_quads(C, mass ? 4 : 3);  // the grid of the single-pass launch
+    arena_per_quad = ((long)(P.arena_fraction * expect) + P.arena_min) / quads;
     nspill = (long)(P.spill_fraction * expect) + P.spill_min;
     gap = dense ? (long)(expect / 256.0) + 4096 : 0;
     int level = -1;
     for (int k = 0; k < 4 && level < 0; k++) {
       const double need =
-          (double)gap + (double)hs[k] + (double)(arena_per_lane * lanes) + (double)nspill + 1.0;
+          (double)gap + (double)hs[k] + (double)(arena_per_quad * quads) + (double)nspill + 1.0;
       if (need * 96.0 <= avail) level = k;
     }
     if (level < 0) {
@@ -2211,12 +2125,12 @@ void clip_pairs(Context& C, const DevMesh& A, const DevMesh& B, long npairs, int
       LSM_HIP(hipGetLastError());
       LSM_HIP(hipMemcpyAsync(&nslots, offs + npairs, sizeof(long), hipMemcpyDeviceToHost, C.stream));
       LSM_HIP(hipStreamSynchronize(C.stream));
-      capacity = nslots + arena_per_lane * lanes + nspill;
+      capacity = nslots + arena_per_quad * quads + nspill;
       g.offsets = offs;
       g.elements = C.elements.as<double>((size_t)(gap + capacity) * 12) + gap * 12;
       g.budget = budget;
       g.arena_base = nslots;
-      g.arena_per_lane = arena_per_lane;
+      g.arena_per_quad = arena_per_quad;
       g.aoff = P.aoff.as<long>((size_t)(nwork > 0 ? nwork : 1));
       g.dropped = P.overflow.as<unsigned char>((size_t)(nwork > 0 ? nwork : 1));
       g.ndropped = C.scalars.as<unsigned long long>(16) + 4;
@@ -2224,7 +2138,7 @@ void clip_pairs(Context& C, const DevMesh& A, const DevMesh& B, long npairs, int
     }
   }
   if (C.timing) LSM_HIP(hipEventRecord(C.ev[14], C.stream));
-  if (dim == 2) launch_clip<2>(C, g, mass, false);
+  if (dim == 2) launch_clip_tri(C, g, mass, false);
   else if (learned) launch_tet_walk(C, g, mass ? 4 : 3);
   else if (npairs > 0) launch_tet_walk(C, g, mass, false);  // without pairs there is no work list to read
   if (C.timing) LSM_HIP(hipEventRecord(C.ev[15], C.stream));
@@ -2313,7 +2227,7 @@ void clip_pairs(Context& C, const DevMesh& A, const DevMesh& B, long npairs, int
     inclusive_scan_long(C, tmp_counts, dofs + 1, npairs);
     g.offsets = dofs;
     g.elements = C.elements.as<double>((size_t)(out->nout > 0 ? out->nout : 1) * loc * dim);
-    if (dim == 2) launch_clip<2>(C, g, false, true);
+    if (dim == 2) launch_clip_tri(C, g, false, true);
     else launch_tet_walk(C, g, false, true);
   }
   out->offsets = dofs;
@@ -2402,7 +2316,7 @@ static void launch_count_tri(Context& C, const ClipArgs& g, const CountShape& s,
   ClipArgs f = g;
   f.work = g.olist;
   f.nwork = g.nolist;
-  hipLaunchKernelGGL((k_clip<2, false, false>), dim3(64), dim3(kClipBlock), 0, C.stream, f);
+  hipLaunchKernelGGL((k_clip_listed<false, false>), dim3(64), dim3(kClipBlock), 0, C.stream, f);
   LSM_HIP(hipGetLastError());
 }
 
@@ -2619,7 +2533,8 @@ void count_pass_graph(Context& C, const DevMesh& A, const DevMesh& B, long npair
 // Clipping an explicit pair list with no allocation, for callers that cannot
 // allocate device memory (code under stream capture, serving loops).  The
 // kernels read the meshes' positions and element lists directly (no staged
-// copies), each lane gathering its pair's two elements; the pass's only device
+// copies): a lane gathers its pair's two elements in 2D, in 3D each of a quad's
+// four lanes does and forms all of B's planes; the pass's only device
 // memory beyond the caller's inputs and outputs is the file-scope `scratch`
 // below: the 2D pairs handed from the LDS clipper to the streaming one, their
 // count, and the partial sums of the measure reduction.  Every call on a GPU
@@ -3298,10 +3213,11 @@ k_tet_row_bounds(long nn, const long* __restrict__ nptr, const int* __restrict__
 // Every entry goes straight into an LDS hash table, where it is added to its
 // column's sum, so a row may hold any number of entries; at the end the
 // columns are sorted and written.  One wave adds to a table, its instructions
-// in order and the lanes of each in theirs, so the sums are the same on every
-// run.  (Rows of up to 2048 entries used to be gathered into LDS and longer
-// ones, which any two like tet meshes have, sorted globally: 6.9 ms of sort
-// and segment sums at 32^3 vs 30^3 against 0.3 ms here.)
+// in order and, where lanes of one meet in a column, the lanes in theirs: so
+// gfx950's LDS does it, and repeated calls agree bit for bit.  (Rows of up to
+// 2048 entries used to be gathered into LDS and longer ones, which any two like
+// tet meshes have, sorted globally: 6.9 ms of sort and segment sums at 32^3 vs
+// 30^3 against 0.36 ms here.)
 __global__ void __launch_bounds__(256)
 k_mass_rows_tet(long nn, const long* __restrict__ nptr, int* __restrict__ nlist, const long* __restrict__ indptr,
                 const int* __restrict__ cols, const int* __restrict__ counts, const double* __restrict__ blocks,

@@ -131,34 +131,22 @@ LSM_HD unsigned planes_cut(uint32_t s, unsigned* inside) {
   return (0x55u & ~in) | out;
 }
 
+#ifdef __HIPCC__
 // Index of the split table for plane j (0..3) of code word s.
-LSM_HD unsigned case_index(uint32_t s, int j) {
-  const uint32_t x = (s >> (2 * j)) & 0x03030303u;
-#ifdef __HIP_DEVICE_COMPILE__
-  return __builtin_amdgcn_udot4(x, 0x40100401u, 0u, false);
-#else
-  // gathers the four bytes' low pairs into the top byte; no two partial
-  // products share a bit, so nothing carries
-  return (x * 0x01041040u) >> 24;
-#endif
+__device__ __forceinline__ unsigned case_index(uint32_t s, int j) {
+  return __builtin_amdgcn_udot4((s >> (2 * j)) & 0x03030303u, 0x40100401u, 0u, false);
 }
+
+// Bytes of (lo: selector 0..3, hi: 4..7) picked by the four selector bytes.
+__device__ __forceinline__ uint32_t byte_permute(uint32_t hi, uint32_t lo, uint32_t sel) {
+  return __builtin_amdgcn_perm(hi, lo, sel);
+}
+#endif
 
 // s with every vertex inside planes 0..j.
 LSM_HD uint32_t done_up_to(uint32_t s, int j) {
   const uint32_t m = ((4u << (2 * j)) - 1u) * 0x01010101u;
   return (s & ~m) | (0x55555555u & m);
-}
-
-// Bytes of (lo: selector 0..3, hi: 4..7) picked by the four selector bytes.
-LSM_HD uint32_t byte_permute(uint32_t hi, uint32_t lo, uint32_t sel) {
-#ifdef __HIP_DEVICE_COMPILE__
-  return __builtin_amdgcn_perm(hi, lo, sel);
-#else
-  const uint64_t both = ((uint64_t)hi << 32) | lo;
-  uint32_t r = 0;
-  for (int i = 0; i < 4; i++) r |= (uint32_t)((both >> (8 * ((sel >> (8 * i)) & 7))) & 0xff) << (8 * i);
-  return r;
-#endif
 }
 
 LSM_HD double plane_distance(const double* pl, const double* v) { return dot3(pl[0], pl[1], pl[2], v[0], v[1], v[2]) - pl[3]; }
