@@ -32,16 +32,17 @@ HBM_PEAK_GBS = 8000.0
 # on these workloads: clip + (2D) the mixed-mass quadrature.
 FLOPS_PER_PAIR = {"tri_1024_vs_1000": 108.6 + 268.0, "tet_64_vs_60": 544.6}
 
-# Algorithmic bytes per candidate pair of the clip count pass: the B element
-# gathered (tri 6 doubles + 3 ids = 60 B; tet 12 doubles + 4 ids = 112 B),
-# the pair's CSR index (4 B), its count (4 B) and measure (8 B); with the
-# mixed mass (2D) also its 3x3 block (72 B).
-BYTES_PER_PAIR = {"tri_1024_vs_1000": 60 + 4 + 4 + 8 + 72, "tet_64_vs_60": 112 + 4 + 4 + 8}
+# Algorithmic bytes per candidate pair of the 2D clip count pass: the B element
+# gathered (6 doubles + 3 ids = 60 B), the pair's CSR index (4 B), its count
+# (4 B) and measure (8 B) and its 3x3 block of the mixed mass (72 B).  The 3D
+# walk has no such figure: most candidates are dropped before it, and the
+# elements of those that are not come from cache more often than not.
+BYTES_PER_PAIR = {"tri_1024_vs_1000": 60 + 4 + 4 + 8 + 72}
 
 # HBM bytes per launch of the same kernel on the same workload, from the two
 # counter runs summarised in profiles/traffic_tri1024_tet64.md (FETCH_SIZE x
-# 1.9992 + WRITE_SIZE x 1.0, the factors a 256 MiB copy calibrates).
-PROFILED_TRAFFIC = {"tri_1024_vs_1000": 3.55e9, "tet_64_vs_60": 3.02e9}
+# 1.9996 + WRITE_SIZE x 1.0, the factors a 256 MiB copy calibrates).
+PROFILED_TRAFFIC = {"tri_1024_vs_1000": 3.55e9, "tet_64_vs_60": 3.01e9}
 
 
 def parse():
@@ -334,26 +335,27 @@ def learned_workload(ctx, name, steps, warmup, weights, quantiles=(0.7, 0.8, 0.8
 def clip_roofline(name, w):
     """Roofline of the clip count pass (the dominant kernel of the 2D step
     and of the 3D step), timed with HIP events on the library's stream over
-    the timed steps.  Both its ceilings are given: HBM (the bound at this
-    arithmetic intensity) and FP64."""
+    the timed steps.  Both its ceilings are given, first the one it is nearer
+    to: in 2D HBM, by the bytes per pair above; in 3D FP64, its HBM rate being
+    that of the profiled traffic."""
     secs = w["clip_kernel_ms"] / 1e3
-    bpp, fpp = BYTES_PER_PAIR.get(name), FLOPS_PER_PAIR.get(name)
-    if not bpp or secs <= 0:
+    bpp, fpp, traffic = BYTES_PER_PAIR.get(name), FLOPS_PER_PAIR.get(name), PROFILED_TRAFFIC.get(name)
+    if not fpp or secs <= 0:
         return {"bound": "hbm", "achieved": None, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": None,
                 "traffic": None, "kernel_ms": w["clip_kernel_ms"]}
-    gbs = bpp * w["pairs"] / secs / 1e9
-    out = {"bound": "hbm", "achieved": gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": gbs / HBM_PEAK_GBS,
-           "traffic": PROFILED_TRAFFIC.get(name), "kernel": "k_clip_tri count pass with mixed mass"
-           if name.startswith("tri") else "k_clip_tet_walk count pass",
-           "bytes_per_pair": bpp, "pairs_per_launch": w["pairs"], "kernel_ms": w["clip_kernel_ms"]}
-    if fpp:
-        tf = fpp * w["pairs"] / secs / 1e12
-        # bit-exactness forbids fused multiply-adds: half the FMA-counted peak
-        # is the attainable one for this code
-        out["fp64"] = {"achieved": tf, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": tf / FP64_PEAK_TFLOPS,
-                       "peak_without_fma": FP64_PEAK_TFLOPS / 2, "frac_without_fma": tf / (FP64_PEAK_TFLOPS / 2),
-                       "flops_per_pair": fpp}
-    return out
+    gbs = (bpp * w["pairs"] if bpp else traffic) / secs / 1e9
+    hbm = {"achieved": gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": gbs / HBM_PEAK_GBS}
+    tf = fpp * w["pairs"] / secs / 1e12
+    # bit-exactness forbids fused multiply-adds: half the FMA-counted peak
+    # is the attainable one for this code
+    fp64 = {"achieved": tf, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": tf / FP64_PEAK_TFLOPS,
+            "peak_without_fma": FP64_PEAK_TFLOPS / 2, "frac_without_fma": tf / (FP64_PEAK_TFLOPS / 2),
+            "flops_per_pair": fpp}
+    common = {"traffic": traffic, "pairs_per_launch": w["pairs"], "kernel_ms": w["clip_kernel_ms"]}
+    if bpp:
+        return {"bound": "hbm", **hbm, "kernel": "k_clip_tri count pass with mixed mass", "bytes_per_pair": bpp,
+                **common, "fp64": fp64}
+    return {"bound": "fp64", **fp64, "kernel": "k_clip_tet_walk count pass", **common, "hbm": hbm}
 
 
 def learned_batched_workload(ctx, steps, warmup, weights, count=1024):
