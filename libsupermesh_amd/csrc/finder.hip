@@ -1449,13 +1449,18 @@ k_scan_rows(int na, const long* __restrict__ row_count, long* __restrict__ indpt
 // Level of the hierarchy at which walks are cut into tasks, levels - 1 for
 // none.  A wave walks its part of the tree by itself, a few microseconds per
 // node on an idle card, so a search of few query waves is cut at nodes of 64
-// elements (tet 11^3 vs 10^3, 250 waves: the call 359 us, 422 uncut, 403 at
-// nodes of 8, 376 at 512).  From 2048 waves, eight per CU, the walks hide each
-// other and the two launches and the larger union are only a loss (tet 32^3 vs
-// 29^3, 6144 waves: 3.40 ms uncut, 3.63 at 512).  In a batch, where a mesh of
-// a few elements may face one of tens of thousands, always at 512 elements
-// (192 uneven mesh pairs: 6.5 ms, 10.8 uncut).  A hierarchy of at most 64
-// elements is walked in less time than the launches that cut it take.
+// elements.  With more waves the walks hide each other, and the two launches and
+// the larger union are only a loss where rows are of like length.  Meshes against
+// others of like size, us cut and uncut: triangles, 64 waves 86 and 93, 256 105
+// and 113, 576 150 and 151, 1024 167 and 154, 2025 226 and 184, 4096 296 and 197;
+// tets, 96 waves 99 and 140, 250 129 and 197, 515 197 and 244, 922 230 and 248,
+// 1500 328 and 316, 1997 461 and 322, 6144 943 and 503.  Where one row is long the
+// cut is what bounds it, which nothing tells beforehand: a triangle over all of
+// 39 000 in 1225 waves 0.35 ms cut and 3.4 uncut, over 58 000 in 1806 0.47 and
+// 5.1.  Up to 2048 waves that outweighs what even rows lose.  In a batch, where a
+// mesh of a few elements may face one of tens of thousands, always at 512 elements
+// (192 uneven mesh pairs: 6.5 ms, 10.8 uncut).  A hierarchy of at most 64 elements
+// is walked in less time than the launches that cut it take.
 static int task_level(const LevelInfo& info, long waves, bool grouped) {
   const int top = info.levels - 1;
   if (top <= 2) return top;

@@ -1,6 +1,7 @@
-"""The candidate search where it changes its way at a limit of its buffers or of
-the order's sort: more tasks than the arrays of the first try hold (in one mesh
-pair and in a batch), and meshes of 2^23 elements and one more."""
+"""The candidate search where it changes its way at a limit of its buffers, of the
+order's sort or of its rules: more tasks than the arrays of the first try hold (in
+one mesh pair and in a batch), meshes of 2^23 elements and one more, and query
+waves on both sides of the number from which walks are not cut."""
 import numpy as np
 import pytest
 
@@ -33,6 +34,24 @@ def test_more_tasks_than_room(dim):
         out = gpu.fetch(ctx.intersection_finder(A, B, flags=gpu.SORTED), dim, ("indptr", "indices", "rows"))
         assert np.array_equal(out["indptr"], ip) and np.array_equal(out["indices"], ix)
         assert np.array_equal(out["rows"], np.repeat(np.arange(na), np.diff(ip)))
+    ctx.close()
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+@pytest.mark.parametrize("na", [32 * 2047 - 1, 32 * 2047, 32 * 2047 + 1, 32 * 2048 + 1])
+def test_waves_about_the_cut(dim, na):
+    rng = np.random.default_rng(na)
+    def simplices(n, size):
+        t = rng.uniform(0, 1, (n, 1, dim)) + np.concatenate([np.zeros((n, 1, dim)), rng.uniform(0, size, (n, dim, dim))], 1)
+        return np.ascontiguousarray(t.reshape(-1, dim)), np.arange(n * (dim + 1), dtype=np.int32).reshape(n, dim + 1)
+    pa, ea = simplices(na, 0.05)
+    pb, eb = simplices(900, 0.1)
+    ip, ix = O.brute_force(pa, ea, pb, eb)
+    ctx = gpu.Context()
+    out = gpu.fetch(ctx.intersection_finder(gpu.DeviceMesh(pa, ea), gpu.DeviceMesh(pb, eb), flags=gpu.SORTED), dim,
+                    ("indptr", "indices", "rows"))
+    assert np.array_equal(out["indptr"], ip) and np.array_equal(out["indices"], ix)
+    assert np.array_equal(out["rows"], np.repeat(np.arange(na), np.diff(ip)))
     ctx.close()
 
 
